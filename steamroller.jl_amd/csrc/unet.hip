@@ -78,6 +78,42 @@ __device__ inline uint4 pack8(const float *o) {
 // convolution as an implicit GEMM on the matrix cores
 // ---------------------------------------------------------------------------
 
+// Epilogue of the convolutions: a lane holds D[4 g + j][col], the output
+// channels 16 r + 4 g + j of its voxel v in column group q.
+template <int R, int OUT>
+__device__ __forceinline__ void conv_store(const f32x4 (&acc)[R][4], int q, int g, int64_t v,
+                                           const float *__restrict__ bias, int nbias, int relu,
+                                           const uint16_t *__restrict__ mask, void *__restrict__ out, int cout_s) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int co0 = 16 * r + 4 * g;
+        if (co0 >= cout_s) continue;
+        float o[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float val = acc[r][q][j];
+            if (bias && co0 + j < nbias) val += bias[co0 + j];
+            if (relu) val = fmaxf(val, 0.f);
+            o[j] = val;
+        }
+        if constexpr (OUT == 0) {
+            if (mask) {
+                const uint2 mm = *reinterpret_cast<const uint2 *>(mask + v * cout_s + co0);
+                if (!bf_pos(mm.x)) o[0] = 0.f;
+                if (!bf_pos(mm.x >> 16)) o[1] = 0.f;
+                if (!bf_pos(mm.y)) o[2] = 0.f;
+                if (!bf_pos(mm.y >> 16)) o[3] = 0.f;
+            }
+            uint2 pk;
+            pk.x = f2bf(o[0]) | (f2bf(o[1]) << 16);
+            pk.y = f2bf(o[2]) | (f2bf(o[3]) << 16);
+            *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(out) + v * cout_s + co0) = pk;
+        } else {
+            if (co0 == 0) static_cast<float *>(out)[v] = o[0];
+        }
+    }
+}
+
 // out[v][co] = act(sum_{t, ci} W[co][t][ci] in[v + off(t)][ci] + bias[co]),
 // zero outside the grid. GEMM view: D (cout x voxels) = W (cout x K) *
 // Xcol (K x voxels), K = taps * cin. A wave owns 16 R output channels x 64
@@ -162,38 +198,157 @@ __global__ __launch_bounds__(TPB) void k_conv(const uint16_t *__restrict__ in, i
 #pragma unroll
                 for (int q = 0; q < 4; q++) acc[r][q] += red[k][r][q][lane];
     }
-    // lane holds D[4 g + j][col]: output channels 16 r + 4 g + j of voxel col
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (!ok[q]) continue;
-        const int64_t v = vbase + 16 * q + col;
+    for (int q = 0; q < 4; q++)
+        if (ok[q]) conv_store<R, OUT>(acc, q, g, vbase + 16 * q + col, bias, nbias, relu, mask, out, cout_s);
+}
+
+// ---------------------------------------------------------------------------
+// tiles of a channels-last grid in LDS
+// ---------------------------------------------------------------------------
+
+// TX x TY x TZ voxels and a halo of one, kept as one plane per 8 channels:
+// 16 bytes per voxel, so that 16 lanes on 16 consecutive voxels read 256
+// contiguous bytes whatever the channel count. The tile shrinks with the
+// channel count so that a work group's tile stays under 56 KB.
+template <int D, int CIN>
+struct ConvTile {
+    static constexpr int C8 = CIN / 8;
+    static constexpr int TX = D == 3 ? (CIN <= 16 ? 16 : 8) : (CIN <= 16 ? 32 : 16);
+    static constexpr int TY = D == 3 ? (CIN == 64 ? 4 : 8) : (CIN == 64 ? 8 : 16);
+    static constexpr int TZ = D == 3 ? 4 : 1;
+    static constexpr int NV = TX * TY * TZ;
+    static constexpr int HX = TX + 2, HY = TY + 2, HZ = D == 3 ? TZ + 2 : 1;
+    static constexpr int HV = HX * HY * HZ;
+    static constexpr int NTAP = D == 3 ? 27 : 9;
+    // plane offset of tap t relative to the tap at the tile's lowest corner
+    __device__ static __forceinline__ int tap(int t) {
+        const int dx = t % 3, dy = (t / 3) % 3, dz = t / 9;
+        return (dz * HY + dy) * HX + dx;
+    }
+    // halo position (lowest tap) of tile voxel t, x fastest
+    __device__ static __forceinline__ int base(int t) {
+        return ((t / (TX * TY)) * HY + (t / TX) % TY) * HX + t % TX;
+    }
+};
+
+// where tile `id` of a batch of grids lies
+struct TileAt {
+    int64_t n;       // first voxel of its grid
+    int x, y, z;     // first voxel of the tile in the grid
+};
+template <class TL>
+__device__ __forceinline__ TileAt tile_at(int id, int n0, int n1, int n2) {
+    const int tx = (n0 + TL::TX - 1) / TL::TX, ty = (n1 + TL::TY - 1) / TL::TY, tz = (n2 + TL::TZ - 1) / TL::TZ;
+    TileAt a;
+    a.x = id % tx * TL::TX;
+    id /= tx;
+    a.y = id % ty * TL::TY;
+    id /= ty;
+    a.z = id % tz * TL::TZ;
+    a.n = (int64_t)(id / tz) * n0 * n1 * n2;
+    return a;
+}
+
+// the tile and its halo into the planes xs; zero outside the grid
+template <int D, int CIN>
+__device__ __forceinline__ void load_tile(uint4 *xs, const uint16_t *__restrict__ in, const TileAt &at, int n0, int n1,
+                                          int n2) {
+    using TL = ConvTile<D, CIN>;
+    constexpr int N = TL::HV * TL::C8, IT = (N + TPB - 1) / TPB;
+    uint4 v[IT];
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int co0 = 16 * r + 4 * g;
-            if (co0 >= cout_s) continue;
-            float o[4];
+    for (int k = 0; k < IT; k++) {
+        const int i = k * TPB + (int)threadIdx.x, c = i % TL::C8, h = i / TL::C8;
+        const int x = at.x + h % TL::HX - 1, y = at.y + (h / TL::HX) % TL::HY - 1;
+        const int z = D == 3 ? at.z + h / (TL::HX * TL::HY) - 1 : 0;
+        v[k] = make_uint4(0u, 0u, 0u, 0u);
+        if (i < N && x >= 0 && x < n0 && y >= 0 && y < n1 && z >= 0 && z < n2)
+            v[k] = *reinterpret_cast<const uint4 *>(in + (at.n + x + (int64_t)n0 * (y + (int64_t)n1 * z)) * CIN + 8 * c);
+    }
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float val = acc[r][q][j];
-                if (bias && co0 + j < nbias) val += bias[co0 + j];
-                if (relu) val = fmaxf(val, 0.f);
-                o[j] = val;
+    for (int k = 0; k < IT; k++) {
+        const int i = k * TPB + (int)threadIdx.x;
+        if (i < N) xs[(i % TL::C8) * TL::HV + i / TL::C8] = v[k];
+    }
+}
+
+// consecutive tiles (which share halos) on one XCD: work group i of n takes
+// tile xcd_tile(i, n)
+__device__ __forceinline__ int xcd_tile(int i, int n) {
+    const int q = n >> 3;
+    return i < 8 * q ? (i & 7) * q + (i >> 3) : i;
+}
+
+// k_conv on tiles in LDS: the same products in the same order (the same bits),
+// with the taps' operands read from the tile instead of gathered once per tap
+// from the caches. Taken where K is not split and the weights of a K step fit
+// (up to 32 channels): 8 to 8 channels on 16 grids of 64^3 take 82 us against
+// 136 us gathered, on one grid 11.5 against 17; bound by the LDS reads and the
+// address arithmetic about equally, then by the 134 to 200 MB it moves.
+template <int D, int CIN, int R, int OUT>
+__global__ __launch_bounds__(TPB) void k_conv_tile(const uint16_t *__restrict__ in, const uint16_t *__restrict__ w,
+                                                   int kp, const float *__restrict__ bias, int nbias, int relu,
+                                                   const uint16_t *__restrict__ mask, void *__restrict__ out,
+                                                   int cout_s, int n0, int n1, int n2) {
+    using TL = ConvTile<D, CIN>;
+    constexpr int KS = (TL::NTAP * CIN + 31) / 32;  // 32-wide K steps
+    constexpr int IT = TL::NV / TPB;                // groups of 64 voxels per wave
+    static_assert(IT >= 1, "a tile holds 64 voxels for every wave");
+    constexpr bool AREG = KS * R <= 16;             // the weights stay in registers
+    __shared__ uint4 xs[TL::C8 * TL::HV + 1];
+    const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, wv = threadIdx.x >> 6;
+    const TileAt at = tile_at<TL>(xcd_tile(blockIdx.x, gridDim.x), n0, n1, n2);
+    auto load_a = [&](int s, int r) {
+        return __builtin_bit_cast(bf16x8,
+                                  *reinterpret_cast<const uint4 *>(w + (size_t)(16 * r + col) * kp + 32 * s + 8 * g));
+    };
+    bf16x8 areg[AREG ? KS : 1][R];
+    if constexpr (AREG) {
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+#pragma unroll
+            for (int r = 0; r < R; r++) areg[s][r] = load_a(s, r);
+    }
+    load_tile<D, CIN>(xs, in, at, n0, n1, n2);
+    if (threadIdx.x == 0) xs[TL::C8 * TL::HV] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        int hb[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) hb[q] = TL::base(it * TPB + 64 * wv + 16 * q + col);
+        f32x4 acc[R][4];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[r][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            const int kk = 32 * s + 8 * g, t = kk / CIN, c = (kk % CIN) / 8;
+            const bool in_k = t < TL::NTAP;
+            const int off = c * TL::HV + TL::tap(t);
+            bf16x8 a[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if constexpr (AREG) a[r] = areg[s][r];
+                else a[r] = load_a(s, r);
             }
-            if constexpr (OUT == 0) {
-                if (mask) {
-                    const uint2 mm = *reinterpret_cast<const uint2 *>(mask + v * cout_s + co0);
-                    if (!bf_pos(mm.x)) o[0] = 0.f;
-                    if (!bf_pos(mm.x >> 16)) o[1] = 0.f;
-                    if (!bf_pos(mm.y)) o[2] = 0.f;
-                    if (!bf_pos(mm.y >> 16)) o[3] = 0.f;
-                }
-                uint2 pk;
-                pk.x = f2bf(o[0]) | (f2bf(o[1]) << 16);
-                pk.y = f2bf(o[2]) | (f2bf(o[3]) << 16);
-                *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(out) + v * cout_s + co0) = pk;
-            } else {
-                if (co0 == 0) static_cast<float *>(out)[v] = o[0];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const bf16x8 b = __builtin_bit_cast(bf16x8, xs[in_k ? hb[q] + off : TL::C8 * TL::HV]);
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b, acc[r][q], 0, 0, 0);
             }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int t = it * TPB + 64 * wv + 16 * q + col;
+            const int x = at.x + t % TL::TX, y = at.y + (t / TL::TX) % TL::TY, z = at.z + t / (TL::TX * TL::TY);
+            if (x >= n0 || y >= n1 || z >= n2) continue;
+            conv_store<R, OUT>(acc, q, g, at.n + x + (int64_t)n0 * (y + (int64_t)n1 * z), bias, nbias, relu, mask, out,
+                               cout_s);
         }
     }
 }
@@ -201,9 +356,10 @@ __global__ __launch_bounds__(TPB) void k_conv(const uint16_t *__restrict__ in, i
 // Weight and bias gradient of one convolution over a chunk of voxels:
 // partial[chunk][co][k] = sum_v dz[v][co] Xcol[v][k], k < ktot, and the bias
 // column k = ktot (Xcol = 1). GEMM view with the voxels as the reduction
-// dimension: a wave owns 16 output channels x 4 tiles of 16 k.
+// dimension: a wave owns 16 output channels x 4 tiles of 16 k. For grids whose
+// z planes are no multiple of 32 voxels; k_wgrad takes the others.
 template <int D>
-__global__ __launch_bounds__(TPB) void k_wgrad(const uint16_t *__restrict__ dz, int cg, int cout,
+__global__ __launch_bounds__(TPB) void k_wgrad_gather(const uint16_t *__restrict__ dz, int cg, int cout,
                                                const uint16_t *__restrict__ x, int cin_log2, int ktot, int kx,
                                                int n0, int n1, int n2, int64_t nvox, int64_t chunk,
                                                float *__restrict__ partial) {
@@ -307,15 +463,181 @@ __global__ __launch_bounds__(TPB) void k_wgrad(const uint16_t *__restrict__ dz, 
         }
 }
 
-// fixed-order sum of the chunk partials into the weight and bias gradients
-__global__ __launch_bounds__(TPB) void k_wgrad_reduce(const float *__restrict__ partial, int nchunk, int cout, int kx,
-                                                      int ktot, float *__restrict__ gw, float *__restrict__ gb) {
-    const int i = blockIdx.x * TPB + threadIdx.x;
-    if (i >= cout * kx) return;
+// The same sums in the same order (the same bits) with both operands from LDS.
+// They want 8 consecutive voxels of one channel per lane, which channels-last
+// memory holds a voxel apart: the LDS transpose reads deliver them (16 lanes
+// read 4 voxels x 16 channels, each lane gets 4 voxels of one channel). Every
+// lane gives its own address, so a tap is an offset into the staged rows, and
+// with 8 channels two taps share one MFMA's 16 columns. A work group takes the
+// chunk in runs of at most `tl` voxels inside one z plane: the grid rows of the
+// run, one row above and below, in the three planes (two halo columns per row
+// stay zero), as one LDS plane of 16 bytes per voxel and 8 channels; the next
+// run's rows are loaded into registers while this one is used. The eight waves
+// split the columns, the last one takes the bias; 16 output channels per
+// blockIdx.y. Bound by the LDS reads (two per MFMA operand) and, with two work
+// groups per CU, by their latency: 8 to 8 channels on 16 grids of 64^3 take
+// 84 us (k_wgrad_gather: 670 us), 16 to 16 on 32^3 22 us (127 us). Longer
+// chunks of cubic tiles took 56 us but moved the sums' rounding.
+constexpr int WGT = 512;  // threads
+constexpr int WG_LDS = 48 << 10;  // rows and gradients of a run: three work groups per CU
+constexpr int WG_RUN = 512;  // voxels of a run at most
+
+// LDS plane size of `rows` rows of n0 voxels with halos, in 16-byte words:
+// 4 mod 16, so that the two planes of a transpose read fall on different banks
+template <int D>
+__host__ __device__ inline int wgrad_plane(int n0, int rows) {
+    const int h = (D == 3 ? 3 : 1) * (rows + 2) * (n0 + 2);
+    return h + ((20 - h % 16) % 16);
+}
+template <int D, int CIN>
+__host__ __device__ inline size_t wgrad_lds(int n0, int rows, int tl) {
+    return ((size_t)wgrad_plane<D>(n0, rows) * (CIN / 8) + 2 * (tl + 4)) * 16 + (size_t)(tl + n0) * 2;
+}
+
+template <int D, int CIN>
+__global__ __launch_bounds__(WGT) void k_wgrad(const uint16_t *__restrict__ dz, int cg, int cout,
+                                               const uint16_t *__restrict__ x, int ktot, int kx, int n0, int n1, int n2,
+                                               int64_t nvox, int64_t chunk, int tl, int rows,
+                                               float *__restrict__ partial) {
+    constexpr int C8 = CIN / 8, NTAP = D == 3 ? 27 : 9, NDZ = D == 3 ? 3 : 1;
+    constexpr int NT = (NTAP * CIN + 15) / 16;              // 16-column tiles
+    constexpr int NTW = CIN == 8 ? (NT + 6) / 7 : (NT + 7) / 8;  // per wave
+    constexpr int IT = WG_LDS / 16 / WGT;                   // 16-byte words per thread of a run's rows
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    extern __shared__ uint4 lds[];
+    const int HX = n0 + 2, HP = (rows + 2) * HX, plane = wgrad_plane<D>(n0, rows), zp = tl + 4;
+    uint4 *xs = lds, *zs = xs + plane * C8;
+    uint16_t *pos = reinterpret_cast<uint16_t *>(zs + 2 * zp);  // run voxel -> its lowest tap in a plane
+    const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, wv = threadIdx.x >> 6;
+    const int co0 = 16 * blockIdx.y;
+    const bool two = co0 + 8 < cg;  // the second plane of dz holds channels
+    // this lane's part of a 16-column row: 8 bytes (half), in plane or tap hi
+    const int hi = (col >> 1) & 1, half = col & 1, row = col >> 2;
+    int off[NTW];
+#pragma unroll
+    for (int j = 0; j < NTW; j++) {
+        const int k = 16 * (wv * NTW + j) + 8 * hi, t = k / CIN, c = (k % CIN) / 8;
+        // columns past the last tap are not written
+        off[j] = t < NTAP ? c * plane + (t / 9) * HP + (t / 3 % 3) * HX + t % 3 : 0;
+    }
+    f32x4 acc[NTW], accb = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NTW; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = threadIdx.x; i < plane * C8 + 2 * zp; i += WGT) lds[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = threadIdx.x; i < tl + n0; i += WGT) pos[i] = (uint16_t)(i / n0 * HX + i % n0);
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+    auto tr = [&](const uint4 *p) {
+        return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4 *)((__attribute__((address_space(3))) char *)p + 8 * half));
+    };
+    auto both = [](s16x4 lo, s16x4 hi4) {
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    const int P = n0 * n1, rw = n0 * C8;
+    const int64_t v0 = (int64_t)blockIdx.x * chunk, v1 = min(nvox, v0 + chunk);
+    // a run: first voxel va, its plane's first voxel vp and z, its offset o in
+    // the plane, its length, its first row
+    struct Run {
+        int64_t va, vp;
+        int z, o, len, y0;
+    };
+    auto run_at = [&](int64_t va) {
+        Run r;
+        r.va = va;
+        const int64_t pl = va / P;
+        r.vp = pl * P;
+        r.z = (int)(pl % n2);
+        r.o = (int)(va - r.vp);
+        r.len = (int)min((int64_t)min(tl, P - r.o), v1 - va);
+        r.y0 = r.o / n0;
+        return r;
+    };
+    uint4 xv[IT], zv[2];
+    auto load = [&](const Run &r) {
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const int i = k * WGT + (int)threadIdx.x, rr = i / rw, e = i - rr * rw;
+            const int y = r.y0 - 1 + rr % (rows + 2), z = D == 3 ? r.z - 1 + rr / (rows + 2) : 0;
+            xv[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (rr < NDZ * (rows + 2) && y >= 0 && y < n1 && z >= 0 && z < n2)
+                xv[k] = *reinterpret_cast<const uint4 *>(x + (r.vp + (int64_t)(z - (D == 3 ? r.z : 0)) * P +
+                                                              (int64_t)y * n0) * CIN + 8 * e);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int i = k * WGT + (int)threadIdx.x, t = i >> 1, c = i & 1;
+            zv[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (t < r.len && (c == 0 || two))
+                zv[k] = *reinterpret_cast<const uint4 *>(dz + (r.va + t) * cg + co0 + 8 * c);
+        }
+    };
+    if (v0 < v1) load(run_at(v0));
+    for (int64_t va = v0; va < v1;) {
+        const Run r = run_at(va);
+        __syncthreads();  // the previous run has been used (first: the zeros are written)
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const int i = k * WGT + (int)threadIdx.x, rr = i / rw, e = i - rr * rw;
+            if (rr < NDZ * (rows + 2)) xs[(e % C8) * plane + rr * HX + 1 + e / C8] = xv[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int i = k * WGT + (int)threadIdx.x, t = i >> 1, c = i & 1;
+            if (t < tl) zs[c * zp + t] = zv[k];
+        }
+        __syncthreads();
+        va += r.len;
+        if (va < v1) load(run_at(va));
+        const int o = r.o - r.y0 * n0;
+        // 32 voxels per step: element 8 g + i of a lane is voxel 8 g + i
+#pragma unroll 2
+        for (int s = 0; s < r.len; s += 32) {
+            const int t0 = s + 8 * g + row, t1 = t0 + 4;
+            const bf16x8 a = both(tr(zs + hi * zp + t0), tr(zs + hi * zp + t1));
+            const uint4 *x0 = xs + pos[o + t0], *x1 = xs + pos[o + t1];
+#pragma unroll
+            for (int j = 0; j < NTW; j++)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, both(tr(x0 + off[j]), tr(x1 + off[j])), acc[j], 0, 0,
+                                                                 0);
+            if (wv == WGT / 64 - 1) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ones, accb, 0, 0, 0);
+        }
+    }
+    float *p = partial + (int64_t)blockIdx.x * cout * kx;
+#pragma unroll
+    for (int j = 0; j < NTW; j++)
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) {
+            const int co = co0 + 4 * g + jj, k = 16 * (wv * NTW + j) + col;
+            if (co < cout && k < ktot) p[(int64_t)co * kx + k] = acc[j][jj];
+        }
+    if (wv == WGT / 64 - 1 && col == 0)
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++)
+            if (co0 + 4 * g + jj < cout) p[(int64_t)(co0 + 4 * g + jj) * kx + ktot] = accb[jj];
+}
+
+// sum of the chunk partials, in chunk order, into the weight and bias
+// gradients: a work group takes 32 outputs, its loads of all chunks go to LDS
+// together and one thread per output adds them (with 16 loads in flight per
+// thread the walk over 512 chunks took 15-39 us)
+constexpr int WRED_OUT = 32, MAX_CHUNKS = 512;
+__global__ __launch_bounds__(1024) void k_wgrad_reduce(const float *__restrict__ partial, int nchunk, int cout, int kx,
+                                                       int ktot, float *__restrict__ gw, float *__restrict__ gb) {
+    __shared__ float red[MAX_CHUNKS][WRED_OUT];
+    const int o = threadIdx.x % WRED_OUT, part = threadIdx.x / WRED_OUT;
+    const int i = blockIdx.x * WRED_OUT + o;
+    const int64_t stride = (int64_t)cout * kx;
+#pragma unroll
+    for (int k = 0; k < MAX_CHUNKS * WRED_OUT / 1024; k++) {
+        const int c = k * (1024 / WRED_OUT) + part;
+        red[c][o] = (c < nchunk && i < cout * kx) ? partial[c * stride + i] : 0.f;
+    }
+    __syncthreads();
+    if (part || i >= cout * kx) return;
     float s = 0.f;
-    // loads of 16 chunks in flight, the sum in chunk order
 #pragma unroll 16
-    for (int c = 0; c < nchunk; c++) s += partial[(int64_t)c * cout * kx + i];
+    for (int c = 0; c < nchunk; c++) s += red[c][o];
     const int co = i / kx, k = i - co * kx;
     if (k < ktot)
         gw[co * ktot + k] = s;
@@ -652,6 +974,14 @@ void pack(srmg_unet *n, hipStream_t st) {
     n->packed = true;
 }
 
+// tiles of every grid of a batch
+template <class TL>
+int64_t tile_count(const Ext &e, int64_t nvox) {
+    const int64_t per = (int64_t)((e.n0 + TL::TX - 1) / TL::TX) * ((e.n1 + TL::TY - 1) / TL::TY) *
+                        ((e.n2 + TL::TZ - 1) / TL::TZ);
+    return per * (nvox / ((int64_t)e.n0 * e.n1 * e.n2));
+}
+
 template <int D, int OUT>
 void conv_launch_r(int R, unsigned grid, hipStream_t st, const uint16_t *in, int cin_log2, const uint16_t *w, int kp,
                    int ktot, const float *bias, int nbias, int relu, const uint16_t *mask, void *out, int cout_s,
@@ -659,6 +989,21 @@ void conv_launch_r(int R, unsigned grid, hipStream_t st, const uint16_t *in, int
     // few voxels: split K over the waves of a work group (one group of 64 voxels per work group)
     const bool split = nvox < SPLITK_NVOX;
     const unsigned gsk = (unsigned)((nvox + 63) / 64);
+#define SRMG_TILE(CC, RR)                                                                                          \
+    if (!split && cin_log2 == ilog2(CC) && R == RR) {                                                              \
+        hipLaunchKernelGGL((k_conv_tile<D, CC, RR, OUT>), dim3((unsigned)tile_count<ConvTile<D, CC>>(e, nvox)),    \
+                           dim3(TPB), 0, st, in, w, kp, bias, nbias, relu, mask, out, cout_s, e.n0, e.n1, e.n2);   \
+        return;                                                                                                    \
+    }
+    SRMG_TILE(8, 1)
+    SRMG_TILE(16, 1)
+    SRMG_TILE(32, 1)
+    if constexpr (OUT == 0) {
+        SRMG_TILE(8, 2)
+        SRMG_TILE(16, 2)
+        SRMG_TILE(32, 2)
+    }
+#undef SRMG_TILE
 #define SRMG_CONV(RR)                                                                                              \
     do {                                                                                                           \
         if (split)                                                                                                 \
@@ -702,22 +1047,50 @@ void conv_bwd_data(srmg_unet *n, hipStream_t st, const ConvL &cv, const uint16_t
                         0, mask, din, cv.cin, n->ext[cv.level], nvox);
 }
 
+template <int D, int CIN>
+bool wgrad_rows(const ConvL &cv, hipStream_t st, const uint16_t *dz, const uint16_t *x, const Ext &e, int64_t nvox,
+                int64_t chunk, unsigned nchunk, float *partial) {
+    // runs of whole 32-voxel steps inside a z plane; as long as their rows fit
+    if ((int64_t)e.n0 * e.n1 % 32) return false;
+    int tl = WG_RUN, rows = 0;
+    size_t need = 0;
+    for (;; tl /= 2) {
+        if (tl < 32) return false;
+        const bool aligned = tl % e.n0 == 0 && chunk % e.n0 == 0;
+        rows = std::min(aligned ? tl / e.n0 : (tl + e.n0 - 2) / e.n0 + 1, e.n1);
+        need = wgrad_lds<D, CIN>(e.n0, rows, tl);
+        if (need <= (size_t)WG_LDS) break;
+    }
+    hipLaunchKernelGGL((k_wgrad<D, CIN>), dim3(nchunk, (unsigned)((cv.cout + 15) / 16)), dim3(WGT), need, st, dz, cv.cg, cv.cout, x, cv.ktot, cv.ktot + 1, e.n0, e.n1,
+                       e.n2, nvox, chunk, tl, rows, partial);
+    return true;
+}
+
 template <int D>
 void conv_bwd_weights(srmg_unet *n, hipStream_t st, const ConvL &cv, const uint16_t *dz, const uint16_t *x, int B) {
     const int64_t nvox = (int64_t)B * n->V[cv.level];
     const int kx = cv.ktot + 1;
-    int64_t nchunk = std::min<int64_t>(512, (nvox + 255) / 256);
+    int64_t nchunk = std::min<int64_t>(MAX_CHUNKS, (nvox + 255) / 256);
     int64_t chunk = (nvox + nchunk - 1) / nchunk;
     chunk = (chunk + 31) / 32 * 32;
     nchunk = (nvox + chunk - 1) / chunk;
     const size_t need = (size_t)nchunk * cv.cout * kx * sizeof(float);
     if (n->partial.bytes < need) n->partial.alloc(need);
-    dim3 grid((unsigned)((kx + 255) / 256), (unsigned)((cv.cout + 15) / 16), (unsigned)nchunk);
     const Ext &e = n->ext[cv.level];
-    hipLaunchKernelGGL((k_wgrad<D>), grid, dim3(TPB), 0, st, dz, cv.cg, cv.cout, x, ilog2(cv.cin), cv.ktot, kx, e.n0,
-                       e.n1, e.n2, nvox, chunk, n->partial.as<float>());
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(nblocks((int64_t)cv.cout * kx)), dim3(TPB), 0, st,
-                       n->partial.as<float>(), (int)nchunk, cv.cout, kx, cv.ktot, n->gr.as<float>() + cv.woff,
+    float *part = n->partial.as<float>();
+    const unsigned nc = (unsigned)nchunk;
+    const bool done = cv.cin == 8    ? wgrad_rows<D, 8>(cv, st, dz, x, e, nvox, chunk, nc, part)
+                      : cv.cin == 16 ? wgrad_rows<D, 16>(cv, st, dz, x, e, nvox, chunk, nc, part)
+                      : cv.cin == 32 ? wgrad_rows<D, 32>(cv, st, dz, x, e, nvox, chunk, nc, part)
+                      : cv.cin == 64 ? wgrad_rows<D, 64>(cv, st, dz, x, e, nvox, chunk, nc, part)
+                                     : false;
+    if (!done) {
+        dim3 grid((unsigned)((kx + 255) / 256), (unsigned)((cv.cout + 15) / 16), nc);
+        hipLaunchKernelGGL((k_wgrad_gather<D>), grid, dim3(TPB), 0, st, dz, cv.cg, cv.cout, x, ilog2(cv.cin), cv.ktot,
+                           kx, e.n0, e.n1, e.n2, nvox, chunk, part);
+    }
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((cv.cout * kx + WRED_OUT - 1) / WRED_OUT)), dim3(1024), 0, st,
+                       part, (int)nchunk, cv.cout, kx, cv.ktot, n->gr.as<float>() + cv.woff,
                        n->gr.as<float>() + cv.boff);
 }
 
