@@ -31,6 +31,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/srmg.h"
@@ -45,6 +46,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int TPB = 256;
 // convolutions over fewer voxels split their K loop over the waves of a work group
 constexpr int64_t SPLITK_NVOX = 65536;
+// ... and lower the voxels per work group until there are this many
+constexpr int64_t SPLIT_WGS = 1024;
 constexpr int MAXLEV = 6;
 constexpr int FEAT = 8;  // input channels
 constexpr int LOSS_WGS = 1024;
@@ -80,13 +83,14 @@ __device__ inline uint4 pack8(const float *o) {
 
 // Epilogue of the convolutions: a lane holds D[4 g + j][col], the output
 // channels 16 r + 4 g + j of its voxel v in column group q.
-template <int R, int OUT>
-__device__ __forceinline__ void conv_store(const f32x4 (&acc)[R][4], int q, int g, int64_t v,
+template <int R, int OUT, int Q>
+__device__ __forceinline__ void conv_store(const f32x4 (&acc)[R][Q], int q, int g, int64_t v,
                                            const float *__restrict__ bias, int nbias, int relu,
-                                           const uint16_t *__restrict__ mask, void *__restrict__ out, int cout_s) {
+                                           const uint16_t *__restrict__ mask, void *__restrict__ out, int cout_s,
+                                           int row0 = 0) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const int co0 = 16 * r + 4 * g;
+        const int co0 = row0 + 16 * r + 4 * g;
         if (co0 >= cout_s) continue;
         float o[4];
 #pragma unroll
@@ -125,10 +129,15 @@ __device__ __forceinline__ void conv_store(const f32x4 (&acc)[R][4], int q, int 
 // OUT 0: BF16 output with cout_s stored channels; OUT 1: FP32, one channel.
 // SK > 1 (grids with few voxels, where a launch of one wave per 64 voxels
 // leaves the chip idle and each wave walks the whole K loop): the SK waves of
-// a work group share one group of 64 voxels and take every SK-th 32-wide K
-// step; waves 1..SK-1 hand their accumulators to wave 0 through LDS, which
-// adds them in wave order before the epilogue.
-template <int D, int R, int OUT, int SK = 1>
+// a work group share 16 Q voxels and take every SK-th 32-wide K step; waves
+// 1..SK-1 hand their accumulators to wave 0 through LDS, which adds them in
+// wave order before the epilogue. Output channels are split over blockIdx.y
+// (16 R per work group) and Q is lowered until the launch has a work group for
+// every CU; neither changes a product's place in its sum. A wave's chain of
+// dependent loads bounds these launches: U steps' operands are loaded before
+// their products. 64 to 64 channels on 8^3: 25 us on 8 work groups, 6 us on
+// 128; 32 to 32 on 16^3 14 against 5, 16 to 16 on 32^3 9 against 7.
+template <int D, int R, int OUT, int SK = 1, int Q = 4, int U = 1>
 __global__ __launch_bounds__(TPB) void k_conv(const uint16_t *__restrict__ in, int cin_log2,
                                               const uint16_t *__restrict__ w, int kp, int ktot,
                                               const float *__restrict__ bias, int nbias, int relu,
@@ -137,57 +146,83 @@ __global__ __launch_bounds__(TPB) void k_conv(const uint16_t *__restrict__ in, i
     static_assert(SK == 1 || SK == TPB / 64, "split K over the waves of a work group");
     const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
     const int wv = threadIdx.x >> 6;
-    const int64_t vbase = (SK > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * (TPB / 64) + wv) * 64;
+    const int row0 = 16 * R * blockIdx.y;
+    const int64_t vbase = (SK > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * (TPB / 64) + wv) * (16 * Q);
     const int64_t V = (int64_t)n0 * n1 * n2;
-    int px[4], py[4], pz[4];
-    int64_t pn[4];
-    bool ok[4];
+    int px[Q], py[Q], pz[Q];
+    int64_t pn[Q];
+    bool ok[Q];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
+    for (int q = 0; q < Q; q++) {
         const int64_t v = vbase + 16 * q + col;
         ok[q] = v < nvox;
-        const int64_t nn = ok[q] ? v / V : 0, r = ok[q] ? v - nn * V : 0;
+        const int64_t nn = ok[q] ? v / V : 0;
+        const int r = ok[q] ? (int)(v - nn * V) : 0;
         pn[q] = nn * V;
-        px[q] = (int)(r % n0);
-        py[q] = (int)((r / n0) % n1);
-        pz[q] = (int)(r / ((int64_t)n0 * n1));
+        px[q] = r % n0;
+        py[q] = (r / n0) % n1;
+        pz[q] = r / (n0 * n1);
     }
-    f32x4 acc[R][4];
+    f32x4 acc[R][Q];
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) acc[r][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int q = 0; q < Q; q++) acc[r][q] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int cin = 1 << cin_log2;
-    for (int kc = SK > 1 ? 32 * wv : 0; kc < kp; kc += 32 * SK) {
-        const int kk = kc + 8 * g;
-        bf16x8 a[R];
-#pragma unroll
-        for (int r = 0; r < R; r++)
-            a[r] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(w + (size_t)(16 * r + col) * kp + kk));
+    auto load_a = [&](int kk, int r) {
+        return __builtin_bit_cast(bf16x8,
+                                  *reinterpret_cast<const uint4 *>(w + (size_t)(row0 + 16 * r + col) * kp + kk));
+    };
+    auto load_b = [&](int kk, int q) {
         const int t = kk >> cin_log2, ci = kk & (cin - 1);
         const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = D == 3 ? t / 9 - 1 : 0;
-        bf16x8 b[4];
+        const int x = px[q] + dx, y = py[q] + dy, z = pz[q] + dz;
+        uint4 val = make_uint4(0u, 0u, 0u, 0u);
+        if (ok[q] && kk < ktot && x >= 0 && x < n0 && y >= 0 && y < n1 && z >= 0 && z < n2)
+            val = *reinterpret_cast<const uint4 *>(in + (pn[q] + x + (int64_t)n0 * (y + (int64_t)n1 * z)) * cin + ci);
+        return __builtin_bit_cast(bf16x8, val);
+    };
+    const int k0 = SK > 1 ? 32 * wv : 0;
+    int kc = k0;
+    for (; kc + 32 * SK * (U - 1) < kp; kc += 32 * SK * U) {
+        bf16x8 a[U][R], b[U][Q];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int x = px[q] + dx, y = py[q] + dy, z = pz[q] + dz;
-            uint4 val = make_uint4(0u, 0u, 0u, 0u);
-            if (ok[q] && kk < ktot && x >= 0 && x < n0 && y >= 0 && y < n1 && z >= 0 && z < n2)
-                val = *reinterpret_cast<const uint4 *>(in + (pn[q] + x + (int64_t)n0 * (y + (int64_t)n1 * z)) * cin +
-                                                       ci);
-            b[q] = __builtin_bit_cast(bf16x8, val);
+        for (int i = 0; i < U; i++) {
+            const int kk = kc + 32 * SK * i + 8 * g;
+#pragma unroll
+            for (int r = 0; r < R; r++) a[i][r] = load_a(kk, r);
+#pragma unroll
+            for (int q = 0; q < Q; q++) b[i][q] = load_b(kk, q);
         }
 #pragma unroll
-        for (int r = 0; r < R; r++)
+        for (int i = 0; i < U; i++)
 #pragma unroll
-            for (int q = 0; q < 4; q++) acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b[q], acc[r][q], 0, 0, 0);
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int q = 0; q < Q; q++)
+                    acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][r], b[i][q], acc[r][q], 0, 0, 0);
+    }
+    if constexpr (U > 1) {
+        for (; kc < kp; kc += 32 * SK) {
+            bf16x8 a[R], b[Q];
+#pragma unroll
+            for (int r = 0; r < R; r++) a[r] = load_a(kc + 8 * g, r);
+#pragma unroll
+            for (int q = 0; q < Q; q++) b[q] = load_b(kc + 8 * g, q);
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int q = 0; q < Q; q++)
+                    acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b[q], acc[r][q], 0, 0, 0);
+        }
     }
     if constexpr (SK > 1) {
-        __shared__ f32x4 red[SK - 1][R][4][64];
+        __shared__ f32x4 red[SK - 1][R][Q][64];
         if (wv > 0) {
 #pragma unroll
             for (int r = 0; r < R; r++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) red[wv - 1][r][q][lane] = acc[r][q];
+                for (int q = 0; q < Q; q++) red[wv - 1][r][q][lane] = acc[r][q];
         }
         __syncthreads();
         if (wv > 0) return;
@@ -196,11 +231,11 @@ __global__ __launch_bounds__(TPB) void k_conv(const uint16_t *__restrict__ in, i
 #pragma unroll
             for (int r = 0; r < R; r++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) acc[r][q] += red[k][r][q][lane];
+                for (int q = 0; q < Q; q++) acc[r][q] += red[k][r][q][lane];
     }
 #pragma unroll
-    for (int q = 0; q < 4; q++)
-        if (ok[q]) conv_store<R, OUT>(acc, q, g, vbase + 16 * q + col, bias, nbias, relu, mask, out, cout_s);
+    for (int q = 0; q < Q; q++)
+        if (ok[q]) conv_store<R, OUT>(acc, q, g, vbase + 16 * q + col, bias, nbias, relu, mask, out, cout_s, row0);
 }
 
 // ---------------------------------------------------------------------------
@@ -759,7 +794,8 @@ __device__ __forceinline__ double wg_max(double m) {
 // max |f| per grid in two stages: ABSMAX_PARTS work groups per grid reduce
 // contiguous chunks, then one work group per grid reduces the chunk maxima
 // (a maximum does not depend on the order: the same value as one pass)
-constexpr int ABSMAX_PARTS = 64;
+// (64 of them took 7 us on 64^3, 256 take 4)
+constexpr int ABSMAX_PARTS = 256;
 template <typename TF>
 __global__ __launch_bounds__(TPB) void k_absmax_part(const TF *__restrict__ f, int64_t V,
                                                      double *__restrict__ part) {
@@ -986,11 +1022,23 @@ template <int D, int OUT>
 void conv_launch_r(int R, unsigned grid, hipStream_t st, const uint16_t *in, int cin_log2, const uint16_t *w, int kp,
                    int ktot, const float *bias, int nbias, int relu, const uint16_t *mask, void *out, int cout_s,
                    const Ext &e, int64_t nvox) {
-    // few voxels: split K over the waves of a work group (one group of 64 voxels per work group)
     const bool split = nvox < SPLITK_NVOX;
-    const unsigned gsk = (unsigned)((nvox + 63) / 64);
+    if (split) {
+        // 64, 32 or 16 voxels and 16 output channels per work group
+        auto go = [&](auto q) {
+            constexpr int Q = decltype(q)::value;
+            hipLaunchKernelGGL((k_conv<D, 1, OUT, TPB / 64, Q, 4>), dim3((unsigned)((nvox + 16 * Q - 1) / (16 * Q)), R),
+                               dim3(TPB), 0, st, in, cin_log2, w, kp, ktot, bias, nbias, relu, mask, out, cout_s, e.n0,
+                               e.n1, e.n2, nvox);
+        };
+        const int64_t wgs = (nvox + 63) / 64 * R;
+        if (wgs >= SPLIT_WGS) go(std::integral_constant<int, 4>());
+        else if (2 * wgs >= SPLIT_WGS) go(std::integral_constant<int, 2>());
+        else go(std::integral_constant<int, 1>());
+        return;
+    }
 #define SRMG_TILE(CC, RR)                                                                                          \
-    if (!split && cin_log2 == ilog2(CC) && R == RR) {                                                              \
+    if (cin_log2 == ilog2(CC) && R == RR) {                                                              \
         hipLaunchKernelGGL((k_conv_tile<D, CC, RR, OUT>), dim3((unsigned)tile_count<ConvTile<D, CC>>(e, nvox)),    \
                            dim3(TPB), 0, st, in, w, kp, bias, nbias, relu, mask, out, cout_s, e.n0, e.n1, e.n2);   \
         return;                                                                                                    \
@@ -1004,15 +1052,9 @@ void conv_launch_r(int R, unsigned grid, hipStream_t st, const uint16_t *in, int
         SRMG_TILE(32, 2)
     }
 #undef SRMG_TILE
-#define SRMG_CONV(RR)                                                                                              \
-    do {                                                                                                           \
-        if (split)                                                                                                 \
-            hipLaunchKernelGGL((k_conv<D, RR, OUT, TPB / 64>), dim3(gsk), dim3(TPB), 0, st, in, cin_log2, w, kp,   \
-                               ktot, bias, nbias, relu, mask, out, cout_s, e.n0, e.n1, e.n2, nvox);                \
-        else                                                                                                       \
-            hipLaunchKernelGGL((k_conv<D, RR, OUT>), dim3(grid), dim3(TPB), 0, st, in, cin_log2, w, kp, ktot,      \
-                               bias, nbias, relu, mask, out, cout_s, e.n0, e.n1, e.n2, nvox);                      \
-    } while (0)
+#define SRMG_CONV(RR)                                                                                          \
+    hipLaunchKernelGGL((k_conv<D, RR, OUT>), dim3(grid), dim3(TPB), 0, st, in, cin_log2, w, kp, ktot, bias,    \
+                       nbias, relu, mask, out, cout_s, e.n0, e.n1, e.n2, nvox)
     if (R == 1)
         SRMG_CONV(1);
     else if (R == 2)
