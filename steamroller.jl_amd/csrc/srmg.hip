@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -15,6 +16,7 @@
 #include <mutex>
 #include <type_traits>
 #include <string>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -97,7 +99,50 @@ struct Graph {
     }
 };
 
+// Pinned host buffers and their device counterparts, through which host fields
+// pass in pieces (srmg_upload, srmg_download): a ring of SLOTS, kept by the
+// context, at most SLOTS x MAX_BYTES on either side (more only where one block needs it).
+struct HostStage {
+    static constexpr int SLOTS = 4;
+    static constexpr size_t MIN_BYTES = (size_t)64 << 10, MAX_BYTES = (size_t)2 << 20;
+    size_t bytes = 0;  // of a slot
+    char *pin = nullptr;
+    DevBuf dev;
+    hipEvent_t ev[SLOTS] = {};  // the slot's last copy has ended
+    char *host(int k) { return pin + (size_t)(k % SLOTS) * bytes; }
+    char *device(int k) { return dev.as<char>() + (size_t)(k % SLOTS) * bytes; }
+    void wait(int k) { HIPCHK(hipEventSynchronize(ev[k % SLOTS])); }
+    // slots that hold `total` bytes, or as much of them as a slot may; at
+    // least one block of `block` bytes
+    void reserve(size_t total, size_t block) {
+        size_t want = MIN_BYTES;
+        while (want < block || (want < total && want < MAX_BYTES)) want *= 2;
+        if (want <= bytes) return;
+        release();
+        for (auto &e : ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIPCHK(hipHostMalloc((void **)&pin, want * SLOTS, hipHostMallocDefault));
+        dev.alloc(want * SLOTS);
+        bytes = want;
+    }
+    void release() {
+        for (auto &e : ev) {
+            if (e) {
+                (void)hipEventSynchronize(e);
+                (void)hipEventDestroy(e);
+            }
+            e = nullptr;
+        }
+        if (pin) (void)hipHostFree(pin);
+        pin = nullptr;
+        dev.release();
+        bytes = 0;
+    }
+    ~HostStage() { release(); }
+};
+
 struct srmg_ctx {
+    HostStage stage;
+    DevBuf d_host2dev;      // host block id - 1 -> device block, or -1 (made on first use)
     int D = 2, M = 16, V = 0, F = 0;
     int nlevels = 0;
     int64_t nhost = 0;      // host block ids 1..nhost (all trees)
@@ -473,6 +518,7 @@ static void set_forest(srmg_ctx *c, const std::vector<TreeRecords> &tr) {
 static void commit_tables(srmg_ctx *c, srmg_ctx &t) {
     c->graphs.clear();
     c->box_ok = false;
+    c->d_host2dev.release();
     c->nlevels = t.nlevels;
     c->nhost = t.nhost;
     c->nb = t.nb;
@@ -1905,93 +1951,162 @@ static int same_type(srmg_ctx *c, std::initializer_list<int> ids) {
 // host <-> device layout conversion
 // ---------------------------------------------------------------------------
 
+// Host fields cross the bus in the caller's own layout, piece by piece through
+// the context's staging ring, and kernels convert between that and the device
+// layout (k_host_in, k_host_out): the host only copies contiguous rows, while
+// the previous piece is on the bus. Bound by the bus (52 GB/s pinned on an
+// MI355X host) and by the host's copies (30 to 45 GB/s); converted cell by cell
+// on the host, a V-cycle with two fields each way took 21.8 ms on a 2D tree of
+// 7,716 blocks of 16^2.
+
+static const int *host_table(srmg_ctx *c) {
+    if (!c->d_host2dev.p) {
+        // kernels index it by host block id - 1
+        c->d_host2dev.alloc((size_t)std::max<int64_t>(c->nhost, 1) * sizeof(int));
+        HIPCHK(hipMemcpyAsync(c->d_host2dev.p, c->host2dev.data() + 1, (size_t)c->nhost * sizeof(int),
+                              hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+    }
+    return c->d_host2dev.as<int>();
+}
+
 template <typename TH, typename TD>
-static void to_device_layout(srmg_ctx *c, const TH *host, int G, std::vector<TD> &data, std::vector<TD> &ib) {
+static void host_to_field(srmg_ctx *c, const TH *host, int G, FieldBuf &f) {
     const int D = c->D, M = c->M, S = M + 2 * G;
-    const size_t SD = (D == 2) ? (size_t)S * S : (size_t)S * S * S;
-    data.assign((size_t)c->nb * c->V, TD(0));
-    ib.assign((size_t)std::max(c->nslot, 1) * c->F, TD(0));
-    auto hoff = [&](int x, int y, int z) {  // 0-based valid coords (may be -1 / M)
-        return (size_t)(x + G) + (size_t)S * ((size_t)(y + G) + (D == 3 ? (size_t)S * (size_t)(z + G) : 0));
-    };
-    for (int b = 0; b < c->nb; b++) {
-        const TH *hb = host + (size_t)(c->dev2host[b] - 1) * SD;
-        TD *db = data.data() + (size_t)b * c->V;
-        int nz = (D == 3) ? M : 1;
-        for (int z = 0; z < nz; z++)
-            for (int y = 0; y < M; y++)
-                for (int x = 0; x < M; x++) {
-                    int odd = (x + y + z + D) & 1;
-                    int pos = (odd ? 0 : c->V / 2) + (x >> 1) + (M / 2) * (y + M * z);
-                    db[pos] = (TD)hb[hoff(x, y, z)];
-                }
+    const size_t SP = (D == 2) ? (size_t)S : (size_t)S * S, SD = SP * S;
+    // of a block, the planes of the last dimension within one cell of the valid ones
+    const size_t PB = SP * (M + 2), skip = SP * (G - 1);
+    HostStage &st = c->stage;
+    st.reserve((size_t)c->nhost * PB * sizeof(TH), PB * sizeof(TH));
+    const int64_t per = (int64_t)(st.bytes / (PB * sizeof(TH)));
+    const int *h2d = host_table(c);
+    int k = 0;
+    for (int64_t h0 = 0; h0 < c->nhost; h0 += per, k++) {
+        const int64_t n = std::min(per, c->nhost - h0);
+        st.wait(k);
+        TH *dst = reinterpret_cast<TH *>(st.host(k));
+        const TH *src = host + (size_t)h0 * SD + skip;
+        if (PB == SD)
+            std::memcpy(dst, src, (size_t)n * SD * sizeof(TH));
+        else
+            for (int64_t b = 0; b < n; b++) std::memcpy(dst + b * PB, src + b * SD, PB * sizeof(TH));
+        HIPCHK(hipMemcpyAsync(st.device(k), dst, (size_t)n * PB * sizeof(TH), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipEventRecord(st.ev[k % HostStage::SLOTS], c->stream));
+        hipLaunchKernelGGL((k_host_in<TH, TD>), dim3((unsigned)n), dim3(WG), 0, c->stream, f.data.as<TD>(),
+                           f.ib.as<TD>(), reinterpret_cast<const TH *>(st.device(k)), h2d + h0,
+                           c->d_nbr.as<int>(), D, M, G);
     }
-    // depth-1 ghost layer of coarse-fine faces
-    for (int k = 0; k < c->nslot; k++) {
-        int4 s = c->h_slots[k];
-        int dim = s.y >> 1, dir = (s.y & 1) ? 1 : -1;
-        const TH *hb = host + (size_t)(c->dev2host[s.x] - 1) * SD;
-        for (int t = 0; t < c->F; t++) {
-            int cc[3] = {0, 0, 0};
-            int ta = t % M, tb = t / M;
-            if (dim == 0) { cc[1] = ta; cc[2] = tb; }
-            else if (dim == 1) { cc[0] = ta; cc[2] = tb; }
-            else { cc[0] = ta; cc[1] = tb; }
-            cc[dim] = dir < 0 ? -1 : M;
-            ib[(size_t)k * c->F + t] = (TD)hb[hoff(cc[0], cc[1], cc[2])];
+    HIPCHK(hipGetLastError());
+}
+
+// One block of the staged layout (a box of M + 2 cells per dimension, or of M
+// without ghosts) into the host block: the valid cells and the face ghosts.
+// skip: faces whose ghosts stay as they are, one bit each.
+template <typename TH, int M>
+static void box_to_host(TH *hb, const TH *box, int D, int G, int skip) {
+    const int S = M + 2 * G;
+    if (G == 0) {
+        std::memcpy(hb, box, (D == 2 ? M * M : M * M * M) * sizeof(TH));
+        return;
+    }
+    constexpr int B = M + 2;
+    for (int z = D == 3 ? -1 : 0; z < (D == 3 ? M + 1 : 1); z++)
+        for (int y = -1; y <= M; y++) {
+            const int yo = y < 0 ? 4 : (y == M ? 8 : 0), zo = D == 3 ? (z < 0 ? 16 : (z == M ? 32 : 0)) : 0;
+            if ((yo && zo) || ((yo | zo) & skip)) continue;
+            TH *d = hb + (size_t)S * ((y + G) + (D == 3 ? (size_t)S * (z + G) : 0)) + G;
+            const TH *q = box + (size_t)B * ((y + 1) + (D == 3 ? B * (z + 1) : 0)) + 1;
+            std::memcpy(d, q, M * sizeof(TH));
+            if (yo | zo) continue;
+            if (!(skip & 1)) d[-1] = q[-1];
+            if (!(skip & 2)) d[M] = q[M];
         }
-    }
 }
 
 template <typename TD, typename TH>
-static void from_device_layout(srmg_ctx *c, const std::vector<TD> &data, const std::vector<TD> &ib, TH *host,
-                               int G, const int8_t *bcsign /* may be null: boundary ghosts untouched */) {
-    const int D = c->D, M = c->M, S = M + 2 * G, V = c->V, ND = 2 * D;
+static void field_to_host(srmg_ctx *c, FieldBuf &f, TH *host, int G,
+                          const int8_t *bcsign /* may be null: boundary ghosts untouched */) {
+    const int D = c->D, M = c->M, S = M + 2 * G, ND = 2 * D;
     const size_t SD = (D == 2) ? (size_t)S * S : (size_t)S * S * S;
-    auto hoff = [&](int x, int y, int z) {
-        return (size_t)(x + G) + (size_t)S * ((size_t)(y + G) + (D == 3 ? (size_t)S * (size_t)(z + G) : 0));
+    const int B = G ? M + 2 : M;
+    const size_t BX = (D == 2) ? (size_t)B * B : (size_t)B * B * B;
+    HostStage &st = c->stage;
+    st.reserve((size_t)c->nhost * BX * sizeof(TH), BX * sizeof(TH));
+    const int64_t per = (int64_t)(st.bytes / (BX * sizeof(TH)));
+    const int *h2d = host_table(c);
+    const int np = (int)((c->nhost + per - 1) / per);
+    Faces6 sg;
+    for (int q = 0; q < 6; q++) sg.s[q] = bcsign ? bcsign[q] : 1;
+    auto issue = [&](int k) {
+        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
+        hipLaunchKernelGGL((k_host_out<TD, TH>), dim3((unsigned)n), dim3(WG), 0, c->stream,
+                           reinterpret_cast<TH *>(st.device(k)), f.data.as<TD>(), f.ib.as<TD>(), h2d + h0,
+                           c->d_nbr.as<int>(), D, M, G ? 1 : 0, sg);
+        HIPCHK(hipMemcpyAsync(st.host(k), st.device(k), (size_t)n * BX * sizeof(TH), hipMemcpyDeviceToHost,
+                              c->stream));
+        HIPCHK(hipEventRecord(st.ev[k % HostStage::SLOTS], c->stream));
     };
-    auto dpos = [&](int x, int y, int z) {
-        int odd = (x + y + z + D) & 1;
-        return (odd ? 0 : V / 2) + (x >> 1) + (M / 2) * (y + M * z);
-    };
-    int nz = (D == 3) ? M : 1;
-    for (int b = 0; b < c->nb; b++) {
-        TH *hb = host + (size_t)(c->dev2host[b] - 1) * SD;
-        const TD *db = data.data() + (size_t)b * V;
-        for (int z = 0; z < nz; z++)
-            for (int y = 0; y < M; y++)
-                for (int x = 0; x < M; x++) hb[hoff(x, y, z)] = (TH)db[dpos(x, y, z)];
-        if (G < 1) continue;
-        // depth-1 face ghosts
-        for (int f = 0; f < ND; f++) {
-            int dim = f >> 1, dir = (f & 1) ? 1 : -1;
-            int t_ = c->h_nbr[(size_t)b * ND + f];
-            if (t_ == NB_BOUNDARY && !bcsign) continue;
-            for (int t = 0; t < c->F; t++) {
-                int cc[3] = {0, 0, 0};
-                int ta = t % M, tb = t / M;
-                if (dim == 0) { cc[1] = ta; cc[2] = tb; }
-                else if (dim == 1) { cc[0] = ta; cc[2] = tb; }
-                else { cc[0] = ta; cc[1] = tb; }
-                int g[3] = {cc[0], cc[1], cc[2]};
-                g[dim] = dir < 0 ? -1 : M;
-                TH v;
-                if (t_ >= 0) {
-                    int w[3] = {cc[0], cc[1], cc[2]};
-                    w[dim] = dir < 0 ? M - 1 : 0;
-                    v = (TH)data[(size_t)t_ * V + dpos(w[0], w[1], w[2])];
-                } else if (t_ == NB_BOUNDARY) {
-                    int w[3] = {cc[0], cc[1], cc[2]};
-                    w[dim] = dir < 0 ? 0 : M - 1;
-                    v = (TH)bcsign[f] * (TH)db[dpos(w[0], w[1], w[2])];
-                } else {
-                    v = (TH)ib[(size_t)nb_slot(t_) * c->F + t];
-                }
-                hb[hoff(g[0], g[1], g[2])] = v;
-            }
+    auto place = [&](int k) {
+        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
+        const TH *box = reinterpret_cast<const TH *>(st.host(k));
+        for (int64_t i = 0; i < n; i++) {
+            const int b = c->host2dev[h0 + i + 1];
+            if (b < 0) continue;
+            int skip = 0;
+            if (!bcsign)
+                for (int q = 0; q < ND; q++)
+                    if (c->h_nbr[(size_t)b * ND + q] == NB_BOUNDARY) skip |= 1 << q;
+            if (M == 16) box_to_host<TH, 16>(host + (size_t)(h0 + i) * SD, box + i * BX, D, G, skip);
+            else box_to_host<TH, 8>(host + (size_t)(h0 + i) * SD, box + i * BX, D, G, skip);
         }
+    };
+    // a few pieces: this thread places them; more: a thread per slot does, as
+    // one thread places 8 to 10 GB/s of rows and the bus brings 50
+    if (np <= HostStage::SLOTS) {
+        for (int k = 0; k < np; k++) issue(k);
+        for (int k = 0; k < np; k++) {
+            st.wait(k);
+            place(k);
+        }
+        return;
     }
+    int device = 0;
+    HIPCHK(hipGetDevice(&device));
+    std::atomic<int> issued{0}, failed{0};
+    std::array<std::atomic<int>, HostStage::SLOTS> placed;  // pieces placed from each slot
+    for (auto &p : placed) p = 0;
+    std::vector<std::thread> th;
+    auto join = [&] {
+        for (auto &t : th) t.join();
+    };
+    try {
+        for (int w = 0; w < HostStage::SLOTS; w++)
+            th.emplace_back([&, w] {
+                if (hipSetDevice(device) != hipSuccess) failed = 1;
+                for (int k = w; k < np && !failed; k += HostStage::SLOTS) {
+                    while (issued <= k && !failed) std::this_thread::yield();
+                    if (failed) return;
+                    if (hipEventSynchronize(st.ev[w]) != hipSuccess) {
+                        failed = 1;
+                        return;
+                    }
+                    place(k);
+                    placed[w]++;
+                }
+            });
+        for (int k = 0; k < np && !failed; k++) {
+            while (placed[k % HostStage::SLOTS] < k / HostStage::SLOTS && !failed) std::this_thread::yield();
+            if (failed) break;
+            issue(k);
+            issued = k + 1;
+        }
+    } catch (...) {
+        failed = 1;
+        join();
+        throw;
+    }
+    join();
+    if (failed) fail("copying the field to the host failed", 2);
 }
 
 // ---------------------------------------------------------------------------
@@ -2770,19 +2885,9 @@ int srmg_upload(srmg_ctx *c, int id, const void *host, int host_dtype, int G) {
         auto go = [&](auto th) {
             using TH = decltype(th);
             const TH *h = static_cast<const TH *>(host);
-            if (f.dtype == SRMG_F64) {
-                std::vector<double> data, ib;
-                to_device_layout(c, h, G, data, ib);
-                HIPCHK(hipMemcpy(f.data.p, data.data(), data.size() * 8, hipMemcpyHostToDevice));
-                HIPCHK(hipMemcpy(f.ib.p, ib.data(), ib.size() * 8, hipMemcpyHostToDevice));
-            } else {
-                std::vector<float> data, ib;
-                to_device_layout(c, h, G, data, ib);
-                HIPCHK(hipMemcpy(f.data.p, data.data(), data.size() * 4, hipMemcpyHostToDevice));
-                HIPCHK(hipMemcpy(f.ib.p, ib.data(), ib.size() * 4, hipMemcpyHostToDevice));
-            }
+            if (f.dtype == SRMG_F64) host_to_field<TH, double>(c, h, G, f);
+            else host_to_field<TH, float>(c, h, G, f);
         };
-        HIPCHK(hipStreamSynchronize(c->stream));
         std::fill(f.cur.begin(), f.cur.end(), 0);
         if (host_dtype == SRMG_F64) go(double());
         else if (host_dtype == SRMG_F32) go(float());
@@ -2797,7 +2902,6 @@ static int download_impl(srmg_ctx *c, int id, void *host, int host_dtype, int G,
         if (!host) fail("null host pointer");
         if (G < 0) fail("bad G");
         if (!f.settled()) dispatch(c, f.dtype, [&](auto &o) { o.settle(f); });
-        HIPCHK(hipStreamSynchronize(c->stream));
         int8_t sg[6] = {1, 1, 1, 1, 1, 1};
         if (bc)
             for (int d = 0; d < c->D; d++)
@@ -2811,13 +2915,10 @@ static int download_impl(srmg_ctx *c, int id, void *host, int host_dtype, int G,
                 }
         auto go = [&](auto td) {
             using TD = decltype(td);
-            std::vector<TD> data(f.data.bytes / sizeof(TD)), ib(f.ib.bytes / sizeof(TD));
-            HIPCHK(hipMemcpy(data.data(), f.data.p, f.data.bytes, hipMemcpyDeviceToHost));
-            HIPCHK(hipMemcpy(ib.data(), f.ib.p, f.ib.bytes, hipMemcpyDeviceToHost));
             if (host_dtype == SRMG_F64)
-                from_device_layout(c, data, ib, static_cast<double *>(host), G, bc ? sg : nullptr);
+                field_to_host<TD, double>(c, f, static_cast<double *>(host), G, bc ? sg : nullptr);
             else
-                from_device_layout(c, data, ib, static_cast<float *>(host), G, bc ? sg : nullptr);
+                field_to_host<TD, float>(c, f, static_cast<float *>(host), G, bc ? sg : nullptr);
         };
         if (host_dtype != SRMG_F64 && host_dtype != SRMG_F32) fail("bad host dtype");
         if (f.dtype == SRMG_F64) go(double());
