@@ -697,35 +697,38 @@ __device__ __forceinline__ int rt_sidx(int D, int M, int x, int y, int z) {
     return (((x + y + z + D) & 1) ? 0 : V / 2) + (x >> 1) + (M / 2) * (y + M * z);
 }
 
-// Staged host blocks -> device blocks (one work group each): the planes of the
-// last dimension from one cell below the valid ones to one above, S = M + 2 G
-// cells in the other dimensions. Valid cells, and the depth-1 ghosts of
-// coarse-fine faces into their slabs.
+// Host blocks in the pinned ring -> device blocks (one work group each): the
+// planes of the last dimension from one cell below the valid ones to one above,
+// S = M + 2 G cells in the other dimensions, read once and in order, as the bus
+// likes it. Valid cells, and the depth-1 ghosts of coarse-fine faces into their
+// slabs.
 template <typename TH, typename TD>
 __global__ __launch_bounds__(WG) void k_host_in(TD *__restrict__ data, TD *__restrict__ ib, const TH *__restrict__ src,
                                                 const int *__restrict__ host2dev, const int *__restrict__ nbr, int D,
                                                 int M, int G) {
     const int b = host2dev[blockIdx.x];
     if (b < 0) return;
-    const int S = M + 2 * G, V = D == 2 ? M * M : M * M * M, F = V / M, H = V / 2, MH = M / 2;
-    const TH *p = src + (size_t)blockIdx.x * (D == 2 ? S : S * S) * (M + 2);
-    auto at = [&](int x, int y, int z) {
-        return D == 2 ? (size_t)S * (y + 1) + x + G : (size_t)S * ((size_t)S * (z + 1) + y + G) + x + G;
-    };
-    for (int q = threadIdx.x; q < V; q += WG) {
-        const int h = q >= H ? 1 : 0, r = q - h * H, row = r / MH, y = row % M, z = row / M;
-        const int x = 2 * (r % MH) + (((h ^ 1) ^ (y + z + D)) & 1);
-        data[(size_t)b * V + q] = (TD)p[at(x, y, z)];
-    }
-    for (int f = 0; f < 2 * D; f++) {
-        const int t = nbr[(size_t)b * 2 * D + f];
-        if (t > -2) continue;
-        const int dim = f >> 1, n = (f & 1) ? M : -1;
-        for (int i = threadIdx.x; i < F; i += WG) {
-            const int a = i % M, c = i / M;
-            const TH v = dim == 0 ? p[at(n, a, c)] : dim == 1 ? p[at(a, n, c)] : p[at(a, c, n)];
-            ib[(size_t)nb_slot(t) * F + i] = (TD)v;
+    const int S = M + 2 * G, V = D == 2 ? M * M : M * M * M, F = V / M;
+    const int n = (D == 2 ? S : S * S) * (M + 2);
+    const TH *p = src + (size_t)blockIdx.x * n;
+    for (int i = threadIdx.x; i < n; i += WG) {
+        const TH v = p[i];
+        const int r = i / S;
+        const int x[3] = {i % S - G, D == 2 ? r - 1 : r % S - G, D == 2 ? 0 : r / S - 1};
+        int f = -1, out = 0;
+        for (int d = 0; d < D; d++)
+            if (x[d] < 0 || x[d] >= M) {
+                out += x[d] < -1 || x[d] > M ? 2 : 1;
+                f = 2 * d + (x[d] < 0 ? 0 : 1);
+            }
+        if (out > 1) continue;
+        if (out == 0) {
+            data[(size_t)b * V + rt_sidx(D, M, x[0], x[1], x[2])] = (TD)v;
+            continue;
         }
+        const int t = nbr[(size_t)b * 2 * D + f], dim = f >> 1;
+        const int a = dim == 0 ? x[1] : x[0], c = dim == 2 ? x[1] : x[2];
+        if (t <= -2) ib[(size_t)nb_slot(t) * F + a + M * c] = (TD)v;
     }
 }
 
@@ -734,7 +737,7 @@ struct Faces6 {
 };
 
 // Device blocks -> boxes of M + 2 g cells per dimension (g = 0 or 1) in the
-// order of the host's block ids (one work group each): valid cells and, with
+// pinned ring, in the order of the host's block ids (one work group each): valid cells and, with
 // g = 1, the face ghosts (copies, +-mirrors, slabs); edges and corners are not
 // written.
 template <typename TD, typename TH>

@@ -99,18 +99,17 @@ struct Graph {
     }
 };
 
-// Pinned host buffers and their device counterparts, through which host fields
+// Pinned host buffers that kernels read and write, through which host fields
 // pass in pieces (srmg_upload, srmg_download): a ring of SLOTS, kept by the
-// context, at most SLOTS x MAX_BYTES on either side (more only where one block needs it).
+// context, at most SLOTS x MAX_BYTES (more only where one block needs it).
 struct HostStage {
-    static constexpr int SLOTS = 4;
-    static constexpr size_t MIN_BYTES = (size_t)64 << 10, MAX_BYTES = (size_t)2 << 20;
+    static constexpr int SLOTS = 8;
+    static constexpr size_t MIN_BYTES = (size_t)64 << 10, MAX_BYTES = (size_t)1 << 20;
     size_t bytes = 0;  // of a slot
-    char *pin = nullptr;
-    DevBuf dev;
-    hipEvent_t ev[SLOTS] = {};  // the slot's last copy has ended
+    char *pin = nullptr, *map = nullptr;  // the host's and the device's address
+    hipEvent_t ev[SLOTS] = {};            // the slot's last kernel has ended
     char *host(int k) { return pin + (size_t)(k % SLOTS) * bytes; }
-    char *device(int k) { return dev.as<char>() + (size_t)(k % SLOTS) * bytes; }
+    char *device(int k) { return map + (size_t)(k % SLOTS) * bytes; }
     void wait(int k) { HIPCHK(hipEventSynchronize(ev[k % SLOTS])); }
     // slots that hold `total` bytes, or as much of them as a slot may; at
     // least one block of `block` bytes
@@ -121,7 +120,7 @@ struct HostStage {
         release();
         for (auto &e : ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         HIPCHK(hipHostMalloc((void **)&pin, want * SLOTS, hipHostMallocDefault));
-        dev.alloc(want * SLOTS);
+        HIPCHK(hipHostGetDevicePointer((void **)&map, pin, 0));
         bytes = want;
     }
     void release() {
@@ -133,8 +132,7 @@ struct HostStage {
             e = nullptr;
         }
         if (pin) (void)hipHostFree(pin);
-        pin = nullptr;
-        dev.release();
+        pin = map = nullptr;
         bytes = 0;
     }
     ~HostStage() { release(); }
@@ -1952,12 +1950,12 @@ static int same_type(srmg_ctx *c, std::initializer_list<int> ids) {
 // ---------------------------------------------------------------------------
 
 // Host fields cross the bus in the caller's own layout, piece by piece through
-// the context's staging ring, and kernels convert between that and the device
-// layout (k_host_in, k_host_out): the host only copies contiguous rows, while
-// the previous piece is on the bus. Bound by the bus (52 GB/s pinned on an
-// MI355X host) and by the host's copies (30 to 45 GB/s); converted cell by cell
-// on the host, a V-cycle with two fields each way took 21.8 ms on a 2D tree of
-// 7,716 blocks of 16^2.
+// the context's pinned ring: kernels read or write the ring and convert between
+// the host's and the device's layout (k_host_in, k_host_out), the host only
+// copies contiguous rows, while other pieces are on the bus. Bound by the bus
+// and the host's copies; converted cell by cell on the host and copied through
+// pageable memory, a V-cycle with two fields each way took 20.4 ms on a 2D tree
+// of 7,716 blocks of 16^2, now 3.3 ms.
 
 static const int *host_table(srmg_ctx *c) {
     if (!c->d_host2dev.p) {
@@ -1970,6 +1968,69 @@ static const int *host_table(srmg_ctx *c) {
     return c->d_host2dev.as<int>();
 }
 
+// The pieces 0 .. np-1 of a field, in order on this thread (which talks to the
+// device) and, where there are more than the ring holds, with a thread per slot
+// for the host's copies: one thread copies 20 to 30 GB/s in and places 8 to 10
+// GB/s of rows, the bus moves 50. in: copy(k) into slot k % SLOTS, then
+// issue(k); out: issue(k), then copy(k) once the slot's event has come.
+template <class Copy, class Issue>
+static void pipe_pieces(HostStage &st, int np, bool in, Copy &&copy, Issue &&issue) {
+    constexpr int W = HostStage::SLOTS;
+    if (np <= W) {
+        for (int k = 0; k < np; k++) {
+            if (in) {
+                st.wait(k);
+                copy(k);
+            }
+            issue(k);
+        }
+        for (int k = 0; k < np && !in; k++) {
+            st.wait(k);
+            copy(k);
+        }
+        return;
+    }
+    int device = 0;
+    HIPCHK(hipGetDevice(&device));
+    std::atomic<bool> failed{false};
+    std::array<std::atomic<int>, W> issued, copied;  // pieces of each slot
+    for (int w = 0; w < W; w++) issued[w] = copied[w] = 0;
+    std::vector<std::thread> th;
+    auto until = [&](const std::atomic<int> &n, int least) {
+        while (n < least && !failed) std::this_thread::yield();
+        return !failed;
+    };
+    auto join = [&] {
+        for (auto &t : th) t.join();
+    };
+    try {
+        for (int w = 0; w < W; w++)
+            th.emplace_back([&, w] {
+                if (hipSetDevice(device) != hipSuccess) failed = true;
+                for (int k = w, n = 0; k < np; k += W, n++) {
+                    // in: the piece before has been sent from this slot; out: this one is on its way into it
+                    if (!until(issued[w], in ? n : n + 1)) return;
+                    if (hipEventSynchronize(st.ev[w]) != hipSuccess) {
+                        failed = true;
+                        return;
+                    }
+                    copy(k);
+                    copied[w]++;
+                }
+            });
+        for (int k = 0; k < np && until(copied[k % W], in ? k / W + 1 : k / W); k++) {
+            issue(k);
+            issued[k % W]++;
+        }
+    } catch (...) {
+        failed = true;
+        join();
+        throw;
+    }
+    join();
+    if (failed) fail("copying a field between host and device failed", 2);
+}
+
 template <typename TH, typename TD>
 static void host_to_field(srmg_ctx *c, const TH *host, int G, FieldBuf &f) {
     const int D = c->D, M = c->M, S = M + 2 * G;
@@ -1980,23 +2041,24 @@ static void host_to_field(srmg_ctx *c, const TH *host, int G, FieldBuf &f) {
     st.reserve((size_t)c->nhost * PB * sizeof(TH), PB * sizeof(TH));
     const int64_t per = (int64_t)(st.bytes / (PB * sizeof(TH)));
     const int *h2d = host_table(c);
-    int k = 0;
-    for (int64_t h0 = 0; h0 < c->nhost; h0 += per, k++) {
-        const int64_t n = std::min(per, c->nhost - h0);
-        st.wait(k);
+    const int np = (int)((c->nhost + per - 1) / per);
+    auto copy = [&](int k) {
+        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
         TH *dst = reinterpret_cast<TH *>(st.host(k));
         const TH *src = host + (size_t)h0 * SD + skip;
         if (PB == SD)
             std::memcpy(dst, src, (size_t)n * SD * sizeof(TH));
         else
             for (int64_t b = 0; b < n; b++) std::memcpy(dst + b * PB, src + b * SD, PB * sizeof(TH));
-        HIPCHK(hipMemcpyAsync(st.device(k), dst, (size_t)n * PB * sizeof(TH), hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipEventRecord(st.ev[k % HostStage::SLOTS], c->stream));
+    };
+    pipe_pieces(st, np, true, copy, [&](int k) {
+        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
         hipLaunchKernelGGL((k_host_in<TH, TD>), dim3((unsigned)n), dim3(WG), 0, c->stream, f.data.as<TD>(),
                            f.ib.as<TD>(), reinterpret_cast<const TH *>(st.device(k)), h2d + h0,
                            c->d_nbr.as<int>(), D, M, G);
-    }
-    HIPCHK(hipGetLastError());
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipEventRecord(st.ev[k % HostStage::SLOTS], c->stream));
+    });
 }
 
 // One block of the staged layout (a box of M + 2 cells per dimension, or of M
@@ -2042,8 +2104,7 @@ static void field_to_host(srmg_ctx *c, FieldBuf &f, TH *host, int G,
         hipLaunchKernelGGL((k_host_out<TD, TH>), dim3((unsigned)n), dim3(WG), 0, c->stream,
                            reinterpret_cast<TH *>(st.device(k)), f.data.as<TD>(), f.ib.as<TD>(), h2d + h0,
                            c->d_nbr.as<int>(), D, M, G ? 1 : 0, sg);
-        HIPCHK(hipMemcpyAsync(st.host(k), st.device(k), (size_t)n * BX * sizeof(TH), hipMemcpyDeviceToHost,
-                              c->stream));
+        HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(st.ev[k % HostStage::SLOTS], c->stream));
     };
     auto place = [&](int k) {
@@ -2060,53 +2121,7 @@ static void field_to_host(srmg_ctx *c, FieldBuf &f, TH *host, int G,
             else box_to_host<TH, 8>(host + (size_t)(h0 + i) * SD, box + i * BX, D, G, skip);
         }
     };
-    // a few pieces: this thread places them; more: a thread per slot does, as
-    // one thread places 8 to 10 GB/s of rows and the bus brings 50
-    if (np <= HostStage::SLOTS) {
-        for (int k = 0; k < np; k++) issue(k);
-        for (int k = 0; k < np; k++) {
-            st.wait(k);
-            place(k);
-        }
-        return;
-    }
-    int device = 0;
-    HIPCHK(hipGetDevice(&device));
-    std::atomic<int> issued{0}, failed{0};
-    std::array<std::atomic<int>, HostStage::SLOTS> placed;  // pieces placed from each slot
-    for (auto &p : placed) p = 0;
-    std::vector<std::thread> th;
-    auto join = [&] {
-        for (auto &t : th) t.join();
-    };
-    try {
-        for (int w = 0; w < HostStage::SLOTS; w++)
-            th.emplace_back([&, w] {
-                if (hipSetDevice(device) != hipSuccess) failed = 1;
-                for (int k = w; k < np && !failed; k += HostStage::SLOTS) {
-                    while (issued <= k && !failed) std::this_thread::yield();
-                    if (failed) return;
-                    if (hipEventSynchronize(st.ev[w]) != hipSuccess) {
-                        failed = 1;
-                        return;
-                    }
-                    place(k);
-                    placed[w]++;
-                }
-            });
-        for (int k = 0; k < np && !failed; k++) {
-            while (placed[k % HostStage::SLOTS] < k / HostStage::SLOTS && !failed) std::this_thread::yield();
-            if (failed) break;
-            issue(k);
-            issued = k + 1;
-        }
-    } catch (...) {
-        failed = 1;
-        join();
-        throw;
-    }
-    join();
-    if (failed) fail("copying the field to the host failed", 2);
+    pipe_pieces(st, np, false, place, issue);
 }
 
 // ---------------------------------------------------------------------------
