@@ -3491,6 +3491,157 @@ __global__ __launch_bounds__(L1T) void k_l1_inv_yx(T *__restrict__ dst, double *
     }
 }
 
+// ---- the same for many stacked grids ----
+//
+// With hundreds of planes the launches are bound by FP64 arithmetic (a product
+// and a sum each, 39 T/s on the chip), not by latency, and the split of a plane
+// over work groups repeats its loads. Here a work group takes a whole plane
+// (or 64 columns along z): lanes along one axis, and per wave eight (four)
+// output rows at once, so that one LDS read per lane and k serves eight sums
+// and the matrix row, equal for all lanes, comes through scalar loads. A work
+// group reads its whole plane before it writes, so a launch may write in place.
+// Same sums in the same order as k_l1_fwd_xy, k_l1_z and k_l1_inv_yx.
+
+// rows row0 .. row0 + RB - 1 of A (n x n, row-major, n a multiple of 8) times
+// the lane's vector x[k ks], into acc
+template <int RB>
+__device__ __forceinline__ void l1b_rows(double (&acc)[RB], const double *__restrict__ A, int row0, int n,
+                                         const double *x, int ks) {
+#pragma unroll
+    for (int r = 0; r < RB; r++) acc[r] = 0.0;
+    const double *a = A + (size_t)row0 * n;
+    for (int k = 0; k < n; k += 8) {
+        double xk[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) xk[i] = x[(k + i) * ks];
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) acc[r] += a[(size_t)r * n + k + i] * xk[i];
+    }
+}
+
+// forward x, then forward y, of plane blockIdx.x
+template <int RB>
+__global__ __launch_bounds__(L1T) void k_l1b_fwd_xy(double *out, const double *in, const double *__restrict__ A0,
+                                                    const double *__restrict__ A1, int N0, int N1) {
+    constexpr int RW = 16 / RB;  // row groups per wave
+    __shared__ double xs[64 * L1S];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const double *p = in + (size_t)blockIdx.x * N1 * N0;
+    l1_rows(N1, N0, [&](int y, int x) { return p[(size_t)y * N0 + x]; },
+            [&](int y, int x, double v) { xs[y * L1S + x] = v; });
+    __syncthreads();
+    double acc[RW][RB];
+    // Y1[y][i] = sum_k A0[i][k] X[y][k], lane = y
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if ((w + 4 * j) * RB < N0) l1b_rows(acc[j], A0, (w + 4 * j) * RB, N0, xs + lane * L1S, 1);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if ((w + 4 * j) * RB < N0)
+#pragma unroll
+            for (int r = 0; r < RB; r++) xs[lane * L1S + (w + 4 * j) * RB + r] = acc[j][r];
+    __syncthreads();
+    // Y2[j][i] = sum_k A1[j][k] Y1[k][i], lane = i
+    double *po = out + (size_t)blockIdx.x * N1 * N0;
+#pragma unroll
+    for (int j = 0; j < RW; j++) {
+        if ((w + 4 * j) * RB >= N1) continue;
+        double v[RB];
+        l1b_rows(v, A1, (w + 4 * j) * RB, N1, xs + lane, L1S);
+        if (lane < N0)
+#pragma unroll
+            for (int r = 0; r < RB; r++) po[(size_t)((w + 4 * j) * RB + r) * N0 + lane] = v[r];
+    }
+}
+
+// forward z, the eigenvalue division, inverse z of 64 columns (y, x)
+template <int RB>
+__global__ __launch_bounds__(L1T) void k_l1b_z(double *g, const double *__restrict__ A2,
+                                               const double *__restrict__ B2, const double *__restrict__ l0,
+                                               const double *__restrict__ l1, const double *__restrict__ l2,
+                                               const double *__restrict__ shift, int N0, int N1, int N2) {
+    constexpr int RW = 16 / RB;
+    __shared__ double zs[64 * 64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ncb = N0 * N1 / 64, gi = blockIdx.x / ncb, c = (blockIdx.x - gi * ncb) * 64 + lane;
+    const size_t plane = (size_t)N0 * N1;
+    double *p = g + (size_t)gi * N2 * plane + c;
+    l1_rows(N2, 64, [&](int z, int) { return p[(size_t)z * plane]; },
+            [&](int z, int i, double v) { zs[z * 64 + i] = v; });
+    double ev0 = shift[gi];
+    ev0 += l0[c % N0];
+    ev0 += l1[c / N0];
+    __syncthreads();
+    double acc[RW][RB];
+#pragma unroll
+    for (int j = 0; j < RW; j++) {
+        if ((w + 4 * j) * RB >= N2) continue;
+        l1b_rows(acc[j], A2, (w + 4 * j) * RB, N2, zs + lane, 64);
+#pragma unroll
+        for (int r = 0; r < RB; r++) acc[j][r] = acc[j][r] / (ev0 + l2[(w + 4 * j) * RB + r]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if ((w + 4 * j) * RB < N2)
+#pragma unroll
+            for (int r = 0; r < RB; r++) zs[((w + 4 * j) * RB + r) * 64 + lane] = acc[j][r];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RW; j++) {
+        if ((w + 4 * j) * RB >= N2) continue;
+        double v[RB];
+        l1b_rows(v, B2, (w + 4 * j) * RB, N2, zs + lane, 64);
+#pragma unroll
+        for (int r = 0; r < RB; r++) p[(size_t)((w + 4 * j) * RB + r) * plane] = v[r];
+    }
+}
+
+// inverse y, then inverse x, of plane blockIdx.x, in place
+template <int RB>
+__global__ __launch_bounds__(L1T) void k_l1b_inv_yx(double *g, const double *__restrict__ B1,
+                                                    const double *__restrict__ B0, int N0, int N1) {
+    constexpr int RW = 16 / RB;
+    __shared__ double vs[64 * L1S];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double *p = g + (size_t)blockIdx.x * N1 * N0;
+    l1_rows(N1, N0, [&](int y, int x) { return p[(size_t)y * N0 + x]; },
+            [&](int y, int x, double v) { vs[y * L1S + x] = v; });
+    __syncthreads();
+    double acc[RW][RB];
+    // T[j][x] = sum_k B1[j][k] V[k][x], lane = x
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if ((w + 4 * j) * RB < N1) l1b_rows(acc[j], B1, (w + 4 * j) * RB, N1, vs + lane, L1S);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if ((w + 4 * j) * RB < N1)
+#pragma unroll
+            for (int r = 0; r < RB; r++) vs[((w + 4 * j) * RB + r) * L1S + lane] = acc[j][r];
+    __syncthreads();
+    // U[j][i] = sum_k B0[i][k] T[j][k], lane = j; back through LDS so that rows
+    // leave whole
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if ((w + 4 * j) * RB < N0) l1b_rows(acc[j], B0, (w + 4 * j) * RB, N0, vs + lane * L1S, 1);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if ((w + 4 * j) * RB < N0)
+#pragma unroll
+            for (int r = 0; r < RB; r++) vs[lane * L1S + (w + 4 * j) * RB + r] = acc[j][r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int y = w + 4 * r;
+        if (y < N1 && lane < N0) p[(size_t)y * N0 + lane] = vs[y * L1S + lane];
+    }
+}
+
 // ---- mixed precision helpers ----
 
 // u += e over n cells (FP64 += FP32)

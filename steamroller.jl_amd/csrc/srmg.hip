@@ -904,6 +904,30 @@ static void launch_l1_fused(hipStream_t st, int ngrid, const int *N, const T *sr
                        st, dst, gout, w2, btab, P[1] + n11, P[0] + n00, N0, N1, N2);
 }
 
+// From this many z planes on, stacked grids take whole planes per work group
+// (see k_l1b_fwd_xy). Kernel time per solve of 64^3 grids, split planes against
+// whole ones: 4 grids 105 and 128 us, 8 grids 189 and 143, 16 grids 361 and
+// 149, 128 grids 2922 and 1084 (0.6 of the FP64 rate without fused
+// multiply-add; the matrices exceed the scalar cache).
+constexpr int64_t L1B_PLANES = 512;
+
+// the solve of many stacked grids from f to u (which may be the same): u holds
+// the transforms in between
+static void launch_l1_many(hipStream_t st, int ngrid, const int *N, const double *f, const double *const *Q,
+                           const double *const *P, const double *const *lam, const double *shift, double *u) {
+    const unsigned np = (unsigned)(ngrid * N[2]), nc = (unsigned)(ngrid * (N[0] * N[1] / 64));
+    auto go = [&](auto rb) {
+        constexpr int RB = decltype(rb)::value;
+        hipLaunchKernelGGL(k_l1b_fwd_xy<RB>, dim3(np), dim3(L1T), 0, st, u, f, Q[0], Q[1], N[0], N[1]);
+        hipLaunchKernelGGL(k_l1b_z<RB>, dim3(nc), dim3(L1T), 0, st, u, Q[2], P[2], lam[0], lam[1], lam[2], shift, N[0],
+                           N[1], N[2]);
+        hipLaunchKernelGGL(k_l1b_inv_yx<RB>, dim3(np), dim3(L1T), 0, st, u, P[1], P[0], N[0], N[1]);
+    };
+    // eight rows per wave where that gives all four waves the same number
+    if (N[0] % 32 == 0 && N[1] % 32 == 0 && N[2] % 32 == 0) go(std::integral_constant<int, 8>());
+    else go(std::integral_constant<int, 4>());
+}
+
 template <int D, int M, typename T>
 struct Ops {
     using LY = Lay<D, M>;
@@ -3675,6 +3699,12 @@ static void grid_solve_run(srmg_ctx *c, const GridSolvePlan &g, double s, const 
     }
     hold.push_back(std::vector<double>(ngrid, op->disc == SRMG_HELMHOLTZ ? -s * op->k2 : 0.0));
     HIPCHK(hipMemcpyAsync(bufs.shift, hold.back().data(), ngrid * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    if (c->axis_gemm == 2 && l1_fused_ok(dims, N) && (int64_t)ngrid * N[2] >= L1B_PLANES) {
+        launch_l1_many(c->stream, ngrid, N, f, bufs.Q, bufs.P, bufs.lam, bufs.shift, u);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return;
+    }
     if (c->axis_gemm == 2 && l1_fused_ok(dims, N)) {
         launch_l1_fused<8, double, false>(c->stream, ngrid, N, nullptr, f, nullptr, nullptr, bufs.Q, bufs.P,
                                           bufs.lam, bufs.shift, bufs.g1, bufs.g2, nullptr, u);
