@@ -138,8 +138,22 @@ struct HostStage {
     ~HostStage() { release(); }
 };
 
+// One axis of a grid solve on the device (P and Q as axis_matrix_both lays them
+// out) for n cells and its two mirror signs.
+struct AxisPlan {
+    int n = 0;
+    bool radial = false;
+    double lo = 0.0, hi = 0.0;
+    uint64_t used = 0;  // the last call that took it
+    DevBuf lam, P, Q;
+};
+
 struct srmg_ctx {
     HostStage stage;
+    // srmg_grid_solve: the axes of recent calls and its buffers (each kept up to GRID_KEEP bytes)
+    std::vector<std::unique_ptr<AxisPlan>> axes;
+    uint64_t grid_calls = 0;
+    DevBuf gs_shift, gs_g1, gs_g2;
     DevBuf d_host2dev;      // host block id - 1 -> device block, or -1 (made on first use)
     int D = 2, M = 16, V = 0, F = 0;
     int nlevels = 0;
@@ -3665,41 +3679,66 @@ static GridSolvePlan grid_solve_plan(srmg_ctx *c, int D, const int *n, const srm
     return g;
 }
 
-// Separable exact solve of ngrid stacked grids: the operands are computed on
-// the host and copied into bufs on the context's stream, then forward
-// transforms along every axis, the eigenvalue scaling and the inverse
-// transforms, the last one into u. Returns when u is complete.
+// whole planes per work group, in place in u
+static bool grid_solve_many(const srmg_ctx *c, const GridSolvePlan &g, int ngrid) {
+    return c->axis_gemm == 2 && l1_fused_ok(g.dims, g.N) && (int64_t)ngrid * g.N[2] >= L1B_PLANES;
+}
+
+// the mirror signs of axis d at its two ends
+static void axis_signs(int dims, const srmg_op *op, int d, double *lo, double *hi) {
+    int il = 0, ih = 0, m = 1;
+    for (int e = 0; e < dims; e++) {
+        il += ((e == d ? -1 : 0) + 1) * m;
+        ih += ((e == d ? 1 : 0) + 1) * m;
+        m *= 3;
+    }
+    *lo = (double)op->bc[il];
+    *hi = (double)op->bc[ih];
+}
+
+// The device operands of an axis, from the context's recent ones or made now:
+// the eigendecomposition and the copies took 0.3 ms per axis of 64 cells on
+// every call. AXES_KEPT of them stay, the least recently used one goes.
+constexpr size_t AXES_KEPT = 16;
+static AxisPlan &axis_plan(srmg_ctx *c, int n, bool radial, double lo, double hi) {
+    for (auto &p : c->axes)
+        if (p->n == n && p->radial == radial && p->lo == lo && p->hi == hi) {
+            p->used = c->grid_calls;
+            return *p;
+        }
+    if (c->axes.size() >= AXES_KEPT) {
+        HIPCHK(hipStreamSynchronize(c->stream));
+        c->axes.erase(std::min_element(c->axes.begin(), c->axes.end(),
+                                       [](const auto &a, const auto &b) { return a->used < b->used; }));
+    }
+    auto p = std::make_unique<AxisPlan>();
+    p->n = n;
+    p->radial = radial;
+    p->lo = lo;
+    p->hi = hi;
+    p->used = c->grid_calls;
+    std::vector<double> lam(n), P((size_t)n * n), Q((size_t)n * n);
+    axis_decomp(n, radial, lo, hi, lam.data(), P.data(), Q.data());
+    p->lam.alloc(n * sizeof(double));
+    HIPCHK(hipMemcpy(p->lam.p, lam.data(), n * sizeof(double), hipMemcpyHostToDevice));
+    upload_axis_matrix(p->P, P, n);
+    upload_axis_matrix(p->Q, Q, n);
+    c->axes.push_back(std::move(p));
+    return *c->axes.back();
+}
+
+// Separable exact solve of ngrid stacked grids with the operands in bufs, on
+// the context's stream: forward transforms along every axis, the eigenvalue
+// scaling and the inverse transforms, the last one into u. Returns when u is
+// complete.
 static void grid_solve_run(srmg_ctx *c, const GridSolvePlan &g, double s, const srmg_op *op, const double *f,
                            double *u, int ngrid, const GridSolveBufs &bufs) {
     const int *N = g.N;
     const size_t total = g.total;
-    // host operands stay alive until the stream is synchronized below
-    std::vector<std::vector<double>> hold;
-    hold.reserve(3 * 3 + 1);
     const int dims = g.dims;
-    for (int d = 0; d < dims; d++) {
-        int il = 0, ih = 0, m = 1;
-        for (int e = 0; e < dims; e++) {
-            il += ((e == d ? -1 : 0) + 1) * m;
-            ih += ((e == d ? 1 : 0) + 1) * m;
-            m *= 3;
-        }
-        const int nd = N[d];
-        std::vector<double> hl(nd), hP((size_t)nd * nd), hQ((size_t)nd * nd);
-        axis_decomp(nd, d == g.rdim, (double)op->bc[il], (double)op->bc[ih], hl.data(), hP.data(), hQ.data());
-        hold.push_back(std::move(hl));
-        HIPCHK(hipMemcpyAsync(bufs.lam[d], hold.back().data(), nd * sizeof(double), hipMemcpyHostToDevice,
-                              c->stream));
-        hold.push_back(axis_matrix_both(hP, nd));
-        HIPCHK(hipMemcpyAsync(bufs.P[d], hold.back().data(), hold.back().size() * sizeof(double),
-                              hipMemcpyHostToDevice, c->stream));
-        hold.push_back(axis_matrix_both(hQ, nd));
-        HIPCHK(hipMemcpyAsync(bufs.Q[d], hold.back().data(), hold.back().size() * sizeof(double),
-                              hipMemcpyHostToDevice, c->stream));
-    }
-    hold.push_back(std::vector<double>(ngrid, op->disc == SRMG_HELMHOLTZ ? -s * op->k2 : 0.0));
-    HIPCHK(hipMemcpyAsync(bufs.shift, hold.back().data(), ngrid * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (c->axis_gemm == 2 && l1_fused_ok(dims, N) && (int64_t)ngrid * N[2] >= L1B_PLANES) {
+    hipLaunchKernelGGL(k_fill<double>, dim3(nwg(ngrid)), dim3(WG), 0, c->stream, bufs.shift,
+                       op->disc == SRMG_HELMHOLTZ ? -s * op->k2 : 0.0, (size_t)ngrid);
+    if (grid_solve_many(c, g, ngrid)) {
         launch_l1_many(c->stream, ngrid, N, f, bufs.Q, bufs.P, bufs.lam, bufs.shift, u);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -3760,19 +3799,30 @@ int srmg_grid_solve(srmg_ctx *c, int D, const int *n, double s, const srmg_op *o
                     int ngrid) {
     return guarded([&] {
         GridSolvePlan g = grid_solve_plan(c, D, n, op, f, u, ngrid);
-        DevBuf P[3], Q[3], lam[3], shift, g1, g2;
         GridSolveBufs bufs{};
+        c->grid_calls++;
         for (int d = 0; d < D; d++) {
-            lam[d].alloc(g.N[d] * sizeof(double));
-            P[d].alloc(2 * (size_t)g.N[d] * g.N[d] * sizeof(double));
-            Q[d].alloc(2 * (size_t)g.N[d] * g.N[d] * sizeof(double));
-            bufs.lam[d] = lam[d].as<double>();
-            bufs.P[d] = P[d].as<double>();
-            bufs.Q[d] = Q[d].as<double>();
+            double lo, hi;
+            axis_signs(D, op, d, &lo, &hi);
+            AxisPlan &p = axis_plan(c, g.N[d], d == g.rdim, lo, hi);
+            bufs.lam[d] = p.lam.as<double>();
+            bufs.P[d] = p.P.as<double>();
+            bufs.Q[d] = p.Q.as<double>();
         }
-        shift.alloc(ngrid * sizeof(double));
-        g1.alloc(g.total * ngrid * sizeof(double));
-        g2.alloc(g.total * ngrid * sizeof(double));
+        // the two grids in between, where the kernels need them (launch_l1_many
+        // does not); small ones stay with the context
+        constexpr size_t GRID_KEEP = (size_t)64 << 20;
+        const bool many = grid_solve_many(c, g, ngrid);
+        const size_t bytes = many ? 16 : g.total * ngrid * sizeof(double);
+        DevBuf l1, l2, l3;
+        DevBuf &g1 = bytes > GRID_KEEP ? l1 : c->gs_g1, &g2 = bytes > GRID_KEEP ? l2 : c->gs_g2;
+        DevBuf &shift = ngrid * sizeof(double) > GRID_KEEP ? l3 : c->gs_shift;
+        auto grow = [](DevBuf &b, size_t n) {
+            if (b.cap < n) b.alloc(n);
+        };
+        grow(shift, ngrid * sizeof(double));
+        grow(g1, bytes);
+        grow(g2, bytes);
         bufs.shift = shift.as<double>();
         bufs.g1 = g1.as<double>();
         bufs.g2 = g2.as<double>();
@@ -3805,6 +3855,24 @@ int srmg_grid_solve_noalloc(srmg_ctx *c, int D, const int *n, double s, const sr
         if (off > NOALLOC_SCRATCH_BYTES)
             fail("srmg_grid_solve_noalloc: the grids need " + std::to_string(off) + " bytes of scratch, above the " +
                  std::to_string(NOALLOC_SCRATCH_BYTES) + "-byte maximum (use srmg_grid_solve)");
+        // host operands stay alive until grid_solve_run has synchronized the stream
+        std::vector<std::vector<double>> hold;
+        hold.reserve(3 * 3);
+        auto put = [&](double *dst, std::vector<double> v) {
+            hold.push_back(std::move(v));
+            HIPCHK(hipMemcpyAsync(dst, hold.back().data(), hold.back().size() * sizeof(double),
+                                  hipMemcpyHostToDevice, c->stream));
+        };
+        for (int d = 0; d < D; d++) {
+            const int nd = g.N[d];
+            double lo, hi;
+            axis_signs(D, op, d, &lo, &hi);
+            std::vector<double> hl(nd), hP((size_t)nd * nd), hQ((size_t)nd * nd);
+            axis_decomp(nd, d == g.rdim, lo, hi, hl.data(), hP.data(), hQ.data());
+            put(bufs.lam[d], std::move(hl));
+            put(bufs.P[d], axis_matrix_both(hP, nd));
+            put(bufs.Q[d], axis_matrix_both(hQ, nd));
+        }
         grid_solve_run(c, g, s, op, f, u, ngrid, bufs);
     });
 }
