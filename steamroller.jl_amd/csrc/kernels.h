@@ -3239,6 +3239,114 @@ __global__ __launch_bounds__(WG) void k_eig_scale(double *__restrict__ g, const 
     g[gi] /= ev;
 }
 
+// ---- level-1 exact solve of 2D grids in four launches ----
+//
+// Gather and forward x (MODE 0), forward y and the division (1), inverse y (2),
+// inverse x and scatter (3), each as k_axis_gemm_full forms an axis (a 16 x 16
+// output tile per work group, the whole k range of its operands in LDS, each
+// output one sum over k in increasing order), each over the grids of every
+// coarse group at once. These launches are bound by latency (two load round
+// trips and a chain of n sums), so what they cost is their number: 50 us per
+// solve of 128 x 256 as seven launches, 31 us as four; a forest with five
+// shapes of level 1 needed 35 launches.
+struct L12Group {
+    int N0, N1, ntree, nper;           // nper: blocks per tree
+    size_t goff;                       // the group's grids in the scratch grids
+    const double *Q[2], *P[2], *lam[2], *shift, *cs;
+    const int *btab;
+};
+constexpr int L12_MAX = 8;  // groups per launch
+struct L12Args {
+    L12Group g[L12_MAX];
+};
+
+__host__ __device__ inline int l12_tiles(const L12Group &g, bool axis0) {
+    const int n = axis0 ? g.N0 : g.N1, ncol = g.ntree * (axis0 ? g.N1 : g.N0);
+    return ((n + AXF - 1) / AXF) * ((ncol + AXF - 1) / AXF);
+}
+
+template <int MODE, int M, typename T>
+__global__ __launch_bounds__(256) void k_l1_2d(L12Args a, double *__restrict__ out, const double *__restrict__ in,
+                                               const T *__restrict__ src, T *__restrict__ dst) {
+    using LY = Lay<2, M>;
+    constexpr bool AX0 = MODE == 0 || MODE == 3;
+    __shared__ double As[AXF * 257];        // As[r][k], row stride n + 1
+    __shared__ double Xs[256 * (AXF + 1)];  // Xs[k][c]
+    int wg = blockIdx.x, gi = 0;
+    while (wg >= l12_tiles(a.g[gi], AX0)) wg -= l12_tiles(a.g[gi++], AX0);
+    const L12Group &g = a.g[gi];
+    const int tid = threadIdx.x, N0 = g.N0, N1 = g.N1, nb0 = N0 / M;
+    const int n = AX0 ? N0 : N1, nother = AX0 ? N1 : N0, ncol = g.ntree * nother;
+    const int ti = (n + AXF - 1) / AXF, i0 = wg % ti * AXF, c0 = wg / ti * AXF, sa = n + 1;
+    const double *__restrict__ A = MODE == 0 ? g.Q[0] : MODE == 1 ? g.Q[1] : MODE == 2 ? g.P[1] : g.P[0];
+    const double *__restrict__ gin = in + g.goff;
+    // 16 rows (or columns) of the tile by 16 consecutive k, 16 times: no
+    // division per element, 128 contiguous bytes per 16 lanes
+    const int hi = tid >> 4, lo = tid & 15;
+    // this thread's column of X: along x its k runs over lo + 16 q, along y over hi + 16 q
+    const int xc = c0 + (AX0 ? hi : lo), xt = min(xc / nother, g.ntree - 1), xj = xc - xt * nother;
+    const bool xok = xc < ncol;
+    double va[16], vx[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const int k = lo + 16 * q;
+        va[q] = (k < n && i0 + hi < n) ? A[(size_t)(i0 + hi) * n + k] : 0.0;
+    }
+    if constexpr (MODE == 0) {
+        const int *tb = g.btab + (size_t)xt * g.nper + (xj / M) * nb0;
+        int blk[16];
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int k = lo + 16 * q;
+            blk[q] = (xok && k < n) ? tb[k / M] : 0;
+        }
+        const double cs = g.cs[xt];
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int k = lo + 16 * q;
+            vx[q] = (xok && k < n) ? cs * (double)src[(size_t)blk[q] * LY::V + LY::sidx(k % M, xj % M, 0)] : 0.0;
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int k = (AX0 ? lo : hi) + 16 * q;
+            vx[q] = 0.0;
+            if (xok && k < n) vx[q] = AX0 ? gin[(size_t)xc * N0 + k] : gin[((size_t)xt * N1 + k) * N0 + xj];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const int k = lo + 16 * q;
+        if (k < n) As[hi * sa + k] = va[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const int k = (AX0 ? lo : hi) + 16 * q;
+        if (k < n) Xs[k * (AXF + 1) + (AX0 ? hi : lo)] = vx[q];
+    }
+    // the output's place, and what it takes besides the sum
+    const int r = AX0 ? tid % AXF : tid / AXF, c = AX0 ? tid / AXF : tid % AXF;
+    const int i = i0 + r, col = c0 + c, t = col / nother, j = col - t * nother;
+    const bool ok = i < n && col < ncol;
+    double ev = 1.0;
+    int blk = 0;
+    if (MODE == 1 && ok) {
+        ev = g.shift[t];
+        ev += g.lam[0][j];
+        ev += g.lam[1][i];
+    }
+    if (MODE == 3 && ok) blk = g.btab[(size_t)t * g.nper + (j / M) * nb0 + i / M];
+    __syncthreads();
+    double acc = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < n; k++) acc += As[r * sa + k] * Xs[k * (AXF + 1) + c];
+    if (!ok) return;
+    if (MODE == 0) out[g.goff + (size_t)col * N0 + i] = acc;
+    if (MODE == 1) out[g.goff + ((size_t)t * N1 + i) * N0 + j] = acc / ev;
+    if (MODE == 2) out[g.goff + ((size_t)t * N1 + i) * N0 + j] = acc;
+    if (MODE == 3) dst[(size_t)blk * LY::V + LY::sidx(i % M, j % M, 0)] = (T)acc;
+}
+
 // ---- level-1 exact solve of 3D grids in three launches ----
 //
 // For stacked 3D grids [g][z][y][x] (x fastest) whose extents are multiples of

@@ -79,6 +79,7 @@ struct CoarseGroup {
     int N[3] = {1, 1, 1};
     int ntree = 0;
     int l1_blk0 = 0, nper = 0;  // level-1 device blocks: contiguous, nper per tree
+    size_t goff = 0;            // its grids in d_grid and d_grid2
     bool valid = false;
     int geom = -1;
     int8_t bc[27] = {0};
@@ -666,7 +667,12 @@ static void upload_tables(srmg_ctx *c) {
     c->d_partial.alloc((size_t)c->maxpartials * sizeof(double));
     c->d_sum.alloc(sizeof(double) * (SUM_CHUNKS + 4 + nt));
     size_t ng = 0;
-    for (auto &G : c->groups) ng = std::max(ng, (size_t)G.ntree * G.N[0] * G.N[1] * (D == 3 ? G.N[2] : 1));
+    // the 2D solve takes all groups at once, the others one after the other
+    for (auto &G : c->groups) {
+        const size_t n = (size_t)G.ntree * G.N[0] * G.N[1] * (D == 3 ? G.N[2] : 1);
+        G.goff = D == 2 ? ng : 0;
+        ng = D == 2 ? ng + n : std::max(ng, n);
+    }
     c->d_grid.alloc(ng * sizeof(double));
     c->d_grid2.alloc(ng * sizeof(double));
     std::vector<std::vector<int>> btabs;
@@ -1565,6 +1571,44 @@ struct Ops {
         sum_partials(np, c->d_rng_blk);
     }
 
+    // coarse_exact of 2D trees whose level-1 extents are at most 256, every
+    // coarse group in the same four launches; false where that does not apply
+    bool coarse_exact_2d(FieldBuf &u, FieldBuf &b) {
+        if (c->axis_gemm != 2) return false;
+        for (const CoarseGroup &G : c->groups)
+            if (G.N[0] > 256 || G.N[1] > 256) return false;
+        double *g = c->d_grid.as<double>(), *g2 = c->d_grid2.as<double>();
+        for (size_t k = 0; k < c->groups.size(); k += L12_MAX) {
+            L12Args a{};
+            unsigned w0 = 0, w1 = 0;  // work groups along x and along y
+            for (size_t i = k; i < std::min(c->groups.size(), k + L12_MAX); i++) {
+                const CoarseGroup &G = c->groups[i];
+                L12Group &q = a.g[i - k];
+                q.N0 = G.N[0];
+                q.N1 = G.N[1];
+                q.ntree = G.ntree;
+                q.nper = G.nper;
+                q.goff = G.goff;
+                for (int d = 0; d < 2; d++) {
+                    q.Q[d] = G.Q[d].template as<double>();
+                    q.P[d] = G.P[d].template as<double>();
+                    q.lam[d] = G.lam[d].template as<double>();
+                }
+                q.shift = G.shift.template as<double>();
+                q.cs = G.cs.template as<double>();
+                q.btab = G.btab.template as<int>();
+                w0 += (unsigned)l12_tiles(q, true);
+                w1 += (unsigned)l12_tiles(q, false);
+            }
+            const T *none = nullptr;
+            T *no = nullptr;
+            hipLaunchKernelGGL((k_l1_2d<0, M, T>), dim3(w0), dim3(256), 0, c->stream, a, g, g2, X(b, 0), no);
+            hipLaunchKernelGGL((k_l1_2d<1, M, T>), dim3(w1), dim3(256), 0, c->stream, a, g2, g, none, no);
+            hipLaunchKernelGGL((k_l1_2d<2, M, T>), dim3(w1), dim3(256), 0, c->stream, a, g, g2, none, no);
+            hipLaunchKernelGGL((k_l1_2d<3, M, T>), dim3(w0), dim3(256), 0, c->stream, a, g2, g, none, X(u, 0));
+        }
+        return true;
+    }
     // exact FP64 solve of L_1 u + s b = 0 on the complete level 1
     void coarse_exact(FieldBuf &u, FieldBuf &b, double s, const srmg_op *op);
     // out = A in along an axis of extent n and stride `inner` (ncol columns)
@@ -1885,6 +1929,11 @@ void Ops<D, M, T>::coarse_exact(FieldBuf &u, FieldBuf &b, double s, const srmg_o
             G.geom = op->geometry;
             std::memcpy(G.bc, op->bc, 27);
         }
+    }
+    if constexpr (D == 2)
+        if (coarse_exact_2d(u, b)) return;
+    for (CoarseGroup &G : c->groups) {
+        const int *N = G.N;
         const size_t total = (size_t)N[0] * N[1] * (D == 3 ? N[2] : 1);
         const int nblk = G.ntree * G.nper;
         double *g = c->d_grid.as<double>(), *g2 = c->d_grid2.as<double>();
