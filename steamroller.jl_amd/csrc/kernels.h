@@ -28,9 +28,9 @@ struct LevelArgs {
     const T *wm;   // (2J-2)/(2J-1) by 1-based global radial index J at this level
     const T *wp;   // 2J/(2J-1)
     // several problems in one launch: (s, cc, nwc) of block blk are
-    // pp[3 pix[blk] + 0..2]; nullptr when the context holds one problem
+    // pp[3 blk + 0..2] (one load; through a per-block problem index it was two
+    // in a row); nullptr when the context holds one problem
     const T *pp;
-    const int *pix;
     // processing order of the level's sibling groups in the column sweeps:
     // work group slot i takes group gord[i]; nullptr: group i
     const int *gord;
@@ -44,7 +44,7 @@ struct BP {
 template <typename T>
 __device__ __forceinline__ BP<T> bparams(const LevelArgs<T> &a, int blk) {
     if (a.pp) {
-        const T *q = a.pp + 3 * a.pix[blk];
+        const T *q = a.pp + 3 * (size_t)blk;
         return {q[0], q[1], q[2]};
     }
     return {a.s, a.cc, a.nwc};
@@ -128,6 +128,15 @@ __device__ __forceinline__ void radial_weights(const LevelArgs<T> &a, const int 
         wm = a.wm[J];
         wp = a.wp[J];
     }
+}
+
+// per-block parameters from the per-(tree, level) ones, blocks' problem
+// indices in pix
+template <typename T>
+__global__ __launch_bounds__(WG) void k_block_params(T *__restrict__ out, const T *__restrict__ pp,
+                                                     const int *__restrict__ pix, int nb) {
+    const int i = blockIdx.x * WG + threadIdx.x;
+    if (i < 3 * nb) out[i] = pp[3 * pix[i / 3] + i % 3];
 }
 
 // One colour of gauss_seidel! (src/multigrid.jl:153-180) on every block of a
@@ -1108,13 +1117,21 @@ __device__ __forceinline__ T tstencil(const T *t, int p, T own, T cc, T wm, T wp
     return v;
 }
 
-template <int D, int M, typename T, int RD>
-__device__ __forceinline__ void rweights(const LevelArgs<T> &a, const int *__restrict__ coord, int blk, int cr,
-                                         T &wm, T &wp) {
+// Radial weights in two load round trips, which the kernels below issue with
+// the trips they make anyway (the block's coordinate with the interior, the
+// weights with the halo) instead of waiting for both before the arithmetic:
+// the radial index J of a block's cell 0, then the weights of a cell at J + cr.
+// With them and the per-block parameters read directly, the launches of a 2D
+// cylindrical forest of 27 trees lose about one microsecond in six.
+template <int D, int M, int RD>
+__device__ __forceinline__ int rbase(const int *__restrict__ coord, int blk) {
+    return RD >= 0 ? M * (coord[blk * D + RD] - 1) + 1 : 0;
+}
+template <typename T, int RD>
+__device__ __forceinline__ void rweights(const LevelArgs<T> &a, int J, T &wm, T &wp) {
     wm = T(1);
     wp = T(1);
     if (RD >= 0) {
-        int J = M * (coord[blk * D + RD] - 1) + cr + 1;
         wm = a.wm[J];
         wp = a.wp[J];
     }
@@ -1253,18 +1270,22 @@ struct RecFace {
     }
 
     // first-half-sweep value of the neighbour cell, written into this block's halo
+    // (wm, wp: the radial weights at that cell, radial_index of this block's J)
     template <int RD>
-    __device__ static __forceinline__ void compute(int dir, int tq, int e, const int *gs, T *tile,
-                                                   const int *__restrict__ coord, const LevelArgs<T> &a,
-                                                   const BP<T> &bp, T rd, T rb, const T *rg) {
+    __device__ static __forceinline__ int radial_index(int dir, int tq, int J) {
+        int cB[3];
+        cell(dir, tq, cB);
+        return RD < 0 ? 0 : J + (DIM == RD ? dir * M : 0) + cB[RD < 0 ? 0 : RD];
+    }
+    template <int RD>
+    __device__ static __forceinline__ void compute(int dir, int tq, const int *gs, T *tile, T wm, T wp,
+                                                   const LevelArgs<T> &a, const BP<T> &bp, T rd, T rb, const T *rg) {
         int cB[3];
         cell(dir, tq, cB);
         int ch[3] = {cB[0], cB[1], cB[2]};
         ch[DIM] = dir > 0 ? M : -1;
         const int ph = TL::at(ch[0], ch[1], ch[2]);
         const T xo = tile[ph];
-        T wm, wp;
-        rweights<D, M, T, RD>(a, coord, e, RD >= 0 ? cB[RD < 0 ? 0 : RD] : 0, wm, wp);
         T nbm[3], nbp[3];
         // across the shared face: this block's cell; one layer deeper: rd
         const int pa = TL::at(DIM == 0 ? (dir > 0 ? M - 1 : 0) : cB[0], DIM == 1 ? (dir > 0 ? M - 1 : 0) : cB[1],
@@ -1348,8 +1369,27 @@ __global__ __launch_bounds__(NT) void k_gs_sweep(T *__restrict__ uo, const T *__
             be[k] = b[o + H];
         }
     }
-    for (int i = tid; i < nloc * HT::N; i += NT) tab[i] = htab[(size_t)blk0 * HT::N + i];
-    if (tid < nloc) prm[tid] = bparams(a, blk0 + tid);
+    constexpr int TP = (BPW * HT::N + NT - 1) / NT;
+    int tv[TP];
+#pragma unroll
+    for (int k = 0; k < TP; k++) {
+        const int i = tid + k * NT;
+        tv[k] = i < nloc * HT::N ? htab[(size_t)blk0 * HT::N + i] : 0;
+    }
+    BP<T> bpl{};
+    if (tid < nloc) bpl = bparams(a, blk0 + tid);
+    // radial index of the thread's cells' blocks and of its recompute items' blocks
+    int Jc[CPT], Jr[RPT];
+#pragma unroll
+    for (int k = 0; k < CPT; k++) Jc[k] = rbase<D, M, RD>(coord, blk0 + min((tid + k * NT) / H, nloc - 1));
+#pragma unroll
+    for (int k = 0; k < RPT; k++) Jr[k] = rbase<D, M, RD>(coord, blk0 + min((tid + k * NT) / (ND * F2), nloc - 1));
+#pragma unroll
+    for (int k = 0; k < TP; k++) {
+        const int i = tid + k * NT;
+        if (i < nloc * HT::N) tab[i] = tv[k];
+    }
+    if (tid < nloc) prm[tid] = bpl;
 #pragma unroll
     for (int k = 0; k < CPT; k++) {
         int i = tid + k * NT, lb = i / H, r = i - lb * H;
@@ -1374,14 +1414,24 @@ __global__ __launch_bounds__(NT) void k_gs_sweep(T *__restrict__ uo, const T *__
         hv[j] = T(0);
         if (i < NHALO && lb < nloc) hv[j] = halo_value_sw<D, M, T>(f, tab[lb * HT::N + f], blk0 + lb, t, ui, ib, a.sg);
     }
+    // the radial weights of the thread's cells
+    T wc[CPT][2][2];
+#pragma unroll
+    for (int k = 0; k < CPT; k++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            int x, y, z;
+            LY::decode(h * H + (tid + k * NT) % H, x, y, z);
+            rweights<T, RD>(a, Jc[k] + (RD == 0 ? x : y), wc[k][h][0], wc[k][h][1]);
+        }
     // ... and the operands of the recomputed neighbour cells
-    T rd[RPT], rb[RPT], rg[RPT][NS];
+    T rd[RPT], rb[RPT], rg[RPT][NS], rw[RPT][2];
     int rj[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
         int j = tid + k * NT;
         rj[k] = -1;
-        rd[k] = rb[k] = T(0);
+        rd[k] = rb[k] = rw[k][0] = rw[k][1] = T(0);
         if (j >= NREC) continue;
         int lb = j / (ND * F2), rem = j - lb * (ND * F2);
         int f = rem / F2, tq = rem - f * F2;
@@ -1391,6 +1441,9 @@ __global__ __launch_bounds__(NT) void k_gs_sweep(T *__restrict__ uo, const T *__
         if (e < 0) continue;
         rj[k] = j;
         int dim = f >> 1, dir = (f & 1) ? 1 : -1;
+        const int J = dim == 0 ? RecFace<D, M, T, 0>::template radial_index<RD>(dir, tq, Jr[k])
+                               : RecFace<D, M, T, 1>::template radial_index<RD>(dir, tq, Jr[k]);
+        rweights<T, RD>(a, J, rw[k][0], rw[k][1]);
         if (dim == 0) RecFace<D, M, T, 0>::prefetch(dir, tq, e, gs, ui, b, ib, rd[k], rb[k], rg[k]);
         else if (dim == 1) RecFace<D, M, T, 1>::prefetch(dir, tq, e, gs, ui, b, ib, rd[k], rb[k], rg[k]);
         else RecFace<D, M, T, (D == 3 ? 2 : 1)>::prefetch(dir, tq, e, gs, ui, b, ib, rd[k], rb[k], rg[k]);
@@ -1411,10 +1464,8 @@ __global__ __launch_bounds__(NT) void k_gs_sweep(T *__restrict__ uo, const T *__
             int x, y, z;
             LY::decode(r, x, y, z);
             int p = lb * TL::SZ + TL::at(x, y, z);
-            T wm, wp;
-            rweights<D, M, T, RD>(a, coord, blk0 + lb, RD == 0 ? x : y, wm, wp);
             const BP<T> bp = prm[lb];
-            T Lu = tstencil<D, M, T, RD>(tile, p, ux[k][0], bp.cc, wm, wp);
+            T Lu = tstencil<D, M, T, RD>(tile, p, ux[k][0], bp.cc, wc[k][0][0], wc[k][0][1]);
             ux[k][0] = fma_t<T>(bp.nwc, fma_t<T>(bp.s, bo[k], Lu), ux[k][0]);
             tile[p] = ux[k][0];
         }
@@ -1428,15 +1479,15 @@ __global__ __launch_bounds__(NT) void k_gs_sweep(T *__restrict__ uo, const T *__
         int f = rem / F2, tq = rem - f * F2;
         const int *tb = tab + lb * HT::N, *gs = tb + HT::ND + f * HT::NS;
         T *tl = tile + lb * TL::SZ;
-        int e = tb[f];
         int dim = f >> 1, dir = (f & 1) ? 1 : -1;
         const BP<T> bp = prm[lb];
+        const T wm = rw[k][0], wp = rw[k][1];
         if (dim == 0)
-            RecFace<D, M, T, 0>::template compute<RD>(dir, tq, e, gs, tl, coord, a, bp, rd[k], rb[k], rg[k]);
+            RecFace<D, M, T, 0>::template compute<RD>(dir, tq, gs, tl, wm, wp, a, bp, rd[k], rb[k], rg[k]);
         else if (dim == 1)
-            RecFace<D, M, T, 1>::template compute<RD>(dir, tq, e, gs, tl, coord, a, bp, rd[k], rb[k], rg[k]);
+            RecFace<D, M, T, 1>::template compute<RD>(dir, tq, gs, tl, wm, wp, a, bp, rd[k], rb[k], rg[k]);
         else
-            RecFace<D, M, T, (D == 3 ? 2 : 1)>::template compute<RD>(dir, tq, e, gs, tl, coord, a, bp, rd[k], rb[k],
+            RecFace<D, M, T, (D == 3 ? 2 : 1)>::template compute<RD>(dir, tq, gs, tl, wm, wp, a, bp, rd[k], rb[k],
                                                                      rg[k]);
     }
     __syncthreads();
@@ -1449,10 +1500,8 @@ __global__ __launch_bounds__(NT) void k_gs_sweep(T *__restrict__ uo, const T *__
             int x, y, z;
             LY::decode(H + r, x, y, z);
             int p = lb * TL::SZ + TL::at(x, y, z);
-            T wm, wp;
-            rweights<D, M, T, RD>(a, coord, blk0 + lb, RD == 0 ? x : y, wm, wp);
             const BP<T> bp = prm[lb];
-            T Lu = tstencil<D, M, T, RD>(tile, p, ux[k][1], bp.cc, wm, wp);
+            T Lu = tstencil<D, M, T, RD>(tile, p, ux[k][1], bp.cc, wc[k][1][0], wc[k][1][1]);
             size_t o = (size_t)(blk0 + lb) * V + r;
             uo[o] = ux[k][0];
             uo[o + H] = fma_t<T>(bp.nwc, fma_t<T>(bp.s, be[k], Lu), ux[k][1]);
@@ -1497,8 +1546,17 @@ __global__ __launch_bounds__(NT) void k_gs_sweep_group(T *__restrict__ uo, const
         bo[k] = b[o];
         be[k] = b[o + H];
     }
-    for (int i = tid; i < NB * HT::N; i += NT) tab[i] = htab[(size_t)blk0 * HT::N + i];
-    if (tid < NB) prm[tid] = bparams(a, blk0 + tid);
+    static_assert(NB * HT::N <= NT, "one table entry per thread");
+    const int tv = tid < NB * HT::N ? htab[(size_t)blk0 * HT::N + tid] : 0;
+    BP<T> bpl{};
+    if (tid < NB) bpl = bparams(a, blk0 + tid);
+    int Jc[CPT], Jr[RPT];
+#pragma unroll
+    for (int k = 0; k < CPT; k++) Jc[k] = rbase<D, M, RD>(coord, blk0 + (tid + k * NT) / H);
+#pragma unroll
+    for (int k = 0; k < RPT; k++) Jr[k] = rbase<D, M, RD>(coord, blk0 + min((tid + k * NT) / (D * F2), NB - 1));
+    if (tid < NB * HT::N) tab[tid] = tv;
+    if (tid < NB) prm[tid] = bpl;
 #pragma unroll
     for (int k = 0; k < CPT; k++) {
         const int i = tid + k * NT, lb = i / H, r = i - lb * H;
@@ -1522,13 +1580,22 @@ __global__ __launch_bounds__(NT) void k_gs_sweep_group(T *__restrict__ uo, const
         hv[j] = T(0);
         if (i < NHALO) hv[j] = halo_value_sw<D, M, T>(f, tab[lb * HT::N + f], blk0 + lb, t, ui, ib, a.sg);
     }
-    T rd[RPT], rb[RPT], rg[RPT][NS];
+    T wc[CPT][2][2];
+#pragma unroll
+    for (int k = 0; k < CPT; k++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            int x, y, z;
+            LY::decode(h * H + (tid + k * NT) % H, x, y, z);
+            rweights<T, RD>(a, Jc[k] + (RD == 0 ? x : y), wc[k][h][0], wc[k][h][1]);
+        }
+    T rd[RPT], rb[RPT], rg[RPT][NS], rw[RPT][2];
     int rj[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
         const int j = tid + k * NT;
         rj[k] = -1;
-        rd[k] = rb[k] = T(0);
+        rd[k] = rb[k] = rw[k][0] = rw[k][1] = T(0);
         if (j >= NREC) continue;
         const int lb = j / (D * F2), rem = j - lb * (D * F2);
         const int d = rem / F2, tq = rem - d * F2;
@@ -1538,6 +1605,9 @@ __global__ __launch_bounds__(NT) void k_gs_sweep_group(T *__restrict__ uo, const
         if (e < 0) continue;
         rj[k] = j;
         const int dir = (f & 1) ? 1 : -1;
+        const int J = d == 0 ? RecFace<D, M, T, 0, TL>::template radial_index<RD>(dir, tq, Jr[k])
+                             : RecFace<D, M, T, 1, TL>::template radial_index<RD>(dir, tq, Jr[k]);
+        rweights<T, RD>(a, J, rw[k][0], rw[k][1]);
         if (d == 0) RecFace<D, M, T, 0, TL>::prefetch(dir, tq, e, gs, ui, b, ib, rd[k], rb[k], rg[k]);
         else if (d == 1) RecFace<D, M, T, 1, TL>::prefetch(dir, tq, e, gs, ui, b, ib, rd[k], rb[k], rg[k]);
         else RecFace<D, M, T, (D == 3 ? 2 : 1), TL>::prefetch(dir, tq, e, gs, ui, b, ib, rd[k], rb[k], rg[k]);
@@ -1558,10 +1628,8 @@ __global__ __launch_bounds__(NT) void k_gs_sweep_group(T *__restrict__ uo, const
         int x, y, z;
         LY::decode(r, x, y, z);
         const int p = TL::origin(lb) + TL::at(x, y, z);
-        T wm, wp;
-        rweights<D, M, T, RD>(a, coord, blk0 + lb, RD == 0 ? x : y, wm, wp);
         const BP<T> bp = prm[lb];
-        T Lu = tstencil<D, M, T, RD, TL>(tile, p, ux[k][0], bp.cc, wm, wp);
+        T Lu = tstencil<D, M, T, RD, TL>(tile, p, ux[k][0], bp.cc, wc[k][0][0], wc[k][0][1]);
         ux[k][0] = fma_t<T>(bp.nwc, fma_t<T>(bp.s, bo[k], Lu), ux[k][0]);
         tile[p] = ux[k][0];
     }
@@ -1574,16 +1642,16 @@ __global__ __launch_bounds__(NT) void k_gs_sweep_group(T *__restrict__ uo, const
         const int f = 2 * d + ((lb >> d) & 1);
         const int *tb = tab + lb * HT::N, *gs = tb + HT::ND + f * HT::NS;
         T *tl = tile + TL::origin(lb);
-        const int e = tb[f];
         const int dir = (f & 1) ? 1 : -1;
         const BP<T> bp = prm[lb];
+        const T wm = rw[k][0], wp = rw[k][1];
         if (d == 0)
-            RecFace<D, M, T, 0, TL>::template compute<RD>(dir, tq, e, gs, tl, coord, a, bp, rd[k], rb[k], rg[k]);
+            RecFace<D, M, T, 0, TL>::template compute<RD>(dir, tq, gs, tl, wm, wp, a, bp, rd[k], rb[k], rg[k]);
         else if (d == 1)
-            RecFace<D, M, T, 1, TL>::template compute<RD>(dir, tq, e, gs, tl, coord, a, bp, rd[k], rb[k], rg[k]);
+            RecFace<D, M, T, 1, TL>::template compute<RD>(dir, tq, gs, tl, wm, wp, a, bp, rd[k], rb[k], rg[k]);
         else
-            RecFace<D, M, T, (D == 3 ? 2 : 1), TL>::template compute<RD>(dir, tq, e, gs, tl, coord, a, bp, rd[k],
-                                                                         rb[k], rg[k]);
+            RecFace<D, M, T, (D == 3 ? 2 : 1), TL>::template compute<RD>(dir, tq, gs, tl, wm, wp, a, bp, rd[k], rb[k],
+                                                                         rg[k]);
     }
     __syncthreads();
 
@@ -1594,10 +1662,8 @@ __global__ __launch_bounds__(NT) void k_gs_sweep_group(T *__restrict__ uo, const
         int x, y, z;
         LY::decode(H + r, x, y, z);
         const int p = TL::origin(lb) + TL::at(x, y, z);
-        T wm, wp;
-        rweights<D, M, T, RD>(a, coord, blk0 + lb, RD == 0 ? x : y, wm, wp);
         const BP<T> bp = prm[lb];
-        T Lu = tstencil<D, M, T, RD, TL>(tile, p, ux[k][1], bp.cc, wm, wp);
+        T Lu = tstencil<D, M, T, RD, TL>(tile, p, ux[k][1], bp.cc, wc[k][1][0], wc[k][1][1]);
         const size_t o = (size_t)(blk0 + lb) * V + r;
         uo[o] = ux[k][0];
         uo[o + H] = fma_t<T>(bp.nwc, fma_t<T>(bp.s, be[k], Lu), ux[k][1]);
@@ -1733,9 +1799,9 @@ struct ColSweep {
             constexpr int DA = DIM == 0 ? 1 : 0, DB = DIM == 2 ? 1 : 2;
             const int k = (rside << DIM) | ((rbf & 1) << DA) | ((rbf >> 1) << DB), f = 2 * DIM + rside;
             if (re[DIM] >= 0)
-                RecFace<D, M, T, DIM, TL>::template compute<RD>(rside ? 1 : -1, rtq, re[DIM],
+                RecFace<D, M, T, DIM, TL>::template compute<RD>(rside ? 1 : -1, rtq,
                                                                 sm.tab + k * HT::N + HT::ND + f * HT::NS,
-                                                                t + TL::origin(k), coord, a, sm.prm[k], rd[DIM],
+                                                                t + TL::origin(k), T(1), T(1), a, sm.prm[k], rd[DIM],
                                                                 rb[DIM], rg[DIM]);
         });
         lds_barrier();
@@ -1808,9 +1874,10 @@ struct ColSweepZ {
         const int rside = q >> 7, rbf = (q >> 5) & 3, rtq = q & 31;
         const int k = (rside << DIM) | ((rbf & 1) << DA) | ((rbf >> 1) << DB), f = 2 * DIM + rside;
         if (re >= 0)
-            RecFace<D, M, T, DIM, TL>::template compute<RD>(rside ? 1 : -1, rtq, re,
+            RecFace<D, M, T, DIM, TL>::template compute<RD>(rside ? 1 : -1, rtq,
                                                             sm.tab + k * HT::N + HT::ND + f * HT::NS,
-                                                            sm.tile + TL::origin(k), coord, a, sm.prm[k], rd, rb, rg);
+                                                            sm.tile + TL::origin(k), T(1), T(1), a, sm.prm[k], rd, rb,
+                                                            rg);
     }
 
     // VAR bit 0: the column goes out with nontemporal stores; bit 1: the
@@ -1950,34 +2017,45 @@ __global__ __launch_bounds__(512) void k_gs_sweep_colz(T *__restrict__ uo, const
 
 // ---- tiled residual kernels ----
 
+struct NoLoads {
+    __device__ __forceinline__ void operator()() const {}
+};
+
 // Stage BPW blocks (valid cells + depth-1 face halo) of x in the LDS tile.
 // list != nullptr selects the blocks through an index list (leaf blocks).
 // Two barriers: after (interior, halo table) and after the halo cells
 // (LDSB: barriers that order LDS only, for callers with loads in flight).
-template <int D, int M, typename T, int BPW, int NT, bool LDSB = false>
+// with1 and with2 issue the caller's own loads with the first and the second
+// round trip; with2 may also store to LDS what is read after the call.
+template <int D, int M, typename T, int BPW, int NT, bool LDSB = false, class W1 = NoLoads, class W2 = NoLoads>
 __device__ __forceinline__ void load_tile(T *tile, int *tab, int *blks, const T *__restrict__ x,
                                           const T *__restrict__ ib, const int *__restrict__ htab,
-                                          const int *__restrict__ list, int first, int nloc, const T *sg) {
+                                          const int *__restrict__ list, int first, int nloc, const T *sg,
+                                          W1 &&with1 = W1(), W2 &&with2 = W2()) {
     using LY = Lay<D, M>;
     using TL = Tile<D, M>;
     using HT = Halo<D>;
     constexpr int F = LY::F, V = LY::V, ND = 2 * D;
+    static_assert(BPW * ND <= NT, "one table entry per thread");
     // each phase issues all of its loads before the first tile store (a loop
     // that stores between its loads waits out each load in turn)
     constexpr int PI = (BPW * V + NT - 1) / NT, PH = (BPW * ND * F + NT - 1) / NT;
     const int tid = threadIdx.x;
-    if (tid < BPW) blks[tid] = (tid < nloc) ? (list ? list[first + tid] : first + tid) : 0;
-    if (LDSB) lds_barrier(); else __syncthreads();
+    auto blk_at = [&](int lb) { return list ? list[first + min(lb, nloc - 1)] : first + min(lb, nloc - 1); };
+    int bl[PI];
+#pragma unroll
+    for (int j = 0; j < PI; j++) bl[j] = blk_at((tid + NT * j) / V);
+    const int bt = blk_at(tid / ND), bs = blk_at(min(tid, BPW - 1));
     T xv[PI];
 #pragma unroll
     for (int j = 0; j < PI; j++) {
         const int i = tid + NT * j, lb = min(i / V, BPW - 1);
-        xv[j] = (i < nloc * V) ? x[(size_t)blks[lb] * V + (i - lb * V)] : T(0);
+        xv[j] = (i < nloc * V) ? x[(size_t)bl[j] * V + (i - lb * V)] : T(0);
     }
-    for (int i = tid; i < nloc * ND; i += NT) {
-        int lb = i / ND;
-        tab[i] = htab[(size_t)blks[lb] * HT::N + (i - lb * ND)];
-    }
+    const int tv = tid < nloc * ND ? htab[(size_t)bt * HT::N + tid % ND] : 0;
+    with1();
+    if (tid < BPW) blks[tid] = tid < nloc ? bs : 0;
+    if (tid < nloc * ND) tab[tid] = tv;
 #pragma unroll
     for (int j = 0; j < PI; j++) {
         const int i = tid + NT * j, lb = min(i / V, BPW - 1);
@@ -1996,6 +2074,7 @@ __device__ __forceinline__ void load_tile(T *tile, int *tab, int *blks, const T 
         hv[j] = T(0);
         if (i < nloc * ND * F) hv[j] = halo_value_sw<D, M, T>(f, tab[lb * ND + f], blks[lb], t, x, ib, sg);
     }
+    with2();
 #pragma unroll
     for (int j = 0; j < PH; j++) {
         const int i = tid + NT * j, lb = min(i / (ND * F), BPW - 1), rem = i - lb * (ND * F);
@@ -2098,17 +2177,35 @@ __global__ __launch_bounds__(NT) void k_resid_tile(TO *__restrict__ out, const T
     const int nloc = min(BPW, n - first);
     const int *lst = (MODE == RES_NORM) ? list : nullptr;
     const int base = (MODE == RES_NORM) ? first : a.blk0 + first;
-    load_tile<D, M, T, BPW, NT>(tile, tab, blks, u, ib, htab, lst, base, nloc, a.sg);
-    if ((int)threadIdx.x < nloc) prm[threadIdx.x] = bparams(a, blks[threadIdx.x]);
-    // the right-hand sides of the thread's cells, all in flight at once
+    // the right-hand sides of the thread's cells, their radial weights and the
+    // block parameters come with the tile's two round trips
     constexpr int PER = (BPW * V + NT - 1) / NT;
-    T bv[PER];
+    T bv[PER], wv[PER][2];
+    int Jc[PER];
+    bool leafs[PER];
+    BP<T> bpl{};
+    auto blk_at = [&](int lb) { return lst ? lst[base + min(lb, nloc - 1)] : base + min(lb, nloc - 1); };
+    load_tile<D, M, T, BPW, NT>(
+        tile, tab, blks, u, ib, htab, lst, base, nloc, a.sg,
+        [&] {
+            if ((int)threadIdx.x < nloc) bpl = bparams(a, blk_at(threadIdx.x));
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int i = threadIdx.x + NT * j, lb = min(i / V, BPW - 1);
-        bv[j] = (i < nloc * V) ? b[(size_t)blks[lb] * V + (i - lb * V)] : T(0);
-    }
-    __syncthreads();
+            for (int j = 0; j < PER; j++) {
+                const int i = threadIdx.x + NT * j, lb = min(i / V, BPW - 1), blk = blk_at(lb);
+                bv[j] = (i < nloc * V) ? b[(size_t)blk * V + (i - lb * V)] : T(0);
+                Jc[j] = rbase<D, M, RD>(coord, blk);
+                leafs[j] = MODE == RES_DEFECT && isleaf[blk];
+            }
+        },
+        [&] {
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                int x, y, z;
+                LY::decode((threadIdx.x + NT * j) % V, x, y, z);
+                rweights<T, RD>(a, Jc[j] + (RD == 0 ? x : y), wv[j][0], wv[j][1]);
+            }
+            if ((int)threadIdx.x < nloc) prm[threadIdx.x] = bpl;
+        });
     double acc[BPW];
 #pragma unroll
     for (int lb = 0; lb < BPW; lb++) acc[lb] = 0.0;
@@ -2121,15 +2218,13 @@ __global__ __launch_bounds__(NT) void k_resid_tile(TO *__restrict__ out, const T
         int x, y, z;
         LY::decode(q, x, y, z);
         int p = lb * TL::SZ + TL::at(x, y, z);
-        T wm, wp;
-        rweights<D, M, T, RD>(a, coord, blk, RD == 0 ? x : y, wm, wp);
         const BP<T> bp = prm[lb];
-        T Lu = tstencil<D, M, T, RD>(tile, p, tile[p], bp.cc, wm, wp);
+        T Lu = tstencil<D, M, T, RD>(tile, p, tile[p], bp.cc, wv[j][0], wv[j][1]);
         size_t o = (size_t)blk * V + q;
         T rr = -(bv[j] + Lu / bp.s);
         if (MODE == RES_WRITE) out[o] = (TO)rr;
         if (MODE == RES_DEFECT) out[o] = (TO)(bv[j] + Lu / bp.s);
-        if (MODE == RES_NORM || (MODE == RES_DEFECT && isleaf[blk])) {
+        if (MODE == RES_NORM || leafs[j]) {
 #pragma unroll
             for (int k = 0; k < BPW; k++)
                 if (k == lb) acc[k] += (double)rr * (double)rr;
@@ -2167,11 +2262,11 @@ __global__ __launch_bounds__(NT) void k_resid_tile(TO *__restrict__ out, const T
 // Tile<D, M, 2> with the halo of the group's exterior faces, its halo table
 // entries and block parameters; every load of a phase is issued before the
 // phase's first LDS store. Ends with a barrier (which also waits for loads
-// the caller issued before the call).
-template <int D, int M, typename T, int NT>
+// the caller issued before the call). with1 and with2: as in load_tile.
+template <int D, int M, typename T, int NT, class W1, class W2>
 __device__ __forceinline__ void stage_group(T *tile, int *tab, BP<T> *prm, const T *__restrict__ u,
                                             const T *__restrict__ ib, const int *__restrict__ htab,
-                                            const LevelArgs<T> &a, int g0) {
+                                            const LevelArgs<T> &a, int g0, W1 &&with1, W2 &&with2) {
     using LY = Lay<D, M>;
     using TL = Tile<D, M, 2>;
     using HT = Halo<D>;
@@ -2184,11 +2279,14 @@ __device__ __forceinline__ void stage_group(T *tile, int *tab, BP<T> *prm, const
         const int i = tid + NT * j;
         uv[j] = (i < NB * V) ? u[(size_t)g0 * V + i] : T(0);
     }
-    for (int i = tid; i < NB * 2 * D; i += NT) {
-        const int lb = i / (2 * D);
-        tab[i] = htab[(size_t)(g0 + lb) * HT::N + (i - lb * 2 * D)];
-    }
-    if (tid < NB) prm[tid] = bparams(a, g0 + tid);
+    static_assert(NB * 2 * D <= NT, "one table entry per thread");
+    int tv = 0;
+    if (tid < NB * 2 * D) tv = htab[(size_t)(g0 + tid / (2 * D)) * HT::N + tid % (2 * D)];
+    BP<T> bpl{};
+    if (tid < NB) bpl = bparams(a, g0 + tid);
+    with1();
+    if (tid < NB * 2 * D) tab[tid] = tv;
+    if (tid < NB) prm[tid] = bpl;
 #pragma unroll
     for (int j = 0; j < PU; j++) {
         const int i = tid + NT * j, lb = min(i / V, NB - 1), q = i - lb * V;
@@ -2208,6 +2306,7 @@ __device__ __forceinline__ void stage_group(T *tile, int *tab, BP<T> *prm, const
         hv[j] = T(0);
         if (i < NB * D * F) hv[j] = halo_value_sw<D, M, T>(f, tab[lb * 2 * D + f], g0 + lb, t, u, ib, a.sg);
     }
+    with2();
 #pragma unroll
     for (int j = 0; j < PH; j++) {
         const int i = tid + NT * j, lb = min(i / (D * F), NB - 1), rem = i - lb * (D * F);
@@ -2256,12 +2355,38 @@ __global__ __launch_bounds__(NT) void k_resid_group(TO *__restrict__ out, const 
             const int q = t + RT * h;
             bv[round][h] = q < V ? b[(size_t)(g0 + team + round * TEAMS) * V + q] : T(0);
         }
-    stage_group<D, M, T, NT>(tile, tab, prm, u, ib, htab, a, g0);
+    // their radial weights come with the staging's two round trips
+    int Jc[NR];
+    T wv[NR][QR][2];
+    auto coords = [&] {
+#pragma unroll
+        for (int round = 0; round < NR; round++) Jc[round] = rbase<D, M, RD>(coord, g0 + team + round * TEAMS);
+    };
+    auto weights = [&] {
+#pragma unroll
+        for (int round = 0; round < NR; round++)
+#pragma unroll
+            for (int h = 0; h < QR; h++) {
+                int x, y, z;
+                LY::decode((t + RT * h) % V, x, y, z);
+                rweights<T, RD>(a, Jc[round] + (RD == 0 ? x : y), wv[round][h][0], wv[round][h][1]);
+            }
+    };
+    bool leafs[NR];
+    stage_group<D, M, T, NT>(
+        tile, tab, prm, u, ib, htab, a, g0,
+        [&] {
+            coords();
+#pragma unroll
+            for (int round = 0; round < NR; round++)
+                leafs[round] = (MODE == RES_DEFECT) && isleaf[g0 + team + round * TEAMS];
+        },
+        weights);
 #pragma unroll
     for (int round = 0; round < NR; round++) {
         const int lb = team + round * TEAMS, blk = g0 + lb;
         const BP<T> bp = prm[lb];
-        const bool leaf = (MODE == RES_DEFECT) && isleaf[blk];
+        const bool leaf = leafs[round];
         double acc = 0.0;
 #pragma unroll
         for (int h = 0; h < QR; h++) {
@@ -2270,9 +2395,7 @@ __global__ __launch_bounds__(NT) void k_resid_group(TO *__restrict__ out, const 
             int x, y, z;
             LY::decode(q, x, y, z);
             const int p = TL::origin(lb) + TL::at(x, y, z);
-            T wm, wp;
-            rweights<D, M, T, RD>(a, coord, blk, RD == 0 ? x : y, wm, wp);
-            T Lu = tstencil<D, M, T, RD, TL>(tile, p, tile[p], bp.cc, wm, wp);
+            T Lu = tstencil<D, M, T, RD, TL>(tile, p, tile[p], bp.cc, wv[round][h][0], wv[round][h][1]);
             const size_t o = (size_t)blk * V + q;
             T rr = -(bv[round][h] + Lu / bp.s);
             if (MODE == RES_WRITE) out[o] = (TO)rr;
@@ -2353,10 +2476,34 @@ __global__ __launch_bounds__(NT) void k_resid_restrict(const T *__restrict__ u, 
             const int q = t + RT * h;
             bv[round][h] = q < V ? b[(size_t)(g0 + team + round * TEAMS) * V + q] : T(0);
         }
-    stage_group<D, M, T, NT>(tile, tab, prm, u, ib, htab, a, g0);
+    // their radial weights come with the staging's two round trips
+    int Jc[NR];
+    T wv[NR][QR][2];
+    auto coords = [&] {
+#pragma unroll
+        for (int round = 0; round < NR; round++) Jc[round] = rbase<D, M, RD>(coord, g0 + team + round * TEAMS);
+    };
+    auto weights = [&] {
+#pragma unroll
+        for (int round = 0; round < NR; round++)
+#pragma unroll
+            for (int h = 0; h < QR; h++) {
+                int x, y, z;
+                LY::decode((t + RT * h) % V, x, y, z);
+                rweights<T, RD>(a, Jc[round] + (RD == 0 ? x : y), wv[round][h][0], wv[round][h][1]);
+            }
+    };
+    int pb = 0;
+    stage_group<D, M, T, NT>(
+        tile, tab, prm, u, ib, htab, a, g0,
+        [&] {
+            coords();
+            pb = parent[g0];
+        },
+        weights);
 #pragma unroll
     for (int round = 0; round < NR; round++) {
-        const int lb = team + round * TEAMS, blk = g0 + lb;
+        const int lb = team + round * TEAMS;
         const BP<T> bp = prm[lb];
 #pragma unroll
         for (int h = 0; h < QR; h++) {
@@ -2365,15 +2512,12 @@ __global__ __launch_bounds__(NT) void k_resid_restrict(const T *__restrict__ u, 
             int x, y, z;
             LY::decode(q, x, y, z);
             const int p = TL::origin(lb) + TL::at(x, y, z);
-            T wm, wp;
-            rweights<D, M, T, RD>(a, coord, blk, RD == 0 ? x : y, wm, wp);
-            T Lu = tstencil<D, M, T, RD, TL>(tile, p, tile[p], bp.cc, wm, wp);
+            T Lu = tstencil<D, M, T, RD, TL>(tile, p, tile[p], bp.cc, wv[round][h][0], wv[round][h][1]);
             rt[lb * V + q] = -(bv[round][h] + Lu / bp.s);
         }
     }
     __syncthreads();
     // the parent's cells: coarse cell X of sub-block k = (X >= MH per dim)
-    const int pb = parent[g0];
     for (int i = tid; i < V; i += NT) {
         int X0, X1, X2;
         LY::decode(i, X0, X1, X2);
@@ -2731,8 +2875,23 @@ __global__ __launch_bounds__(256) void k_postrestrict_group(T *__restrict__ bout
         const int q = threadIdx.x + 256 * j;
         rv[j] = q < V ? r[(size_t)pb * V + q] : T(0);
     }
-    load_tile<D, M, T, 1, 256, true>(tile, tab, blks, u, ib, htab, nullptr, pb, 1, ac.sg);
-    const BP<T> bp = bparams(ac, pb);
+    int Jc = 0;
+    BP<T> bp{};
+    T wv[PER][2];
+    load_tile<D, M, T, 1, 256, true>(
+        tile, tab, blks, u, ib, htab, nullptr, pb, 1, ac.sg,
+        [&] {
+            Jc = rbase<D, M, RD>(coord, pb);
+            bp = bparams(ac, pb);
+        },
+        [&] {
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                int x, y, z;
+                LY::decode((threadIdx.x + 256 * j) % V, x, y, z);
+                rweights<T, RD>(ac, Jc + (RD == 0 ? x : y), wv[j][0], wv[j][1]);
+            }
+        });
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int q = threadIdx.x + 256 * j;
@@ -2740,9 +2899,7 @@ __global__ __launch_bounds__(256) void k_postrestrict_group(T *__restrict__ bout
         int x, y, z;
         LY::decode(q, x, y, z);
         const int p = TL::at(x, y, z);
-        T wm, wp;
-        rweights<D, M, T, RD>(ac, coord, pb, RD == 0 ? x : y, wm, wp);
-        T Lu = tstencil<D, M, T, RD>(tile, p, tile[p], bp.cc, wm, wp);
+        T Lu = tstencil<D, M, T, RD>(tile, p, tile[p], bp.cc, wv[j][0], wv[j][1]);
         bout[(size_t)pb * V + q] = -(rv[j] + Lu / bp.s);
     }
 }

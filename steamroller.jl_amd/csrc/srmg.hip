@@ -190,7 +190,8 @@ struct srmg_ctx {
     std::vector<srmg_op> pops;
     double pomega = 1.0;
     std::vector<double> pp_host;   // 3 x ntrees x nlevels: (s_l, cc, nwc)
-    DevBuf d_pp64, d_pp32;
+    DevBuf d_pp64, d_pp32;         // the same on the device
+    DevBuf d_bp64, d_bp32;         // several trees: one (s_l, cc, nwc) per block
     // captured solve steps, keyed by everything their launches bake in (solve
     // kind, fields, scales, operators, options, tile shapes, kernel switches);
     // cleared whenever a buffer they point to may move or change its role
@@ -700,6 +701,10 @@ static void upload_tables(srmg_ctx *c) {
     c->pp_host.clear();
     c->d_pp64.alloc((size_t)3 * nt * nlevels * sizeof(double));
     c->d_pp32.alloc((size_t)3 * nt * nlevels * sizeof(float));
+    if (nt > 1) {
+        c->d_bp64.alloc((size_t)3 * nb * sizeof(double));
+        c->d_bp32.alloc((size_t)3 * nb * sizeof(float));
+    }
     for (auto &f : c->fields)
         if (f) alloc_field(c, *f);
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -718,6 +723,8 @@ static void level_scalars(int D, int l, double s, const srmg_op *op, double omeg
     if (op->disc == SRMG_HELMHOLTZ) cc = cc - sl * op->k2;
     nwc = -(omega / cc);
 }
+
+static inline unsigned nwg(int64_t threads) { return (unsigned)((threads + WG - 1) / WG); }
 
 // Install the problems of the next calls: scale s[t] and operator ops[t] of
 // every tree (one value each when `same`). Geometry, boundary table and
@@ -754,6 +761,13 @@ static void prepare(srmg_ctx *c, const double *s, const srmg_op *ops, double ome
         for (size_t i = 0; i < pp.size(); i++) pf[i] = (float)pp[i];
         HIPCHK(hipMemcpy(c->d_pp64.p, pp.data(), pp.size() * sizeof(double), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(c->d_pp32.p, pf.data(), pf.size() * sizeof(float), hipMemcpyHostToDevice));
+        if (nt > 1) {
+            hipLaunchKernelGGL(k_block_params<double>, dim3(nwg((int64_t)3 * c->nb)), dim3(WG), 0, c->stream,
+                               c->d_bp64.as<double>(), c->d_pp64.as<double>(), c->d_pix.as<int>(), c->nb);
+            hipLaunchKernelGGL(k_block_params<float>, dim3(nwg((int64_t)3 * c->nb)), dim3(WG), 0, c->stream,
+                               c->d_bp32.as<float>(), c->d_pp32.as<float>(), c->d_pix.as<int>(), c->nb);
+            HIPCHK(hipGetLastError());
+        }
         for (auto &G : c->groups) {
             std::vector<double> cs(G.ntree), sh(G.ntree);
             for (int t = 0; t < nt; t++) {
@@ -804,17 +818,14 @@ static LevelArgs<T> level_args(srmg_ctx *c, int l /*0-based*/, double s, const s
     // several trees: per-block values from the tables installed by prepare()
     // (their -(omega/diagelm) is for c->pomega; residual kernels do not use it)
     if (c->trees.size() > 1) {
-        a.pp = std::is_same<T, double>::value ? (const T *)c->d_pp64.p : (const T *)c->d_pp32.p;
-        a.pix = c->d_pix.as<int>();
+        a.pp = std::is_same<T, double>::value ? (const T *)c->d_bp64.p : (const T *)c->d_bp32.p;
     } else {
         a.pp = nullptr;
-        a.pix = nullptr;
     }
     a.gord = (c->group_order && c->lv[l].gord0 >= 0) ? c->d_gord.as<int>() + c->lv[l].gord0 : nullptr;
     return a;
 }
 
-static inline unsigned nwg(int64_t threads) { return (unsigned)((threads + WG - 1) / WG); }
 
 // ---------------------------------------------------------------------------
 // kernel launchers, dispatched on (D, M, T)
