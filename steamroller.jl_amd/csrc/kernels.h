@@ -990,69 +990,38 @@ __global__ __launch_bounds__(WG) void k_diff_fill(T *dst, const T *a1, const T *
     }
 }
 
-// acc + p[i0] + p[i0 + WG] + ... over i < end, added in that order, with
-// four loads in flight at a time
-__device__ __forceinline__ double strided_sum(const double *__restrict__ p, int i0, int end, double acc) {
-    int i = i0;
-    for (; i + 3 * WG < end; i += 4 * WG) {
-        const double p0 = p[i], p1 = p[i + WG], p2 = p[i + 2 * WG], p3 = p[i + 3 * WG];
-        acc += p0;
-        acc += p1;
-        acc += p2;
-        acc += p3;
-    }
-    for (; i < end; i += WG) acc += p[i];
-    return acc;
-}
-
-// First stage of a fixed-order sum: work group g sums the contiguous chunk
-// [g * chunk, (g + 1) * chunk) of the n partials.
-__global__ __launch_bounds__(WG) void k_sum_chunks(const double *__restrict__ partial, int n, int chunk,
-                                                   double *__restrict__ out) {
-    __shared__ double red[WG];
-    int lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
-    const double acc = strided_sum(partial, lo + (int)threadIdx.x, hi, 0.0);
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = WG / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[blockIdx.x] = red[0];
-}
-
-// Work group g sums the ranges rng[g * nr .. (g + 1) * nr) of the partials
-// (int2: first, count) in order into out[g]: the per-problem totals when one
-// launch holds several problems.
-__global__ __launch_bounds__(WG) void k_sum_ranges(const double *__restrict__ partial, const int2 *__restrict__ rng,
-                                                   int nr, double *__restrict__ out) {
-    __shared__ double red[WG];
+// Sums of the residual partials, one work group per tree: the ranges
+// rng[t nr .. (t + 1) nr) (int2: first, count) in order, each thread every
+// SUM_NT-th partial with 16 loads in flight, then a halving tree. out is
+// host memory that the device can write: no copy follows. (Two launches and a
+// copy before: 12 us per norm on one tree, 8 on several.)
+constexpr int SUM_NT = 1024;
+__global__ __launch_bounds__(SUM_NT) void k_sum_ranges(const double *__restrict__ partial,
+                                                       const int2 *__restrict__ rng, int nr,
+                                                       double *__restrict__ out) {
+    __shared__ double red[SUM_NT / 64];
+    const int tid = threadIdx.x;
     double acc = 0.0;
     for (int k = 0; k < nr; k++) {
         const int2 r = rng[blockIdx.x * nr + k];
-        acc = strided_sum(partial, r.x + (int)threadIdx.x, r.x + r.y, acc);
+        const int end = r.x + r.y;
+        for (int i = r.x + tid; i < end; i += 16 * SUM_NT) {
+            double p[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) p[j] = i + j * SUM_NT < end ? partial[i + j * SUM_NT] : 0.0;
+#pragma unroll
+            for (int j = 0; j < 16; j++) acc += p[j];
+        }
     }
-    red[threadIdx.x] = acc;
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) acc += __shfl_down(acc, w, 64);
+    if ((tid & 63) == 0) red[tid >> 6] = acc;
     __syncthreads();
-    for (int w = WG / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[blockIdx.x] = red[0];
-}
-
-// Sum n partials in a fixed order (single work group).
-__global__ __launch_bounds__(WG) void k_sum(const double *__restrict__ partial, int n, double *__restrict__ out) {
-    __shared__ double red[WG];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += WG) acc += partial[i];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = WG / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = red[0];
+    if (tid >= SUM_NT / 64) return;
+    acc = red[tid];
+#pragma unroll
+    for (int w = SUM_NT / 128; w > 0; w >>= 1) acc += __shfl_down(acc, w, SUM_NT / 64);
+    if (tid == 0) out[blockIdx.x] = acc;
 }
 
 // ---- fused red-black sweep ----
@@ -2159,21 +2128,29 @@ enum { RES_WRITE = 0, RES_NORM = 1, RES_DEFECT = 2 };
 //   RES_DEFECT: out (float) = b + L u / s = -r on the level's blocks, and
 //               partial[k] = wgt * sum of r^2 over block k if it is a leaf (else 0)
 // Each block's partial is an LDS tree sum in a fixed order.
+// (work group wg of nwg; sm: the work group's LDS)
+template <int D, int M, typename T, int BPW, int NT, int MODE>
+struct ResidTileLds {
+    double red[MODE == RES_WRITE ? 1 : BPW * NT];
+    T tile[BPW * Tile<D, M>::SZ];
+    BP<T> prm[BPW];
+    int tab[BPW * 2 * D], blks[BPW];
+};
 template <int D, int M, typename T, typename TO, int BPW, int NT, int MODE, int RD>
-__global__ __launch_bounds__(NT) void k_resid_tile(TO *__restrict__ out, const T *__restrict__ u,
-                                                   const T *__restrict__ b, const T *__restrict__ ib,
-                                                   const int *__restrict__ htab, const int *__restrict__ coord,
-                                                   const int *__restrict__ list, const int *__restrict__ isleaf,
-                                                   int n, LevelArgs<T> a, double wgt, double *__restrict__ partial) {
+__device__ __forceinline__ void resid_tile(ResidTileLds<D, M, T, BPW, NT, MODE> &sm, int wg, int nwg,
+                                           TO *__restrict__ out, const T *__restrict__ u, const T *__restrict__ b,
+                                           const T *__restrict__ ib, const int *__restrict__ htab,
+                                           const int *__restrict__ coord, const int *__restrict__ list,
+                                           const int *__restrict__ isleaf, int n, const LevelArgs<T> &a, double wgt,
+                                           double *__restrict__ partial) {
     using LY = Lay<D, M>;
     using TL = Tile<D, M>;
     constexpr int V = LY::V;
-    __shared__ T tile[BPW * TL::SZ];
-    __shared__ int tab[BPW * 2 * D];
-    __shared__ int blks[BPW];
-    __shared__ BP<T> prm[BPW];
-    __shared__ double red[MODE == RES_WRITE ? 1 : BPW * NT];
-    const int first = xcd_remap(blockIdx.x, gridDim.x) * BPW;
+    T *tile = sm.tile;
+    int *tab = sm.tab, *blks = sm.blks;
+    BP<T> *prm = sm.prm;
+    double *red = sm.red;
+    const int first = xcd_remap(wg, nwg) * BPW;
     const int nloc = min(BPW, n - first);
     const int *lst = (MODE == RES_NORM) ? list : nullptr;
     const int base = (MODE == RES_NORM) ? first : a.blk0 + first;
@@ -2258,6 +2235,17 @@ __global__ __launch_bounds__(NT) void k_resid_tile(TO *__restrict__ out, const T
     }
 }
 
+template <int D, int M, typename T, typename TO, int BPW, int NT, int MODE, int RD>
+__global__ __launch_bounds__(NT) void k_resid_tile(TO *__restrict__ out, const T *__restrict__ u,
+                                                   const T *__restrict__ b, const T *__restrict__ ib,
+                                                   const int *__restrict__ htab, const int *__restrict__ coord,
+                                                   const int *__restrict__ list, const int *__restrict__ isleaf,
+                                                   int n, LevelArgs<T> a, double wgt, double *__restrict__ partial) {
+    __shared__ ResidTileLds<D, M, T, BPW, NT, MODE> sm;
+    resid_tile<D, M, T, TO, BPW, NT, MODE, RD>(sm, blockIdx.x, gridDim.x, out, u, b, ib, htab, coord, list, isleaf, n, a,
+                                               wgt, partial);
+}
+
 // Stage sibling group g0 (2^D blocks from device block g0) of u into a
 // Tile<D, M, 2> with the halo of the group's exterior faces, its halo table
 // entries and block parameters; every load of a phase is issued before the
@@ -2325,24 +2313,30 @@ __device__ __forceinline__ void stage_group(T *tile, int *tab, BP<T> *prm, const
 // threads take one block at a time and visit its cells in the order of
 // k_resid_tile<.., 1, RT, ..> (cells t, t + RT, ...; partials as the same
 // RT-wide tree sum), so outputs and partials are bitwise the same.
-template <int D, int M, typename T, typename TO, int RT, int MODE, int RD, int NT = 1024>
-__global__ __launch_bounds__(NT) void k_resid_group(TO *__restrict__ out, const T *__restrict__ u,
-                                                      const T *__restrict__ b, const T *__restrict__ ib,
-                                                      const int *__restrict__ htab, const int *__restrict__ coord,
-                                                      const int *__restrict__ isleaf, LevelArgs<T> a, double wgt,
-                                                      double *__restrict__ partial) {
+template <int D, int M, typename T, int MODE, int NT>
+struct ResidGroupLds {
+    double red[MODE == RES_DEFECT ? NT : 1];
+    T tile[Tile<D, M, 2>::SZ];
+    BP<T> prm[1 << D];
+    int tab[(1 << D) * 2 * D];
+};
+template <int D, int M, typename T, typename TO, int RT, int MODE, int RD, int NT>
+__device__ __forceinline__ void resid_group(ResidGroupLds<D, M, T, MODE, NT> &sm, int wg, int nwg,
+                                            TO *__restrict__ out, const T *__restrict__ u, const T *__restrict__ b,
+                                            const T *__restrict__ ib, const int *__restrict__ htab,
+                                            const int *__restrict__ coord, const int *__restrict__ isleaf,
+                                            const LevelArgs<T> &a, double wgt, double *__restrict__ partial) {
     using LY = Lay<D, M>;
     using TL = Tile<D, M, 2>;
-    using HT = Halo<D>;
-    constexpr int NB = 1 << D, V = LY::V, F = LY::F;
+    constexpr int NB = 1 << D, V = LY::V;
     constexpr int TEAMS = NT / RT;
     static_assert(NB % TEAMS == 0 && RT >= 64, "team layout");
-    __shared__ T tile[TL::SZ];
-    __shared__ int tab[NB * 2 * D];
-    __shared__ BP<T> prm[NB];
-    __shared__ double red[MODE == RES_DEFECT ? NT : 1];
+    T *tile = sm.tile;
+    int *tab = sm.tab;
+    BP<T> *prm = sm.prm;
+    double *red = sm.red;
     constexpr int NR = NB / TEAMS, QR = (V + RT - 1) / RT;
-    const int gl = xcd_remap(blockIdx.x, gridDim.x);
+    const int gl = xcd_remap(wg, nwg);
     const int g0 = a.blk0 + gl * NB;
     const int tid = threadIdx.x;
     const int team = tid / RT, t = tid - team * RT;
@@ -2425,6 +2419,17 @@ __global__ __launch_bounds__(NT) void k_resid_group(TO *__restrict__ out, const 
             __syncthreads();
         }
     }
+}
+
+template <int D, int M, typename T, typename TO, int RT, int MODE, int RD, int NT = 1024>
+__global__ __launch_bounds__(NT) void k_resid_group(TO *__restrict__ out, const T *__restrict__ u,
+                                                      const T *__restrict__ b, const T *__restrict__ ib,
+                                                      const int *__restrict__ htab, const int *__restrict__ coord,
+                                                      const int *__restrict__ isleaf, LevelArgs<T> a, double wgt,
+                                                      double *__restrict__ partial) {
+    __shared__ ResidGroupLds<D, M, T, MODE, NT> sm;
+    resid_group<D, M, T, TO, RT, MODE, RD, NT>(sm, blockIdx.x, gridDim.x, out, u, b, ib, htab, coord, isleaf, a, wgt,
+                                               partial);
 }
 
 // The V-cycle descent's residual and restrictions on a level of complete
@@ -2790,17 +2795,18 @@ struct ColDefect {
     }
 };
 
+// work group wg of nwg
 template <int D, int M, int RD>
-__global__ __launch_bounds__(256) void k_defect_col(float *__restrict__ out, const double *__restrict__ u,
-                                                    const double *__restrict__ b, const double *__restrict__ ib,
-                                                    const int *__restrict__ htab, const int *__restrict__ isleaf,
-                                                    LevelArgs<double> a, double wgt, double *__restrict__ partial) {
+__device__ __forceinline__ void defect_col(typename ColDefect<D, M, RD>::Smem &sm, int wg, int nwg,
+                                           float *__restrict__ out, const double *__restrict__ u,
+                                           const double *__restrict__ b, const double *__restrict__ ib,
+                                           const int *__restrict__ htab, const int *__restrict__ isleaf,
+                                           const LevelArgs<double> &a, double wgt, double *__restrict__ partial) {
     using CD = ColDefect<D, M, RD>;
     using HT = Halo<D>;
     constexpr int ND = CD::ND;
-    __shared__ typename CD::Smem sm;
     const int tid = threadIdx.x;
-    const int g0 = a.blk0 + xcd_remap(blockIdx.x, gridDim.x) * CD::NB;
+    const int g0 = a.blk0 + xcd_remap(wg, nwg) * CD::NB;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     int tv = 0;
     if (tid < CD::NB * ND) {
@@ -2814,6 +2820,70 @@ __global__ __launch_bounds__(256) void k_defect_col(float *__restrict__ out, con
     }
     if (w & 1) CD::template run<1>(sm, out, u, b, ib, a, g0, w, lane, tv, bpl, wgt, partial);
     else CD::template run<0>(sm, out, u, b, ib, a, g0, w, lane, tv, bpl, wgt, partial);
+}
+
+// ---- residual norms and defects of several levels in one launch ----
+//
+// A solve's norm needs every level, and a level that does not fill the chip
+// costs a launch of 5 to 8 us whatever its size. Each segment is one level
+// with the kernel that suits it: resid_tile on its leaves (NORM) or blocks,
+// resid_group or defect_col on complete sibling groups. Segments start at
+// multiples of eight work groups, so that xcd_remap's places hold.
+enum { SEG_TILE = 0, SEG_GROUP = 1, SEG_COL = 2 };
+template <typename T>
+struct ResidSeg {
+    LevelArgs<T> a;
+    double wgt;
+    int wg0, nwg;  // its work groups
+    int kind;
+    int n, list0;  // SEG_TILE: blocks, and where its leaves start in the list (NORM)
+    int p0;        // its first partial
+};
+constexpr int SEG_MAX = 12;
+template <typename T>
+struct ResidSegs {
+    ResidSeg<T> s[SEG_MAX];
+    int n;
+};
+
+template <int D, int M, typename T, typename TO, int BPW, int NT, bool NORM, int RD>
+__global__ __launch_bounds__(NT) void k_resid_levels(ResidSegs<T> g, TO *__restrict__ out, const T *__restrict__ u,
+                                                     const T *__restrict__ b, const T *__restrict__ ib,
+                                                     const int *__restrict__ htab, const int *__restrict__ coord,
+                                                     const int *__restrict__ leaves, const int *__restrict__ isleaf,
+                                                     double *__restrict__ partial) {
+    constexpr bool GROUPS = D == 2 && M == 16 && NT == 256, COLS = D == 3 && M == 8 && RD < 0 && sizeof(T) == 8;
+    constexpr int TM = NORM ? RES_NORM : RES_DEFECT;
+    using TileLds = ResidTileLds<D, M, T, BPW, NT, TM>;
+    using GroupLds = ResidGroupLds<D, M, T, RES_DEFECT, GROUPS ? NT : 1>;
+    constexpr size_t tb = sizeof(TileLds), gb = GROUPS ? sizeof(GroupLds) : 0;
+    size_t constexpr cb = [] {
+        if constexpr (COLS) return sizeof(typename ColDefect<D, M, RD>::Smem);
+        else return (size_t)0;
+    }();
+    __shared__ __align__(16) char sm[tb > gb ? (tb > cb ? tb : cb) : (gb > cb ? gb : cb)];
+    int k = 0;
+    while (k + 1 < g.n && (int)blockIdx.x >= g.s[k + 1].wg0) k++;
+    const ResidSeg<T> &s = g.s[k];
+    const int wg = blockIdx.x - s.wg0;
+    if (wg >= s.nwg) return;
+    if constexpr (GROUPS) {
+        if (s.kind == SEG_GROUP) {
+            resid_group<D, M, T, TO, NT, RES_DEFECT, RD, NT>(*reinterpret_cast<GroupLds *>(sm), wg, s.nwg, out, u, b, ib,
+                                                             htab, coord, isleaf, s.a, s.wgt, partial + s.p0);
+            return;
+        }
+    }
+    if constexpr (COLS) {
+        if (s.kind == SEG_COL) {
+            defect_col<D, M, RD>(*reinterpret_cast<typename ColDefect<D, M, RD>::Smem *>(sm), wg, s.nwg,
+                                 (float *)out, u, b, ib, htab, isleaf, s.a, s.wgt, partial + s.p0);
+            return;
+        }
+    }
+    resid_tile<D, M, T, TO, BPW, NT, TM, RD>(*reinterpret_cast<TileLds *>(sm), wg, s.nwg, out, u, b, ib, htab, coord,
+                                             NORM ? leaves + s.list0 : nullptr, isleaf, s.n, s.a, s.wgt,
+                                             partial + s.p0);
 }
 
 template <int D, int M, typename T, int RD>
@@ -3030,10 +3100,14 @@ __global__ __launch_bounds__(WG) void k_fb_setouter(double *__restrict__ q, cons
 // resnorm partials of u = 0 (the residual is -b): the same blocks, visiting
 // order and tree sums as k_resid_tile<RES_NORM>, so the partials are bitwise
 // those of a residual norm of a zero field, without reading one. be (may be
-// null) receives (float) b on the visited blocks.
+// null) receives (float) b on the visited blocks. list: the leaves of all
+// levels, lv.first[l] .. of level l, weighted by 2^(-D l).
+struct LeafLevels {
+    int n, first[32];
+};
 template <int D, int M, typename T, int BPW, int NT>
 __global__ __launch_bounds__(NT) void k_bnorm(const T *__restrict__ b, const int *__restrict__ list, int n,
-                                              double wgt, double *__restrict__ partial, float *__restrict__ be) {
+                                              LeafLevels lv, double *__restrict__ partial, float *__restrict__ be) {
     constexpr int V = Lay<D, M>::V;
     __shared__ int blks[BPW];
     __shared__ double red[BPW * NT];
@@ -3085,7 +3159,11 @@ __global__ __launch_bounds__(NT) void k_bnorm(const T *__restrict__ b, const int
             const double o = __shfl_down(v, w, 64);
             if (lane < w) v += o;
         }
-        if (lane == 0 && lb < nloc) partial[first + lb] = v * wgt;
+        if (lane == 0 && lb < nloc) {
+            int l = 0;
+            while (l + 1 < lv.n && first + lb >= lv.first[l + 1]) l++;
+            partial[first + lb] = v * ldexp(1.0, -D * l);
+        }
     }
 }
 

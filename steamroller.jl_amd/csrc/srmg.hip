@@ -28,11 +28,6 @@
 
 using namespace srmg;
 
-// first-stage work groups of the fixed-order sum of partials
-constexpr int SUM_CHUNKS = 256;
-// per-tree totals start here in d_sum
-constexpr int TSUM = SUM_CHUNKS + 4;
-
 // ---------------------------------------------------------------------------
 // context
 // ---------------------------------------------------------------------------
@@ -98,6 +93,25 @@ struct Graph {
         if (x) (void)hipGraphExecDestroy(x);
         if (g) (void)hipGraphDestroy(g);
     }
+};
+
+// Pinned host memory that kernels write directly.
+struct PinnedBuf {
+    double *host = nullptr, *dev = nullptr;
+    size_t bytes = 0;
+    void reserve(size_t n) {
+        if (n <= bytes) return;
+        release();
+        HIPCHK(hipHostMalloc((void **)&host, n, hipHostMallocDefault));
+        HIPCHK(hipHostGetDevicePointer((void **)&dev, host, 0));
+        bytes = n;
+    }
+    void release() {
+        if (host) (void)hipHostFree(host);
+        host = dev = nullptr;
+        bytes = 0;
+    }
+    ~PinnedBuf() { release(); }
 };
 
 // Pinned host buffers that kernels read and write, through which host fields
@@ -171,7 +185,8 @@ struct srmg_ctx {
     // device tables
     DevBuf d_nbr, d_coord, d_parent, d_sub, d_slots, d_leaves, d_halo, d_isleaf, d_pix;
     DevBuf d_w64, d_w32;    // radial weights (double / float), per level and dim
-    DevBuf d_partial, d_sum;
+    DevBuf d_partial;
+    PinnedBuf norms;        // per tree: the sum of the norm queued last, written by the device
     DevBuf d_rng_leaf, d_rng_blk;  // per (tree, level): ranges of the leaf / block partials
     DevBuf d_gord;                 // per grouped 3D level: processing order of its sibling groups
     DevBuf d_grid, d_grid2; // stacked level-1 uniform grids (coarse solve)
@@ -666,7 +681,7 @@ static void upload_tables(srmg_ctx *c) {
     // per-block partials: at most one per block of every level
     c->maxpartials = nb + 16;
     c->d_partial.alloc((size_t)c->maxpartials * sizeof(double));
-    c->d_sum.alloc(sizeof(double) * (SUM_CHUNKS + 4 + nt));
+    c->norms.reserve(nt * sizeof(double));
     size_t ng = 0;
     // the 2D solve takes all groups at once, the others one after the other
     for (auto &G : c->groups) {
@@ -1200,21 +1215,10 @@ struct Ops {
         hipLaunchKernelGGL((k_residual<D, M, T>), dim3(nwg((int64_t)a.nblk * LY::V)), dim3(WG), 0, c->stream,
                            X(r, l), X(u, l), X(b, l), I(u), nbr(), coord(), a);
     }
-    // fixed-order totals of the partials: one tree -> d_sum[0] (chunked
-    // two-stage sum of the first np partials); several trees -> one total per
-    // tree at d_sum[TSUM + t] over its (tree, level) ranges
-    void sum_partials(int np, const DevBuf &ranges) {
-        if (c->trees.size() == 1) {
-            int chunk = (np + SUM_CHUNKS - 1) / SUM_CHUNKS;
-            double *p2 = c->d_sum.as<double>() + 4;
-            hipLaunchKernelGGL(k_sum_chunks, dim3(SUM_CHUNKS), dim3(WG), 0, c->stream, c->d_partial.as<double>(), np,
-                               chunk, p2);
-            hipLaunchKernelGGL(k_sum, dim3(1), dim3(WG), 0, c->stream, p2, SUM_CHUNKS, c->d_sum.as<double>());
-        } else {
-            hipLaunchKernelGGL(k_sum_ranges, dim3((unsigned)c->trees.size()), dim3(WG), 0, c->stream,
-                               c->d_partial.as<double>(), ranges.as<int2>(), c->nlevels,
-                               c->d_sum.as<double>() + TSUM);
-        }
+    // fixed-order total of every tree's partials over its (tree, level) ranges
+    void sum_partials(const DevBuf &ranges) {
+        hipLaunchKernelGGL(k_sum_ranges, dim3((unsigned)c->trees.size()), dim3(SUM_NT), 0, c->stream,
+                           c->d_partial.as<double>(), ranges.as<int2>(), c->nlevels, c->norms.dev);
     }
     void restrict_(FieldBuf &x, int l) {
         const LevelInfo &L = c->lv[l];
@@ -1478,64 +1482,71 @@ struct Ops {
         hipLaunchKernelGGL((k_fill_interp<D, M, T>), dim3(nwg((int64_t)L.nslot * LY::F)), dim3(WG), 0, c->stream,
                            I(x), X(x, l - 1), nbr(), c->d_slots.as<int4>(), L.slot0, L.nslot, ac);
     }
-    // queue the squared-residual sums (leaf blocks, weighted by 2^(-D(l-1))) and their totals
-    int resnorm_partials(FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
-        int np = 0;
-        for (int l = 0; l < c->nlevels; l++) {
-            const LevelInfo &L = c->lv[l];
-            if (!L.nleaf) continue;
-            LevelArgs<T> a = level_args<T>(c, l, s, op, 1.0);
-            double wgt = std::ldexp(1.0, -c->D * l);
-            unsigned g = (unsigned)((L.nleaf + RB - 1) / RB);
-            with_rd(a.rdim, [&](auto rd) {
+    // residual norms (NORM: of the leaf blocks, out unused) or defects into out
+    // with the norms' partials (of every block), all levels in one launch for
+    // each SEG_MAX of them; levels keep their values in the primary buffer
+    template <bool NORM, typename TO>
+    void resid_levels(TO *out, FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
+        settle(u);
+        settle(b);
+        ResidSegs<T> g{};
+        int wgs = 0, np = 0, rdim = -1;
+        auto flush = [&] {
+            if (!g.n) return;
+            with_rd(rdim, [&](auto rd) {
                 constexpr int RD = decltype(rd)::value;
-                // grouped 3D 8^3 Cartesian level of leaves in block order: the
-                // column form (the same per-block sums)
-                if constexpr (GROUP_OK && D == 3 && M == 8 && RD < 0 && std::is_same<T, double>::value) {
-                    if (grouped(l) && L.all_leaves) {
-                        hipLaunchKernelGGL((k_defect_col<D, M, RD>), dim3((unsigned)(L.nblk >> D)), dim3(256), 0,
-                                           c->stream, (float *)nullptr, X(u, l), X(b, l), I(u),
-                                           c->d_halo.as<int>(), c->d_isleaf.as<int>(), a, wgt,
-                                           c->d_partial.as<double>() + np);
-                        return;
-                    }
-                }
-                // grouped 2D level of leaves in block order: the sibling-group
-                // form, partials only (the same per-block sums)
-                if constexpr (GROUP_OK && D == 2) {
-                    if (grouped(l) && L.all_leaves) {
-                        hipLaunchKernelGGL((k_resid_group<D, M, T, T, RNT, RES_DEFECT, RD, GNT>),
-                                           dim3((unsigned)(L.nblk >> D)), dim3(GNT), 0, c->stream, (T *)nullptr,
-                                           X(u, l), X(b, l), I(u), c->d_halo.as<int>(), coord(),
-                                           c->d_isleaf.as<int>(), a, wgt, c->d_partial.as<double>() + np);
-                        return;
-                    }
-                }
-                hipLaunchKernelGGL((k_resid_tile<D, M, T, T, RB, RNT, RES_NORM, RD>), dim3(g), dim3(RNT), 0,
-                                   c->stream, (T *)nullptr, X(u, l), X(b, l), I(u), c->d_halo.as<int>(), coord(),
-                                   c->d_leaves.as<int>() + L.leaf0, (const int *)nullptr, L.nleaf, a, wgt,
-                                   c->d_partial.as<double>() + np);
+                hipLaunchKernelGGL((k_resid_levels<D, M, T, TO, RB, RNT, NORM, RD>), dim3((unsigned)wgs), dim3(RNT), 0,
+                                   c->stream, g, out, u.data.as<T>(), b.data.as<T>(), I(u), c->d_halo.as<int>(),
+                                   coord(), c->d_leaves.as<int>(), c->d_isleaf.as<int>(), c->d_partial.as<double>());
             });
-            np += L.nleaf;
+            g.n = 0;
+            wgs = 0;
+        };
+        // largest (finest) levels first: the small ones run beside their tail
+        std::vector<int> p0(c->nlevels);
+        for (int l = 0; l < c->nlevels; l++) {
+            p0[l] = np;
+            np += NORM ? c->lv[l].nleaf : c->lv[l].nblk;
         }
-        sum_partials(np, c->d_rng_leaf);
-        return np;
+        for (int l = c->nlevels - 1; l >= 0; l--) {
+            const LevelInfo &L = c->lv[l];
+            if (!(NORM ? L.nleaf : L.nblk)) continue;
+            if (g.n == SEG_MAX) flush();
+            ResidSeg<T> &q = g.s[g.n++];
+            q.a = level_args<T>(c, l, s, op, 1.0);
+            rdim = q.a.rdim;
+            q.wgt = std::ldexp(1.0, -c->D * l);
+            // complete sibling groups; for a norm only where every block is a
+            // leaf in block order (the same per-block sums)
+            const bool gr = GROUP_OK && grouped(l) && (!NORM || L.all_leaves);
+            q.kind = !gr ? SEG_TILE : D == 2 ? SEG_GROUP : (q.a.rdim < 0 && std::is_same<T, double>::value) ? SEG_COL : SEG_TILE;
+            q.n = NORM ? L.nleaf : L.nblk;
+            q.list0 = L.leaf0;
+            q.nwg = q.kind == SEG_TILE ? (q.n + RB - 1) / RB : L.nblk >> D;
+            q.wg0 = wgs;
+            q.p0 = p0[l];
+            wgs += (q.nwg + 7) / 8 * 8;
+        }
+        flush();
+    }
+    // queue the squared-residual sums (leaf blocks, weighted by 2^(-D(l-1))) and their totals
+    void resnorm_partials(FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
+        resid_levels<true>((T *)nullptr, u, b, s, op);
+        sum_partials(c->d_rng_leaf);
     }
     // resnorm partials of u = 0 from b alone (bitwise those of resnorm_partials
     // on a zero field); be (may be null): (float) b on every leaf block
-    int bnorm_partials(FieldBuf &b, float *be = nullptr) {
-        int np = 0;
-        for (int l = 0; l < c->nlevels; l++) {
-            const LevelInfo &L = c->lv[l];
-            if (!L.nleaf) continue;
-            double wgt = std::ldexp(1.0, -c->D * l);
-            unsigned g = (unsigned)((L.nleaf + BB - 1) / BB);
-            hipLaunchKernelGGL((k_bnorm<D, M, T, BB, RNT>), dim3(g), dim3(RNT), 0, c->stream, X(b, l),
-                               c->d_leaves.as<int>() + L.leaf0, L.nleaf, wgt, c->d_partial.as<double>() + np, be);
-            np += L.nleaf;
-        }
-        sum_partials(np, c->d_rng_leaf);
-        return np;
+    void bnorm_partials(FieldBuf &b, float *be = nullptr) {
+        settle(b);
+        const int n = (int)c->h_leaves.size();
+        LeafLevels lv{};
+        if (c->nlevels > 32) fail("more than 32 levels");
+        lv.n = c->nlevels;
+        for (int l = 0; l < c->nlevels; l++) lv.first[l] = c->lv[l].leaf0;
+        if (n)
+            hipLaunchKernelGGL((k_bnorm<D, M, T, BB, RNT>), dim3((unsigned)((n + BB - 1) / BB)), dim3(RNT), 0, c->stream,
+                               b.data.as<T>(), c->d_leaves.as<int>(), n, lv, c->d_partial.as<double>(), be);
+        sum_partials(c->d_rng_leaf);
     }
     // u = 0 on every level and slab (values in the primary buffer)
     void zero_all(FieldBuf &u) {
@@ -1547,39 +1558,8 @@ struct Ops {
     // mixed precision: be = b + L u / s (FP32) on every level, plus the leaf
     // residual norm partials, in one pass (T = double)
     void defect_and_norm(float *be, FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
-        int np = 0;
-        for (int l = 0; l < c->nlevels; l++) {
-            LevelArgs<T> a = level_args<T>(c, l, s, op, 1.0);
-            if (!a.nblk) continue;
-            double wgt = std::ldexp(1.0, -c->D * l);
-            unsigned g = (unsigned)((a.nblk + RB - 1) / RB);
-            bool grouped = false;
-            if constexpr (GROUP_OK) grouped = this->grouped(l);
-            with_rd(a.rdim, [&](auto rd) {
-                constexpr int RD = decltype(rd)::value;
-                if constexpr (GROUP_OK) {
-                    if (grouped) {
-                        // 3D 8^3 Cartesian: the column form (k_defect_col), same bits
-                        if constexpr (D == 3 && M == 8 && RD < 0 && std::is_same<T, double>::value)
-                            hipLaunchKernelGGL((k_defect_col<D, M, RD>), dim3((unsigned)(a.nblk >> D)), dim3(256),
-                                               0, c->stream, be, X(u, l), X(b, l), I(u), c->d_halo.as<int>(),
-                                               c->d_isleaf.as<int>(), a, wgt, c->d_partial.as<double>() + np);
-                        else
-                            hipLaunchKernelGGL((k_resid_group<D, M, T, float, RNT, RES_DEFECT, RD, GNT>),
-                                               dim3((unsigned)(a.nblk >> D)), dim3(GNT), 0, c->stream, be,
-                                               X(u, l), X(b, l), I(u), c->d_halo.as<int>(), coord(),
-                                               c->d_isleaf.as<int>(), a, wgt, c->d_partial.as<double>() + np);
-                        return;
-                    }
-                }
-                hipLaunchKernelGGL((k_resid_tile<D, M, T, float, RB, RNT, RES_DEFECT, RD>), dim3(g), dim3(RNT), 0,
-                                   c->stream, be, X(u, l), X(b, l), I(u), c->d_halo.as<int>(), coord(),
-                                   (const int *)nullptr, c->d_isleaf.as<int>(), a.nblk, a, wgt,
-                                   c->d_partial.as<double>() + np);
-            });
-            np += a.nblk;
-        }
-        sum_partials(np, c->d_rng_blk);
+        resid_levels<false>(be, u, b, s, op);
+        sum_partials(c->d_rng_blk);
     }
 
     // coarse_exact of 2D trees whose level-1 extents are at most 256, every
@@ -2318,14 +2298,8 @@ static Graph &solve_graph(srmg_ctx *c, int kind, std::initializer_list<const Fie
 
 // the residual norms queued last (one per tree)
 static std::vector<double> read_norms(srmg_ctx *c) {
-    const int nt = (int)c->trees.size();
-    std::vector<double> v(nt);
-    if (nt == 1)
-        HIPCHK(hipMemcpyAsync(v.data(), c->d_sum.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    else
-        HIPCHK(hipMemcpyAsync(v.data(), c->d_sum.as<double>() + TSUM, nt * sizeof(double), hipMemcpyDeviceToHost,
-                              c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    std::vector<double> v(c->norms.host, c->norms.host + c->trees.size());
     for (auto &x : v) x = std::sqrt(x);
     return v;
 }
