@@ -71,12 +71,20 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// a field formed from two while it is read
+template <typename T>
+struct Diff {
+    const T *__restrict__ a, *__restrict__ b;
+    __device__ __forceinline__ T operator[](size_t i) const { return a[i] - b[i]; }
+};
+
 // Value of cell (c0,c1,c2) + dir e_dim of block blk, crossing the block face if
 // needed: same-level neighbour cell, mirror (depth-1 ghost = sign * own cell,
 // src/boundary.jl:45-47 with src/blockfield.jl:513-521), or the coarse-fine
 // ghost buffer.
-template <int D, int M, typename T>
-__device__ __forceinline__ T nbv(const T *__restrict__ x, const T *__restrict__ ib,
+// (x: a field's values, or a difference of two fields'.)
+template <int D, int M, typename T, class X>
+__device__ __forceinline__ T nbv(const X x, const T *__restrict__ ib,
                                  const int *__restrict__ nbr, int blk, int c0, int c1, int c2,
                                  int dim, int dir, const T *sg) {
     using LY = Lay<D, M>;
@@ -914,8 +922,8 @@ __global__ __launch_bounds__(WG) void k_regrid_restrict(T *__restrict__ un, cons
 // face. The coarse layer adjacent to the face feeds the fine ghost layer next
 // to the fine block's valid cells, i.e. child offset 1 on a low face and 0 on a
 // high face in the face dimension. `a` describes the coarse level (mirror signs).
-template <int D, int M, typename T>
-__device__ __forceinline__ void fill_interp_one(int gt, T *__restrict__ ib, const T *__restrict__ x,
+template <int D, int M, typename T, class X>
+__device__ __forceinline__ void fill_interp_one(int gt, T *__restrict__ ib, const X x,
                                                 const int *__restrict__ nbr, const int4 *__restrict__ slots,
                                                 int slot0, int nslot, const LevelArgs<T> &a) {
     using LY = Lay<D, M>;
@@ -1121,9 +1129,8 @@ __device__ __forceinline__ int halo_at(int t) {
     return TL::at(c[0], c[1], c[2]);
 }
 
-template <int D, int M, typename T, int F>
-__device__ __forceinline__ T halo_value(int e, int blk, int t, const T *__restrict__ x, const T *__restrict__ ib,
-                                        T sg) {
+template <int D, int M, typename T, int F, class X>
+__device__ __forceinline__ T halo_value(int e, int blk, int t, const X x, const T *__restrict__ ib, T sg) {
     using LY = Lay<D, M>;
     constexpr int DIM = F >> 1, DIR = (F & 1) ? 1 : -1;
     int c[3] = {0, 0, 0};
@@ -1165,9 +1172,9 @@ __device__ __forceinline__ void halo_switch(T *tl, int e, int f, int blk, int t,
     SRMG_FACE_SWITCH(f, (halo_cell<D, M, T, FF, TL>(tl, e, blk, t, x, ib, sg[FF])))
 }
 
-template <int D, int M, typename T>
-__device__ __forceinline__ T halo_value_sw(int f, int e, int blk, int t, const T *__restrict__ x,
-                                           const T *__restrict__ ib, const T *sg) {
+template <int D, int M, typename T, class X>
+__device__ __forceinline__ T halo_value_sw(int f, int e, int blk, int t, const X x, const T *__restrict__ ib,
+                                           const T *sg) {
     T v = T(0);
     SRMG_FACE_SWITCH(f, (v = halo_value<D, M, T, FF>(e, blk, t, x, ib, sg[FF])))
     return v;
@@ -1996,9 +2003,9 @@ struct NoLoads {
 // (LDSB: barriers that order LDS only, for callers with loads in flight).
 // with1 and with2 issue the caller's own loads with the first and the second
 // round trip; with2 may also store to LDS what is read after the call.
-template <int D, int M, typename T, int BPW, int NT, bool LDSB = false, class W1 = NoLoads, class W2 = NoLoads>
-__device__ __forceinline__ void load_tile(T *tile, int *tab, int *blks, const T *__restrict__ x,
-                                          const T *__restrict__ ib, const int *__restrict__ htab,
+template <int D, int M, typename T, int BPW, int NT, bool LDSB = false, class W1 = NoLoads, class W2 = NoLoads,
+          class X = const T *>
+__device__ __forceinline__ void load_tile(T *tile, int *tab, int *blks, const X x, const T *__restrict__ ib, const int *__restrict__ htab,
                                           const int *__restrict__ list, int first, int nloc, const T *sg,
                                           W1 &&with1 = W1(), W2 &&with2 = W2()) {
     using LY = Lay<D, M>;
@@ -2058,8 +2065,8 @@ __device__ __forceinline__ void load_tile(T *tile, int *tab, int *blks, const T 
 // halo: neighbour cells, mirrors, coarse-fine slabs of level l-1) in LDS and
 // interpolates every child cell from there. Same operations and order as
 // k_interp_add, so the result is bitwise the same.
-template <int D, int M, typename T, int NT>
-__device__ __forceinline__ void interp_add_group_one(int g, T *__restrict__ u, const T *__restrict__ u1,
+template <int D, int M, typename T, int NT, class X>
+__device__ __forceinline__ void interp_add_group_one(int g, T *__restrict__ u, const X u1,
                                                      const T *__restrict__ ib1, const int *__restrict__ htab,
                                                      const int *__restrict__ parent, int blk0,
                                                      const LevelArgs<T> &ac) {
@@ -2076,7 +2083,7 @@ __device__ __forceinline__ void interp_add_group_one(int g, T *__restrict__ u, c
     T uo[NB * V / NT];
 #pragma unroll
     for (int k = 0; k < NB * V / NT; k++) uo[k] = u[(size_t)g0 * V + threadIdx.x + k * NT];
-    load_tile<D, M, T, 1, NT, true>(tile, tab, blks, u1, ib1, htab, nullptr, pb, 1, ac.sg);
+    load_tile<D, M, T, 1, NT, true, NoLoads, NoLoads, X>(tile, tab, blks, u1, ib1, htab, nullptr, pb, 1, ac.sg);
 #pragma unroll
     for (int k = 0; k < NB * V / NT; k++) {
         const int i = threadIdx.x + k * NT, lb = i / V, q = i - lb * V;
@@ -2118,6 +2125,30 @@ __global__ __launch_bounds__(NT) void k_interp_fill_group(T *__restrict__ u, con
         interp_add_group_one<D, M, T, NT>(blockIdx.x, u, u1, ib1, htab, parent, blk0, ac);
     else
         fill_interp_one<D, M, T>((blockIdx.x - ngroups) * NT + threadIdx.x, ibu, xc, nbr, slots, slot0, nslot, ac);
+}
+
+// k_interp_fill_group with the correction u - u1 of the coarse level formed as
+// it is read (u1: u there before the correction) instead of by a launch of its
+// own (k_diff_fill, 3 to 5 us on a small level and a pass over the coarse level on
+// a large one). The work groups past ngroups + nwg_fill fill u1's slabs of the
+// fine level with the correction's ghosts, which the next finer level's
+// prolongation reads (nslot1: 0 on the finest level).
+template <int D, int M, typename T, int NT>
+__global__ __launch_bounds__(NT) void k_interp_fill_diff(T *__restrict__ u, const T *__restrict__ uc,
+                                                         const T *__restrict__ u1c, T *__restrict__ ib1,
+                                                         const int *__restrict__ htab,
+                                                         const int *__restrict__ parent, int blk0, unsigned ngroups,
+                                                         unsigned nwg_fill, T *__restrict__ ibu,
+                                                         const int *__restrict__ nbr, const int4 *__restrict__ slots,
+                                                         int slot0, int nslot, int nslot1, LevelArgs<T> ac) {
+    const Diff<T> d{uc, u1c};
+    if (blockIdx.x < ngroups)
+        interp_add_group_one<D, M, T, NT>(blockIdx.x, u, d, ib1, htab, parent, blk0, ac);
+    else if (blockIdx.x < ngroups + nwg_fill)
+        fill_interp_one<D, M, T>((blockIdx.x - ngroups) * NT + threadIdx.x, ibu, uc, nbr, slots, slot0, nslot, ac);
+    else
+        fill_interp_one<D, M, T>((blockIdx.x - ngroups - nwg_fill) * NT + threadIdx.x, ib1, d, nbr, slots, slot0,
+                                 nslot1, ac);
 }
 
 enum { RES_WRITE = 0, RES_NORM = 1, RES_DEFECT = 2 };

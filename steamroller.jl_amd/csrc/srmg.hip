@@ -1475,6 +1475,29 @@ struct Ops {
         interp_add(u, u1, l, ac);
         fill_interp(u, l, ac);
     }
+    // diff_fill(u1, u, l - 1) and interp_fill(u, u1, l) in one launch on a
+    // grouped level, with the slabs of the correction on level l where a finer
+    // level follows (k_interp_fill_diff; u1 keeps the values before the
+    // correction). ok_diff: every refined level below lmax is grouped
+    bool ok_diff(int lmax) const {
+        if constexpr ((LY::V << D) % 256 == 0 && (LY::V << D) / 256 <= 16) {
+            for (int l = 1; l < lmax; l++)
+                if (c->lv[l].nblk && !grouped(l)) return false;
+            return true;
+        }
+        return false;
+    }
+    void interp_fill_diff(FieldBuf &u, FieldBuf &u1, int l, const LevelArgs<T> &ac, bool finer) {
+        if constexpr ((LY::V << D) % 256 == 0 && (LY::V << D) / 256 <= 16) {
+            const LevelInfo &L = c->lv[l];
+            if (!L.nblk) return;
+            const unsigned ng = (unsigned)(L.nblk >> D), nf = nwg((int64_t)L.nslot * LY::F);
+            hipLaunchKernelGGL((k_interp_fill_diff<D, M, T, 256>), dim3(ng + nf + (finer ? nf : 0)), dim3(256), 0,
+                               c->stream, X(u, l), X(u, l - 1), X(u1, l - 1), I(u1), c->d_halo.as<int>(),
+                               c->d_parent.as<int>(), L.blk0, ng, nf, I(u), nbr(), c->d_slots.as<int4>(), L.slot0,
+                               L.nslot, finer ? L.nslot : 0, ac);
+        }
+    }
     // refresh the coarse-fine ghost slabs of level l from level l-1
     void fill_interp(FieldBuf &x, int l, const LevelArgs<T> &ac) {
         const LevelInfo &L = c->lv[l];
@@ -1625,9 +1648,11 @@ struct Ops {
     // back at the end so that every cycle starts from the same buffers.
     // zin: u and its ghost slabs are zero on the finest level lmax - 1 (its
     // first sweep reads none of them; only with zin_ok)
+    // in_fmg: fmg! goes on with the corrections that the reference leaves in u1
     void vcycle(FieldBuf &u, FieldBuf &b, FieldBuf &r, FieldBuf &u1, double s, const srmg_op *op, int lmax,
-                int ndown, int ntop, int nup, double omega, bool zin = false) {
+                int ndown, int ntop, int nup, double omega, bool zin = false, bool in_fmg = false) {
         if (lmax == 0) lmax = c->nlevels;
+        const bool diff_read = !in_fmg && ok_diff(lmax);
         for (int l = lmax - 1; l >= 1; l--) {
             LevelArgs<T> a = level_args<T>(c, l, s, op, omega);
             LevelArgs<T> ac = level_args<T>(c, l - 1, s, op, omega);
@@ -1644,13 +1669,17 @@ struct Ops {
         for (int l = 1; l < lmax; l++) {
             LevelArgs<T> a = level_args<T>(c, l, s, op, omega);
             LevelArgs<T> ac = level_args<T>(c, l - 1, s, op, omega);
-            if (l - 1 >= 1) {
-                LevelArgs<T> a2 = level_args<T>(c, l - 2, s, op, omega);
-                diff_fill(u1, u, l - 1, &a2);
+            if (diff_read) {
+                interp_fill_diff(u, u1, l, ac, l + 1 < lmax);
             } else {
-                diff_fill(u1, u, l - 1, nullptr);
+                if (l - 1 >= 1) {
+                    LevelArgs<T> a2 = level_args<T>(c, l - 2, s, op, omega);
+                    diff_fill(u1, u, l - 1, &a2);
+                } else {
+                    diff_fill(u1, u, l - 1, nullptr);
+                }
+                interp_fill(u, u1, l, ac);
             }
-            interp_fill(u, u1, l, ac);
             smooth(u, b, a, l, nup);
         }
         settle(u);
@@ -1694,7 +1723,7 @@ struct Ops {
                 }
                 interp_fill(u, u1, l, ac);
             }
-            vcycle(u, b, r, u1, s, op, l + 1, ndown, ntop, nup, omega);
+            vcycle(u, b, r, u1, s, op, l + 1, ndown, ntop, nup, omega, false, true);
         }
     }
 };
