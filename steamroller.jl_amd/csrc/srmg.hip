@@ -89,6 +89,8 @@ struct Graph {
     hipGraphExec_t x = nullptr;
     uint64_t gen = 0;     // srmg_ctx::graph_gen when captured
     bool ran = false;     // the step has run eagerly once (lazily built state exists)
+    bool vcycle = false;  // a single V-cycle's, called `calls` times
+    int calls = 0;
     ~Graph() {
         if (x) (void)hipGraphExecDestroy(x);
         if (g) (void)hipGraphDestroy(g);
@@ -545,6 +547,7 @@ static void set_forest(srmg_ctx *c, const std::vector<TreeRecords> &tr) {
 }
 
 static void commit_tables(srmg_ctx *c, srmg_ctx &t) {
+    HIPCHK(hipStreamSynchronize(c->stream));  // a replay of them may be running
     c->graphs.clear();
     c->box_ok = false;
     c->d_host2dev.release();
@@ -1227,17 +1230,17 @@ struct Ops {
                            c->stream, X(x, l - 1), X(x, l), c->d_parent.as<int>(), c->d_sub.as<int>(), L.blk0,
                            L.nblk);
     }
-    // rhs_level! (src/multigrid.jl:378-388) of level l: b1 = R b on every block
-    void rhs_level(FieldBuf &b1, FieldBuf &b, int l, const LevelArgs<T> &a, bool order4) {
+    // rhs_level! (src/multigrid.jl:378-388) of level l: the order-4 b1 = R b on every block
+    void rhs4_level(FieldBuf &b1, FieldBuf &b, int l, const LevelArgs<T> &a) {
         const LevelInfo &L = c->lv[l];
         if (!L.nblk) return;
-        const size_t n = (size_t)L.nblk * LY::V, o = (size_t)L.blk0 * LY::V;
-        if (order4)
-            hipLaunchKernelGGL((k_rhs4<D, M, T>), dim3(nwg((int64_t)n)), dim3(WG), 0, c->stream, X(b1, l), X(b, l),
-                               I(b), nbr(), coord(), a);
-        else
-            hipLaunchKernelGGL((k_copy<T>), dim3(nwg((int64_t)n)), dim3(WG), 0, c->stream, X(b1, l) + o,
-                               X(b, l) + o, n);
+        hipLaunchKernelGGL((k_rhs4<D, M, T>), dim3(nwg((int64_t)L.nblk * LY::V)), dim3(WG), 0, c->stream, X(b1, l),
+                           X(b, l), I(b), nbr(), coord(), a);
+    }
+    // every block's cells (both fields settled)
+    void copy_all(FieldBuf &dst, FieldBuf &src) {
+        const size_t n = (size_t)c->nb * LY::V;
+        hipLaunchKernelGGL((k_copy<T>), dim3(nwg(n)), dim3(WG), 0, c->stream, dst.data.as<T>(), src.data.as<T>(), n);
     }
     // ---- LaplacianDiscretization{D,4}: vcycle! (src/multigrid.jl:60-106) with
     // the four-colour smoother on complete levels, step by step ----
@@ -2277,6 +2280,18 @@ static void run_first_step(srmg_ctx *c, Graph &g, bool use_graph, F &&body) {
     g.ran = true;
 }
 
+// A caller who varies a V-cycle's parameters at every call leaves one entry
+// each: all of them go when they become many.
+constexpr int VCYCLE_GRAPHS = 64;
+static void drop_vcycle_graphs(srmg_ctx *c) {
+    int n = 0;
+    for (auto &e : c->graphs) n += e.second->vcycle;
+    if (n < VCYCLE_GRAPHS) return;
+    HIPCHK(hipStreamSynchronize(c->stream));  // none is running
+    for (auto it = c->graphs.begin(); it != c->graphs.end();)
+        it = it->second->vcycle ? c->graphs.erase(it) : std::next(it);
+}
+
 // The cached graph of a solve step: the key holds every value the step's
 // launches bake in. Field buffers keep their addresses until a regrid or a
 // field destroy, which clear the cache; coarse-solve matrices keep theirs until
@@ -2287,10 +2302,14 @@ static void run_first_step(srmg_ctx *c, Graph &g, bool use_graph, F &&body) {
 static Graph &solve_graph(srmg_ctx *c, int kind, std::initializer_list<const FieldBuf *> fs,
                           const srmg_solve_opts *o) {
     // drop graphs captured before the last coarse-solve rebuild (no solve is
-    // running here, so nothing refers to them)
+    // running here, so nothing refers to them; a V-cycle's replay may be)
     for (auto it = c->graphs.begin(); it != c->graphs.end();) {
-        if (it->second->x && it->second->gen != c->graph_gen) it = c->graphs.erase(it);
-        else ++it;
+        if (it->second->x && it->second->gen != c->graph_gen) {
+            HIPCHK(hipStreamSynchronize(c->stream));
+            it = c->graphs.erase(it);
+        } else {
+            ++it;
+        }
     }
     std::string k;
     auto add = [&](const auto &v) { k.append(reinterpret_cast<const char *>(&v), sizeof(v)); };
@@ -2320,8 +2339,12 @@ static Graph &solve_graph(srmg_ctx *c, int kind, std::initializer_list<const Fie
     add(c->group_tiles);
     add(c->axis_gemm);
     add(c->group_order);
+    if (kind == 4 && !c->graphs.count(k)) drop_vcycle_graphs(c);
     auto &slot = c->graphs[k];
-    if (!slot) slot = std::make_unique<Graph>();
+    if (!slot) {
+        slot = std::make_unique<Graph>();
+        slot->vcycle = kind == 4;
+    }
     return *slot;
 }
 
@@ -2952,8 +2975,10 @@ int srmg_rhs(srmg_ctx *c, int b1, int b, const srmg_op *op) {
             // (src/streamer.jl:314-318)
             for (int l = 0; l < c->nlevels; l++) {
                 if (l > 0) o.fill_interp(fb, l, level_args<T>(c, l - 1, 1.0, op, 1.0));
-                o.rhs_level(fb1, fb, l, level_args<T>(c, l, 1.0, op, 1.0), op->disc == SRMG_LAPLACIAN4);
+                if (op->disc == SRMG_LAPLACIAN4) o.rhs4_level(fb1, fb, l, level_args<T>(c, l, 1.0, op, 1.0));
             }
+            // order 2: b1 = b, on all levels at once
+            if (op->disc != SRMG_LAPLACIAN4) o.copy_all(fb1, fb);
         });
         HIPCHK(hipGetLastError());
     });
@@ -3078,14 +3103,30 @@ int srmg_fill_ghost_all(srmg_ctx *c, int id, const int8_t *bc) {
     });
 }
 
-static void do_vcycle(srmg_ctx *c, int u, int b, int r, int u1, int lmax, int ndown, int ntop, int nup,
+// A V-cycle on its own. Its 20 to 60 launches cost the host 3.6 us each when
+// issued one by one, more than a small tree's kernels take: from the third call
+// of a configuration on they are replayed as a graph (capturing costs about
+// what three calls save).
+static void do_vcycle(srmg_ctx *c, int ui, int bi, int ri, int u1i, int lmax, int ndown, int ntop, int nup,
                       double omega) {
     if (lmax < 0 || lmax > c->nlevels) fail("lmax out of range");
-    int t = same_type(c, {u, b, r, u1});
-    dispatch(c, t, [&](auto &o) {
-        o.vcycle(field(c, u), field(c, b), field(c, r), field(c, u1), c->ps[0], &c->pops[0], lmax, ndown, ntop, nup,
-                 omega);
+    const int t = same_type(c, {ui, bi, ri, u1i});
+    FieldBuf &u = field(c, ui), &b = field(c, bi), &r = field(c, ri), &u1 = field(c, u1i);
+    srmg_solve_opts o{};
+    o.ndown = ndown;
+    o.ntop = ntop;
+    o.nup = nup;
+    o.omega = omega;
+    o.inner_cycles = lmax;
+    Graph &g = solve_graph(c, 4, {&u, &b, &r, &u1}, &o);
+    dispatch(c, t, [&](auto &ops) {
+        // the captured launches start from and end in the primary buffers
+        for (FieldBuf *f : {&u, &b, &r, &u1}) ops.settle(*f);
+        run_maybe_graph(c, g, g.calls >= 2, [&] {
+            ops.vcycle(u, b, r, u1, c->ps[0], &c->pops[0], lmax, ndown, ntop, nup, omega);
+        });
     });
+    g.calls = std::min(g.calls + 1, 2);
     HIPCHK(hipGetLastError());
 }
 
