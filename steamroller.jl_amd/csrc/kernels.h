@@ -203,6 +203,44 @@ struct Bc27 {
     T v[27];
 };
 
+// restrict! (src/restrict.jl:5-37): a coarse cell of the parent subblock = mean
+// of its 2^D children, summed with the first index fastest. gt: the cell among
+// those covered by the level's blocks; its place (index o, block pb, X) and mean f
+template <int D, int M, typename T>
+__device__ __forceinline__ bool restricted(const T *__restrict__ xf, const int *__restrict__ parent,
+                                           const int *__restrict__ sub, int blk0, int nblk, int gt, size_t &o, int &pb,
+                                           int &X0, int &X1, int &X2, T &f) {
+    using LY = Lay<D, M>;
+    constexpr int NS = LY::V / LY::NC;  // coarse cells per subblock
+    const int lb = gt / NS;
+    if (lb >= nblk) return false;
+    const int fb = blk0 + lb, j = gt - lb * NS;
+    const int j0 = j % LY::MH, j1 = (j / LY::MH) % LY::MH, j2 = (D == 3) ? j / (LY::MH * LY::MH) : 0;
+    f = T(0);
+#pragma unroll
+    for (int q = 0; q < LY::NC; q++) {
+        int i0 = q & 1, i1 = (q >> 1) & 1, i2 = (q >> 2) & 1;
+        f += xf[(size_t)fb * LY::V + LY::sidx(2 * j0 + i0, 2 * j1 + i1, D == 3 ? 2 * j2 + i2 : 0)];
+    }
+    f = f / T(LY::NC);
+    pb = parent[fb];
+    const int sb = sub[fb];
+    X0 = (sb & 1) * LY::MH + j0;
+    X1 = ((sb >> 1) & 1) * LY::MH + j1;
+    X2 = (D == 3) ? ((sb >> 2) & 1) * LY::MH + j2 : 0;
+    o = (size_t)pb * LY::V + LY::sidx(X0, X1, X2);
+    return true;
+}
+template <int D, int M, typename T>
+__device__ __forceinline__ void restrict_cell(T *__restrict__ xc, const T *__restrict__ xf,
+                                              const int *__restrict__ parent, const int *__restrict__ sub, int blk0,
+                                              int nblk, int gt) {
+    size_t o;
+    int pb, X0, X1, X2;
+    T f;
+    if (restricted<D, M, T>(xf, parent, sub, blk0, nblk, gt, o, pb, X0, X1, X2, f)) xc[o] = f;
+}
+
 // ---- LaplacianDiscretization{D,4}: the 9- and 19-point operators ----
 //
 // Their stencils reach corner (2D) and edge (3D) ghosts, so the order-4 path
@@ -266,10 +304,10 @@ __device__ __forceinline__ bool frame_cell(int q, int *c, int *dir, int &k) {
 // the domain: a same-level neighbour's cell (read from the neighbour, the value
 // the copy writes) or a coarse-fine ghost (read from the frame, as the
 // interpolation that refills it comes after both fills). Coarse-fine ghosts
-// themselves are read from the frame.
+// themselves are read from the frame. row: the block's entries of box.
 template <int D, int M, typename T>
 __device__ __forceinline__ T ghost_value(const T *__restrict__ x, const T *__restrict__ g,
-                                         const int *__restrict__ box, const Bc27<T> &bc, int blk, int *c) {
+                                         const int *row, const Bc27<T> &bc, int blk, int *c) {
     using LY = Lay<D, M>;
     constexpr int P = Frame<D, M>::P, NB3 = D == 3 ? 27 : 9;
     int dir[3] = {0, 0, 0}, k = 0, m = 1;
@@ -279,7 +317,7 @@ __device__ __forceinline__ T ghost_value(const T *__restrict__ x, const T *__res
         k += (dir[d] + 1) * m;
         m *= 3;
     }
-    const int e = box[blk * NB3 + k];
+    const int e = row[k];
     if (e >= 0) {
 #pragma unroll
         for (int d = 0; d < D; d++) c[d] -= dir[d] * M;
@@ -298,7 +336,7 @@ __device__ __forceinline__ T ghost_value(const T *__restrict__ x, const T *__res
         m *= 3;
     }
     T v;
-    const int e2 = box[blk * NB3 + k2];
+    const int e2 = row[k2];
     if (k2 == NB3 / 2) {
         v = x[(size_t)blk * LY::V + LY::sidx(c[0], c[1], c[2])];
     } else if (e2 >= 0) {
@@ -321,7 +359,7 @@ __device__ __forceinline__ void frame_copybnd_cell(T *__restrict__ g, const T *_
     int c[3], dir[3], k;
     if (!frame_cell<D, M>(q, c, dir, k)) return;
     if (box[blk * NB3 + k] < -8) return;  // coarse-fine: k_frame_interp
-    g[(size_t)blk * P + q] = ghost_value<D, M, T>(x, g, box, bc, blk, c);
+    g[(size_t)blk * P + q] = ghost_value<D, M, T>(x, g, box + blk * NB3, bc, blk, c);
 }
 
 // fill_ghost_copy! then fill_ghost_bnd! in one pass (ghost_value); one pass
@@ -359,7 +397,7 @@ struct LiveRead {
         if (c0 >= 0 && c0 < M && c1 >= 0 && c1 < M && (D == 2 || (c2 >= 0 && c2 < M)))
             return x[(size_t)blk * LY::V + LY::sidx(c0, c1, c2)];
         int c[3] = {c0, c1, D == 3 ? c2 : 0};
-        return ghost_value<D, M, T>(x, g, box, bc, blk, c);
+        return ghost_value<D, M, T>(x, g, box + blk * (D == 3 ? 27 : 9), bc, blk, c);
     }
 };
 
@@ -368,21 +406,9 @@ struct LiveRead {
 // under it with its axis neighbours (coarse ghosts from the coarse frame),
 // the offsets towards this block in the dimensions of the direction
 template <int D, int M, typename T>
-__global__ __launch_bounds__(WG) void k_frame_interp(T *__restrict__ g, const T *__restrict__ x,
-                                                     const int *__restrict__ box, const int2 *__restrict__ slots,
-                                                     int blk0, int nblk) {
+__device__ __forceinline__ T interp_value(const T *__restrict__ g, const T *__restrict__ x, const int2 sl, const int *c,
+                                          const int *dir) {
     using LY = Lay<D, M>;
-    constexpr int P = Frame<D, M>::P, NB3 = D == 3 ? 27 : 9;
-    // 64-bit: a level's nblk * P frame cells can pass 2^31 before its nblk * V cells do
-    const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t lb = gt / P;
-    if (lb >= nblk) return;
-    const int q = (int)(gt - lb * P), blk = blk0 + (int)lb;
-    int c[3], dir[3], k;
-    if (!frame_cell<D, M>(q, c, dir, k)) return;
-    const int e = box[blk * NB3 + k];
-    if (e > -16) return;
-    const int2 sl = slots[-16 - e];
     const int pb = sl.x, sb = sl.y;
     int J[3] = {0, 0, 0}, i[3] = {0, 0, 0};
 #pragma unroll
@@ -403,7 +429,54 @@ __global__ __launch_bounds__(WG) void k_frame_interp(T *__restrict__ g, const T 
         K[j] += 2 * i[j] - 1;
         f += w1<T>() * boxv<D, M, T>(x, g, pb, K[0], K[1], K[2]);
     }
+    return f;
+}
+
+// into g, and into g2 as well unless it is null
+template <int D, int M, typename T>
+__global__ __launch_bounds__(WG) void k_frame_interp(T *g, T *g2, const T *__restrict__ x,
+                                                     const int *__restrict__ box, const int2 *__restrict__ slots,
+                                                     int blk0, int nblk) {
+    constexpr int P = Frame<D, M>::P, NB3 = D == 3 ? 27 : 9;
+    // 64-bit: a level's nblk * P frame cells can pass 2^31 before its nblk * V cells do
+    const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t lb = gt / P;
+    if (lb >= nblk) return;
+    const int q = (int)(gt - lb * P), blk = blk0 + (int)lb;
+    int c[3], dir[3], k;
+    if (!frame_cell<D, M>(q, c, dir, k)) return;
+    const int e = box[blk * NB3 + k];
+    if (e > -16) return;
+    const T f = interp_value<D, M, T>(g, x, slots[-16 - e], c, dir);
     g[(size_t)blk * P + q] = f;
+    if (g2) g2[(size_t)blk * P + q] = f;
+}
+
+// fill_ghost!'s three steps for a 2D level in one launch, a wave pair a block:
+// every ghost is read before any is written, since a boundary ghost may mirror
+// a coarse-fine one of the same block as it was before the interpolation (no
+// other read of this level's frames; the coarse level's are not written here).
+// One launch of 3.6 us for k_frame_copybnd's 3.1 and k_frame_interp's 2.7.
+template <int M, typename T>
+__global__ __launch_bounds__(128) void k_frame_fill2(T *g, const T *__restrict__ x, const T *__restrict__ xc,
+                                                     const int *__restrict__ box, const int2 *__restrict__ slots,
+                                                     int blk0, Bc27<T> bc) {
+    constexpr int S = M + 2, P = Frame<2, M>::P;
+    static_assert(4 * (M + 1) <= 128, "a thread for each ghost");
+    const int blk = blk0 + blockIdx.x, i = threadIdx.x;
+    // the ring: the rows below and above, then the columns
+    const int q = i < S ? i : (i < 2 * S ? i + S * (S - 2) : S + (i - 2 * S) / 2 * S + ((i - 2 * S) & 1) * (S - 1));
+    const bool in = i < 4 * (M + 1);
+    T v = T(0);
+    if (in) {
+        int c[3], dir[3], k;
+        (void)frame_cell<2, M>(q, c, dir, k);
+        const int e = box[blk * 9 + k];
+        if (e <= -16) v = interp_value<2, M, T>(g, xc, slots[-16 - e], c, dir);
+        else v = ghost_value<2, M, T>(x, g, box + blk * 9, bc, blk, c);
+    }
+    __syncthreads();
+    if (in) g[(size_t)blk * P + q] = v;
 }
 
 // interp_add_level! (src/interp.jl:102-115) reading the coarse ghosts from
@@ -456,34 +529,41 @@ __device__ __forceinline__ T stencil4(const A &at, int blk, int c0, int c1, int 
 // 156-201) at 1-based global radial index i: the 3x3 literal's entries
 // (integer ratios rounded once), visited column-major, divided by 6; and its
 // diagelm
-template <int M, typename T, typename A>
-__device__ __forceinline__ T stencil4cyl(const A &at, int blk, int c0, int c1, int N, long long i) {
+template <typename T>
+struct Cyl4 {
+    T lo, hi, pm, pp, cc, dg;
+};
+template <typename T>
+__device__ __forceinline__ Cyl4<T> cyl4(long long i) {
     const long long q = 2 * i - 1;
-    const T lo = (T)(2 * (i - 1)) / (T)q, hi = (T)(2 * i) / (T)q;
-    const T pm = (T)(4 * (-2 + 9 * i - 16 * i * i + 8 * i * i * i)) / (T)(q * q * q);
-    const T pp = (T)(4 * (1 + i - 8 * i * i + 8 * i * i * i)) / (T)(q * q * q);
-    const T cc = (T)(-16 * (1 - 5 * i + 5 * i * i)) / (T)((1 - 2 * i) * (1 - 2 * i));
+    Cyl4<T> w;
+    w.lo = (T)(2 * (i - 1)) / (T)q;
+    w.hi = (T)(2 * i) / (T)q;
+    w.pm = (T)(4 * (-2 + 9 * i - 16 * i * i + 8 * i * i * i)) / (T)(q * q * q);
+    w.pp = (T)(4 * (1 + i - 8 * i * i + 8 * i * i * i)) / (T)(q * q * q);
+    w.cc = (T)(-16 * (1 - 5 * i + 5 * i * i)) / (T)((1 - 2 * i) * (1 - 2 * i));
+    w.dg = w.cc / T(6);
+    return w;
+}
+// at(a, b): the value at offset (a, b)
+template <typename T, typename A>
+__device__ __forceinline__ T stencil4cyl(const A &at, int N, const Cyl4<T> &l) {
     T w[3][3];
     if (N == 0) {
-        w[0][0] = lo; w[0][1] = pm; w[0][2] = lo;
-        w[1][0] = T(4); w[1][1] = cc; w[1][2] = T(4);
-        w[2][0] = hi; w[2][1] = pp; w[2][2] = hi;
+        w[0][0] = l.lo; w[0][1] = l.pm; w[0][2] = l.lo;
+        w[1][0] = T(4); w[1][1] = l.cc; w[1][2] = T(4);
+        w[2][0] = l.hi; w[2][1] = l.pp; w[2][2] = l.hi;
     } else {
-        w[0][0] = lo; w[0][1] = T(4); w[0][2] = hi;
-        w[1][0] = pm; w[1][1] = cc; w[1][2] = pp;
-        w[2][0] = lo; w[2][1] = T(4); w[2][2] = hi;
+        w[0][0] = l.lo; w[0][1] = T(4); w[0][2] = l.hi;
+        w[1][0] = l.pm; w[1][1] = l.cc; w[1][2] = l.pp;
+        w[2][0] = l.lo; w[2][1] = T(4); w[2][2] = l.hi;
     }
     T v = T(0);
 #pragma unroll
     for (int b = 0; b < 3; b++)
 #pragma unroll
-        for (int a = 0; a < 3; a++) v += w[a][b] * at(blk, c0 + a - 1, c1 + b - 1, 0);
+        for (int a = 0; a < 3; a++) v += w[a][b] * at(a - 1, b - 1);
     return v / T(6);
-}
-
-template <typename T>
-__device__ __forceinline__ T diag4cyl(long long i) {
-    return (T)(-16 * (1 - 5 * i + 5 * i * i)) / (T)((1 - 2 * i) * (1 - 2 * i)) / T(6);
 }
 
 // the order-4 operator at cell (c0, c1, c2) of blk: Cartesian (rd < 0) or
@@ -494,8 +574,9 @@ __device__ __forceinline__ T apply4a(const A &at, const int *__restrict__ coord,
     if constexpr (D == 2) {
         if (rd >= 0) {
             const long long i = (long long)(rd == 0 ? c0 : c1) + 1 + (long long)M * (coord[blk * D + rd] - 1);
-            diag = diag4cyl<T>(i);
-            return stencil4cyl<M, T>(at, blk, c0, c1, rd, i);
+            const Cyl4<T> w = cyl4<T>(i);
+            diag = w.dg;
+            return stencil4cyl<T>([&](int x, int y) { return at(blk, c0 + x, c1 + y, 0); }, rd, w);
         }
     }
     diag = D == 2 ? T(-20.0 / 6.0) : T(-4);
@@ -537,39 +618,212 @@ __global__ __launch_bounds__(WG) void k_defect4(float *__restrict__ be, const do
 // pass that follows a copy-then-boundary fill: the cells one pass reads across
 // a block face are of other colours, or, for a boundary mirror, the cell being
 // updated itself (read before its write), so none changes during the pass
-// colour cell q of block blk in the FourColors{P1,P2} pass
-template <int D, int M, typename T, bool LIVE>
-__device__ __forceinline__ void gs4_cell(T *__restrict__ u, const T *__restrict__ b, const T *__restrict__ g,
-                                         const int *__restrict__ coord, int rd, int blk, int q, T s, T omega, int P1,
-                                         int P2, const int *__restrict__ box, const Bc27<T> &bc) {
-    using LY = Lay<D, M>;
-    constexpr int H2 = M / 2;
-    const int i0 = q % H2, i1 = (q / H2) % H2, z = D == 3 ? q / (H2 * H2) : 0;
-    const int p1 = D == 3 ? (P1 + z + 3) & 1 : P1, p2 = D == 3 ? (P2 + z + 3) & 1 : P2;
-    const int x0 = 2 * i0 + p1, x1 = 2 * i1 + p2;
-    const size_t o = (size_t)blk * LY::V + LY::sidx(x0, x1, z);
-    T c, Lu;
-    if constexpr (LIVE)
-        Lu = apply4a<D, M, T>(LiveRead<D, M, T>{u, g, box, bc}, coord, blk, x0, x1, z, rd, c);
-    else
-        Lu = apply4a<D, M, T>(FrameRead<D, M, T>{u, g}, coord, blk, x0, x1, z, rd, c);
-    u[o] = u[o] - omega * (Lu + s * b[o]) / c;
-}
-
-template <int D, int M, typename T, bool LIVE>
+// (3D; k_gs4_sweep takes 2D levels: a 3D block's halo would be several times
+// the block)
+template <int M, typename T, bool LIVE>
 __global__ __launch_bounds__(WG) void k_gs4_pass(T *__restrict__ u, const T *__restrict__ b,
-                                                 const T *__restrict__ g, const int *__restrict__ coord, int rd,
-                                                 int blk0, int nblk, T s, T omega, int P1, int P2,
-                                                 const int *__restrict__ box, Bc27<T> bc) {
-    constexpr int H2 = M / 2, NCC = D == 3 ? H2 * H2 * M : H2 * H2;
+                                                 const T *__restrict__ g, int blk0, int nblk, T s, T omega, int P1,
+                                                 int P2, const int *__restrict__ box, Bc27<T> bc) {
+    using LY = Lay<3, M>;
+    constexpr int H2 = M / 2, NCC = H2 * H2 * M;
     const int gt = blockIdx.x * blockDim.x + threadIdx.x;
     const int lb = gt / NCC;
     if (lb >= nblk) return;
-    gs4_cell<D, M, T, LIVE>(u, b, g, coord, rd, blk0 + lb, gt - lb * NCC, s, omega, P1, P2, box, bc);
+    const int blk = blk0 + lb, q = gt - lb * NCC, z = q / (H2 * H2);
+    const int x0 = 2 * (q % H2) + ((P1 + z + 3) & 1), x1 = 2 * ((q / H2) % H2) + ((P2 + z + 3) & 1);
+    const size_t o = (size_t)blk * LY::V + LY::sidx(x0, x1, z);
+    T c, Lu;
+    if constexpr (LIVE)
+        Lu = apply4a<3, M, T>(LiveRead<3, M, T>{u, g, box, bc}, nullptr, blk, x0, x1, z, -1, c);
+    else
+        Lu = apply4a<3, M, T>(FrameRead<3, M, T>{u, g}, nullptr, blk, x0, x1, z, -1, c);
+    u[o] = u[o] - omega * (Lu + s * b[o]) / c;
 }
 
+// NS sweeps, with their four colour passes each, of a 2D level in one launch
+// and out of place: a work group takes a block with the cells around it that
+// its passes depend on (for a sweep one cell to the sides and three above and
+// below: the colours' order (0,0), (0,1), (1,0), (1,1) needs no more; for each
+// sweep before it two and four more), and runs the passes there, those of the
+// neighbours' cells too (325 cells for 256 with M = 16, 565 in the first of
+// two sweeps). In place and pass by pass a sweep of 24 blocks took four launches
+// of 4.4 us, all of it round trips: the box row, the cells, the divisions for
+// the radial weights (here one table for the block). Two
+// sweeps of 20 to 32 blocks take 12 to 13 us (one: 8.4; 1.2 us a pass, 60 FP64
+// instructions in a chain), where the eight passes took 35; of 1024 blocks 25 us
+// for 53.
+//
+// The tile holds the live ghosts: a boundary ghost is written again with its
+// mirror cell, a coarse-fine ghost does not change during a sweep (its value
+// depends on its place only, not on the block it is a ghost of). FRAME0: the
+// first pass reads the ghosts of every block from its frame as it was last
+// filled (LiveRead and FrameRead differ there if the level was not filled just
+// before, and where a boundary mirrors a coarse-fine ghost).
+template <int M>
+constexpr int GS4_THREADS = M == 16 ? 256 : 128;
+template <int M, typename T, int NS, bool FRAME0>
+__global__ __launch_bounds__(GS4_THREADS<M>) void k_gs4_sweep(T *__restrict__ out, const T *__restrict__ u,
+                                                              const T *__restrict__ b, const T *__restrict__ g,
+                                                              const int *__restrict__ coord, int rd, int blk0, T s,
+                                                              T omega, const int *__restrict__ box, Bc27<T> bc) {
+    using LY = Lay<2, M>;
+    constexpr int J = NS - 1, NT = GS4_THREADS<M>, P = Frame<2, M>::P, H2 = M / 2;
+    constexpr int X0 = -1 - 2 * J, Y0 = -3 - 4 * J, W = M - 2 * X0 + 1, H = M - 2 * Y0 + 1, NR = M - 2 * Y0 - 1;
+    constexpr int LW = M == 16 ? 32 : 16, RY = NT / LW, NI = (H + RY - 1) / RY;  // loads: RY rows at a time
+    constexpr int CW = LW / 2;                                                   // a pass: CW columns of cells
+    static_assert(H2 + 1 + 2 * J <= CW && (H2 + 3 + 4 * J) * CW <= NT, "a colour's cells are one for each thread");
+    static_assert(Y0 >= -M && W <= LW && NR <= NT, "a row, and the radial weights, are one for each thread");
+    // the iterate and b, the columns of one parity together: a pass reads
+    // cells two apart in x
+    constexpr int WH = (W + 1) / 2;
+    __shared__ T t[2 * WH * H], tb[2 * WH * H];
+    const auto at_ = [](int x, int y) { return ((y - Y0) * 2 + ((x - X0) & 1)) * WH + ((x - X0) >> 1); };
+    __shared__ Cyl4<T> wr[NR];
+    __shared__ int rows[9][9];  // the entries of box of the blocks around (4: this one)
+    const int tid = threadIdx.x, blk = blk0 + blockIdx.x;
+    if (tid < 9) rows[4][tid] = box[blk * 9 + tid];
+    const int rc = rd >= 0 ? coord[blk * 2 + rd] - 1 : 0;
+    __syncthreads();
+    for (int i = tid; i < 81; i += NT) {
+        const int n = i / 9, e = rows[4][n];
+        if (n != 4 && e >= 0) rows[n][i - 9 * n] = box[e * 9 + i - 9 * n];
+    }
+    const auto side = [](int c) { return c < 0 ? 0 : (c >= M ? 2 : 1); };
+    // the tile's cells in the blocks around
+    const int lx = tid % LW + X0, ly = tid / LW + Y0, sx = side(lx);
+    T v[NI], vb[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int y = ly + i * RY, sy = side(y), e = rows[4][sx + 3 * sy];
+        v[i] = vb[i] = T(0);
+        if (lx < X0 + W && y < Y0 + H && e >= 0) {
+            const size_t o = (size_t)e * LY::V + LY::sidx(lx - M * (sx - 1), y - M * (sy - 1), 0);
+            v[i] = u[o];
+            vb[i] = b[o];
+        }
+    }
+    // the cell of this thread in colour 0, as place in the tile: colour col's
+    // is at (col / 2, col) from it, a later sweep's at (2, 4)
+    const int px = 2 * (tid % CW) - 2 * J, py = 2 * (tid / CW) - 2 - 4 * J;
+    T f0[9];
+    if constexpr (FRAME0) {
+        const int x = px - M * (side(px) - 1), y = py - M * (side(py) - 1);
+        const bool edge = x == 0 || x == M - 1 || y == 0 || y == M - 1;
+        const int e = px <= M + 2 * J && py <= M + 2 + 4 * J ? rows[4][side(px) + 3 * side(py)] : -1;
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            f0[k] = T(0);
+            if (edge && e >= 0 && (side(x + k % 3 - 1) != 1 || side(y + k / 3 - 1) != 1))
+                f0[k] = g[(size_t)e * P + Frame<2, M>::at(x + k % 3 - 1, y + k / 3 - 1, 0)];
+        }
+    }
+    if (rd >= 0 && tid < NR) wr[tid] = cyl4<T>((long long)tid + Y0 + 2 + (long long)M * rc);
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+        if (lx < X0 + W && ly + i * RY < Y0 + H) {
+            t[at_(lx, ly + i * RY)] = v[i];
+            tb[at_(lx, ly + i * RY)] = vb[i];
+        }
+    __syncthreads();
+    // the ghosts among them: each is one of the block next to it in x, in y or
+    // in both (ghost_value, the cells taken from the tile)
+#pragma unroll 1
+    for (int i = 0; i < NI; i++) {
+        const int y = ly + i * RY, sy = side(y);
+        if (lx >= X0 + W || y >= Y0 + H || rows[4][sx + 3 * sy] >= 0) continue;
+        const int ax = lx == -1 || lx == M ? 1 : (lx == 0 ? 0 : (lx == M - 1 ? 2 : sx));
+        const int ay = y == -1 || y == M ? 1 : (y == 0 ? 0 : (y == M - 1 ? 2 : sy));
+        int n = ax + 3 * sy;
+        if (rows[4][n] < 0) n = sx + 3 * ay;
+        if (rows[4][n] < 0) n = ax + 3 * ay;
+        const int en = rows[4][n];
+        if (en < 0) continue;  // no pass reads it
+        const int x0 = M * (n % 3 - 1), y0 = M * (n / 3 - 1);
+        int c0 = lx - x0, c1 = y - y0, k = side(c0) + 3 * side(c1);
+        int bi = 4, e = rows[n][k];
+        if (e >= -8) {
+            const int mask = -1 - e;
+            if (mask & 1) {
+                bi += side(c0) - 1;
+                k += 1 - side(c0);
+                c0 = c0 < 0 ? 0 : M - 1;
+            }
+            if (mask & 2) {
+                bi += 3 * (side(c1) - 1);
+                k += 3 * (1 - side(c1));
+                c1 = c1 < 0 ? 0 : M - 1;
+            }
+            e = rows[n][k];
+        }
+        const T m = e >= 0 ? t[at_(c0 + x0, c1 + y0)] : g[(size_t)en * P + Frame<2, M>::at(c0, c1, 0)];
+        t[at_(lx, y)] = bi == 4 ? m : bc.v[bi] * m;
+    }
+    // the passes in which this thread has a cell, and the domain's faces
+    unsigned act = 0;
+#pragma unroll
+    for (int pass = 0; pass < 4 * NS; pass++) {
+        const int col = pass & 3, j = J - (pass >> 2);
+        const int x = px + 2 * (J - j) + (col >> 1), y = py + 4 * (J - j) + col;
+        const bool in = x <= M - (col >> 1) + 2 * j && y <= M + 2 - col + 4 * j;
+        if (in && rows[4][side(x) + 3 * side(y)] >= 0) act |= 1u << pass;
+    }
+    const auto outside = [&](int k) { return rows[4][k] < 0 && rows[4][k] >= -8; };
+    const bool out0 = outside(3), out1 = outside(5), out2 = outside(1), out3 = outside(7);
+    __syncthreads();
+    const auto run = [&](int pass, auto framed) {
+        const int x = px + 2 * (pass >> 2) + ((pass & 3) >> 1), y = py + pass;
+        if ((act >> pass) & 1) {
+            const int q = at_(x, y), qe = at_(x - 1, y), qo = at_(x + 1, y);
+            const auto at = [&](int a, int c) {
+                if constexpr (decltype(framed)::value) {
+                    const int xa = x - M * (side(x) - 1) + a, yc = y - M * (side(y) - 1) + c;
+                    if (side(xa) != 1 || side(yc) != 1) return f0[a + 1 + 3 * (c + 1)];
+                }
+                return t[(a < 0 ? qe : (a > 0 ? qo : q)) + c * 2 * WH];
+            };
+            T d, Lu;
+            if (rd >= 0) {
+                const Cyl4<T> &w = wr[(rd == 0 ? x : y) - Y0 - 1];
+                d = w.dg;
+                Lu = stencil4cyl<T>(at, rd, w);
+            } else {
+                d = T(-20.0 / 6.0);
+                Lu = stencil4<2, M, T>([&](int, int a, int c, int) { return at(a, c); }, 0, 0, 0, 0);
+            }
+            const T nv = t[q] - omega * (Lu + s * tb[q]) / d;
+            t[q] = nv;
+            // its boundary ghosts
+            const int gx = x == 0 && out0 ? -1 : (x == M - 1 && out1 ? 1 : 0);
+            const int gy = y == 0 && out2 ? -1 : (y == M - 1 && out3 ? 1 : 0);
+            if (gx) t[at_(x + gx, y)] = bc.v[gx + 4] * nv;
+            if (gy) t[at_(x, y + gy)] = bc.v[3 * gy + 4] * nv;
+            if (gx && gy) t[at_(x + gx, y + gy)] = bc.v[3 * gy + gx + 4] * nv;
+        }
+        __syncthreads();
+    };
+    if constexpr (FRAME0) run(0, std::true_type{});
+#pragma unroll 1
+    for (int pass = FRAME0 ? 1 : 0; pass < 4 * NS; pass++) run(pass, std::false_type{});
+    for (int i = tid; i < LY::V; i += NT) {
+        int c0, c1, c2;
+        LY::decode(i, c0, c1, c2);
+        out[(size_t)blk * LY::V + i] = t[at_(c0, c1)];
+    }
+}
 
 // residual! (src/multigrid.jl:309-323) with the order-4 operator
+template <int D, int M, typename T>
+__device__ __forceinline__ void resid4_cell(T *__restrict__ r, const T *__restrict__ u, const T *__restrict__ b,
+                                            const T *__restrict__ g, const int *__restrict__ coord, int rd, int blk,
+                                            int q, T s) {
+    using LY = Lay<D, M>;
+    int c0, c1, c2;
+    LY::decode(q, c0, c1, c2);
+    const size_t o = (size_t)blk * LY::V + q;
+    T c;
+    const T Lu = apply4<D, M, T>(u, g, coord, blk, c0, c1, c2, rd, c);
+    r[o] = -(b[o] + Lu / s);
+}
 template <int D, int M, typename T>
 __global__ __launch_bounds__(WG) void k_resid4(T *__restrict__ r, const T *__restrict__ u, const T *__restrict__ b,
                                                const T *__restrict__ g, const int *__restrict__ coord, int rd,
@@ -578,37 +832,92 @@ __global__ __launch_bounds__(WG) void k_resid4(T *__restrict__ r, const T *__res
     const int gt = blockIdx.x * blockDim.x + threadIdx.x;
     const int lb = gt / LY::V;
     if (lb >= nblk) return;
-    const int blk = blk0 + lb, q = gt - lb * LY::V;
-    int c0, c1, c2;
-    LY::decode(q, c0, c1, c2);
-    const size_t o = (size_t)blk * LY::V + q;
-    T c;
-    const T Lu = apply4<D, M, T>(u, g, coord, blk, c0, c1, c2, rd, c);
-    r[o] = -(b[o] + Lu / s);
+    resid4_cell<D, M, T>(r, u, b, g, coord, rd, blk0 + lb, gt - lb * LY::V, s);
 }
 
-// residual_postrestrict_level! (src/multigrid.jl:112-119, 331-344) with the
-// order-4 operator on the coarse cells covered by the fine blocks
+// The steps of an order-4 cycle around its sweeps that do not wait for each
+// other share a launch, each with its own work groups: on small levels a step
+// is one round trip of 2 to 4 us, whatever it does (a cycle on three levels of
+// 20 to 32 blocks: 17 launches between its sweeps instead of 38).
+//
+// After the sweeps down: refill the copy and boundary ghosts of the level
+// (nframe work groups), restrict it.
+template <int D, int M, typename T>
+__global__ __launch_bounds__(WG) void k4_refill_restrict(T *__restrict__ g, T *__restrict__ xc, const T *__restrict__ x,
+                                                         const int *__restrict__ box, const int *__restrict__ parent,
+                                                         const int *__restrict__ sub, int blk0, int nblk, Bc27<T> bc,
+                                                         unsigned nframe) {
+    using LY = Lay<D, M>;
+    constexpr int P = Frame<D, M>::P;
+    if (blockIdx.x < nframe) {
+        const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, lb = gt / P;
+        if (lb < nblk) frame_copybnd_cell<D, M, T>(g, x, box, blk0 + (int)lb, (int)(gt - lb * P), bc);
+        return;
+    }
+    restrict_cell<D, M, T>(xc, x, parent, sub, blk0, nblk, (int)((blockIdx.x - nframe) * blockDim.x + threadIdx.x));
+}
+// Then: the level's residual (nres work groups), the copy and boundary ghosts
+// of the coarse level (nframe), and its values kept in u1.
+template <int D, int M, typename T>
+__global__ __launch_bounds__(WG) void k4_resid_coarse(T *__restrict__ r, const T *__restrict__ u,
+                                                      const T *__restrict__ b, const T *g,
+                                                      const int *__restrict__ coord, int rd, int blk0, int nblk, T s,
+                                                      T *gw, T *__restrict__ u1, const T *__restrict__ uc,
+                                                      const int *__restrict__ box, int cblk0, int ncoarse, Bc27<T> bc,
+                                                      unsigned nres, unsigned nframe) {
+    using LY = Lay<D, M>;
+    constexpr int P = Frame<D, M>::P;
+    if (blockIdx.x < nres) {
+        const int gt = blockIdx.x * blockDim.x + threadIdx.x, lb = gt / LY::V;
+        if (lb < nblk) resid4_cell<D, M, T>(r, u, b, g, coord, rd, blk0 + lb, gt - lb * LY::V, s);
+    } else if (blockIdx.x < nres + nframe) {
+        const int64_t gt = (int64_t)(blockIdx.x - nres) * blockDim.x + threadIdx.x, lb = gt / P;
+        if (lb < ncoarse) frame_copybnd_cell<D, M, T>(gw, uc, box, cblk0 + (int)lb, (int)(gt - lb * P), bc);
+    } else {
+        const size_t i = (size_t)(blockIdx.x - nres - nframe) * blockDim.x + threadIdx.x;
+        if (i < (size_t)ncoarse * LY::V) u1[(size_t)cblk0 * LY::V + i] = uc[(size_t)cblk0 * LY::V + i];
+    }
+}
+// Before the correction: u1 = u - u1 on the coarse level's cells (nval work
+// groups) and, with coarse-fine ghosts on it, ghosts (ndiff), and the copy and
+// boundary ghosts of u's top level after its sweeps.
+template <int D, int M, typename T>
+__global__ __launch_bounds__(WG) void k4_diff(T *__restrict__ u1, const T *__restrict__ u, T *__restrict__ g1, T *g,
+                                              const int *__restrict__ box, int blk0, int nblk, Bc27<T> bc,
+                                              unsigned nval, unsigned ndiff) {
+    using LY = Lay<D, M>;
+    constexpr int P = Frame<D, M>::P;
+    if (blockIdx.x < nval) {
+        const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, o = (size_t)blk0 * LY::V + i;
+        if (i < (size_t)nblk * LY::V) u1[o] = u[o] - u1[o];
+    } else if (blockIdx.x < nval + ndiff) {
+        const size_t i = (size_t)(blockIdx.x - nval) * blockDim.x + threadIdx.x, o = (size_t)blk0 * P + i;
+        if (i < (size_t)nblk * P) g1[o] = g[o] - g1[o];
+    } else {
+        const int64_t gt = (int64_t)(blockIdx.x - nval - ndiff) * blockDim.x + threadIdx.x, lb = gt / P;
+        if (lb < nblk) frame_copybnd_cell<D, M, T>(g, u, box, blk0 + (int)lb, (int)(gt - lb * P), bc);
+    }
+}
+
+// restrict! of the residual, and residual_postrestrict_level!
+// (src/multigrid.jl:112-119, 331-344) with the order-4 operator on the coarse
+// cells covered by the fine blocks
 template <int D, int M, typename T>
 __global__ __launch_bounds__(WG) void k_postrestrict4(T *__restrict__ bout, const T *__restrict__ u,
-                                                      const T *__restrict__ r, const T *__restrict__ g,
-                                                      const int *__restrict__ coord, int rd,
+                                                      T *__restrict__ rc, const T *__restrict__ r,
+                                                      const T *__restrict__ g, const int *__restrict__ coord, int rd,
                                                       const int *__restrict__ parent, const int *__restrict__ sub,
                                                       int fblk0, int nfine, T s) {
     using LY = Lay<D, M>;
-    constexpr int NS = LY::V / LY::NC;
-    const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lb = gt / NS;
-    if (lb >= nfine) return;
-    const int fb = fblk0 + lb, j = gt - lb * NS;
-    const int j0 = j % LY::MH, j1 = (j / LY::MH) % LY::MH, j2 = (D == 3) ? j / (LY::MH * LY::MH) : 0;
-    const int pb = parent[fb], sb = sub[fb];
-    const int X0 = (sb & 1) * LY::MH + j0, X1 = ((sb >> 1) & 1) * LY::MH + j1;
-    const int X2 = (D == 3) ? ((sb >> 2) & 1) * LY::MH + j2 : 0;
-    const size_t o = (size_t)pb * LY::V + LY::sidx(X0, X1, X2);
+    size_t o;
+    int pb, X0, X1, X2;
+    T f;
+    if (!restricted<D, M, T>(r, parent, sub, fblk0, nfine, blockIdx.x * blockDim.x + threadIdx.x, o, pb, X0, X1, X2, f))
+        return;
+    rc[o] = f;
     T c;
     const T Lu = apply4<D, M, T>(u, g, coord, pb, X0, X1, X2, rd, c);
-    bout[o] = -(r[o] + Lu / s);
+    bout[o] = -(f + Lu / s);
 }
 
 // rhs! (src/multigrid.jl:363-388) of the compact 4th-order Laplacian
@@ -636,32 +945,12 @@ __global__ __launch_bounds__(WG) void k_rhs4(T *__restrict__ b1, const T *__rest
     b1[o] = v / T(12);
 }
 
-// restrict! over the Child edges of a level (src/restrict.jl:5-37): each
-// coarse cell of the parent subblock = mean of its 2^D children, summed with
-// the first index fastest. xf holds the fine level, xc the coarse one.
+// restrict! over the Child edges of a level
 template <int D, int M, typename T>
 __global__ __launch_bounds__(WG) void k_restrict(T *__restrict__ xc, const T *__restrict__ xf,
                                                  const int *__restrict__ parent, const int *__restrict__ sub,
                                                  int blk0, int nblk) {
-    using LY = Lay<D, M>;
-    constexpr int NS = LY::V / LY::NC;  // coarse cells per subblock
-    int gt = blockIdx.x * blockDim.x + threadIdx.x;
-    int lb = gt / NS;
-    if (lb >= nblk) return;
-    int fb = blk0 + lb;
-    int j = gt - lb * NS;
-    int j0 = j % LY::MH, j1 = (j / LY::MH) % LY::MH, j2 = (D == 3) ? j / (LY::MH * LY::MH) : 0;
-    T f = T(0);
-#pragma unroll
-    for (int q = 0; q < LY::NC; q++) {
-        int i0 = q & 1, i1 = (q >> 1) & 1, i2 = (q >> 2) & 1;
-        f += xf[(size_t)fb * LY::V + LY::sidx(2 * j0 + i0, 2 * j1 + i1, D == 3 ? 2 * j2 + i2 : 0)];
-    }
-    int pb = parent[fb];
-    int sb = sub[fb];
-    int X0 = (sb & 1) * LY::MH + j0, X1 = ((sb >> 1) & 1) * LY::MH + j1;
-    int X2 = (D == 3) ? ((sb >> 2) & 1) * LY::MH + j2 : 0;
-    xc[(size_t)pb * LY::V + LY::sidx(X0, X1, X2)] = f / T(LY::NC);
+    restrict_cell<D, M, T>(xc, xf, parent, sub, blk0, nblk, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // residual_postrestrict_level! (src/multigrid.jl:112-119, 331-344): FAS
@@ -698,13 +987,6 @@ template <typename T>
 __global__ __launch_bounds__(WG) void k_copy(T *__restrict__ dst, const T *__restrict__ src, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
-}
-
-template <typename T>
-__global__ __launch_bounds__(WG) void k_diff(T *__restrict__ dst, const T *__restrict__ a,
-                                             const T *__restrict__ b, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = a[i] - b[i];
 }
 
 // storage position of local cell (x, y, z) and its inverse, as Lay<D, M>, for
@@ -971,7 +1253,7 @@ template <> struct Vec16<float> { using V = float4; };
 template <> struct Vec16<double> { using V = double2; };
 
 // Two independent steps of the V-cycle ascent in one launch: the first
-// nwg_diff work groups form dst = a1 - a2 over n values (k_diff; 16 bytes
+// nwg_diff work groups form dst = a1 - a2 over n values (16 bytes
 // per lane, n a multiple of 16 / sizeof(T), the arrays 16-byte aligned; dst
 // may be a2), the rest refresh nslot coarse-fine ghost slabs
 // (k_fill_interp). The slabs read another level than the difference writes.

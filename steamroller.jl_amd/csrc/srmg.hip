@@ -219,6 +219,7 @@ struct srmg_ctx {
     // the order-4 operator's box neighbour table and coarse-fine slots (built
     // on first use; see box_table)
     DevBuf d_box, d_box_slots;
+    std::vector<uint8_t> box_cf;  // per level: some direction of a block is coarse-fine (with box_ok)
     bool box_ok = false;  // bumped when coarse-solve matrices are rebuilt (older graphs point to freed ones)
 };
 
@@ -1009,6 +1010,10 @@ struct Ops {
         fail("cylindrical geometry is two-dimensional");
     }
 
+    // the second buffer of ping-pong sweeps
+    void need_alt(FieldBuf &u) {
+        if (!u.alt.p || u.alt.bytes != u.data.bytes) u.alt.alloc(u.data.bytes);
+    }
     // bring every level back to the primary buffer
     void settle(FieldBuf &f) {
         for (int l = 0; l < c->nlevels; l++) {
@@ -1112,7 +1117,7 @@ struct Ops {
     // zin: u and its ghost slabs are zero on level l (only with zin_ok(l))
     void sweep(FieldBuf &u, FieldBuf &b, const LevelArgs<T> &a, int l, int cfg = -1, bool zin = false) {
         if (!a.nblk) return;
-        if (!u.alt.p || u.alt.bytes != u.data.bytes) u.alt.alloc(u.data.bytes);
+        need_alt(u);
         T *in = X(u, l);
         T *out = u.cur[l] ? u.data.as<T>() : u.alt.as<T>();
         cfg = sweep_shape(l, cfg);
@@ -1262,46 +1267,112 @@ struct Ops {
         const LevelInfo &L = c->lv[l];
         if (!L.nblk) return;
         T *g = frame(x);
-        const unsigned grid = nwg((int64_t)L.nblk * FP);
-        hipLaunchKernelGGL((k_frame_copybnd<D, M, T>), dim3(grid), dim3(WG), 0, c->stream, g, X(x, l),
-                           c->d_box.as<int>(), L.blk0, L.nblk, bc);
-        if (interp && l > 0)
-            hipLaunchKernelGGL((k_frame_interp<D, M, T>), dim3(grid), dim3(WG), 0, c->stream, g, X(x, l - 1),
-                               c->d_box.as<int>(), c->d_box_slots.as<int2>(), L.blk0, L.nblk);
+        interp = interp && c->box_cf[l];
+        if constexpr (D == 2) {
+            if (interp) {
+                hipLaunchKernelGGL((k_frame_fill2<M, T>), dim3((unsigned)L.nblk), dim3(128), 0, c->stream, g, X(x, l),
+                                   X(x, l - 1), c->d_box.as<int>(), c->d_box_slots.as<int2>(), L.blk0, bc);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_frame_copybnd<D, M, T>), dim3(nwg((int64_t)L.nblk * FP)), dim3(WG), 0, c->stream, g,
+                           X(x, l), c->d_box.as<int>(), L.blk0, L.nblk, bc);
+        if (interp) frame_interp(x, nullptr, l);
     }
-    // copyto! / diffto! include the ghosts (src/blockfield.jl:557-576)
+    void frame_interp(FieldBuf &x, FieldBuf *x2, int l) {
+        const LevelInfo &L = c->lv[l];
+        if (!L.nblk || !c->box_cf[l]) return;
+        hipLaunchKernelGGL((k_frame_interp<D, M, T>), dim3(nwg((int64_t)L.nblk * FP)), dim3(WG), 0, c->stream, frame(x),
+                           x2 ? frame(*x2) : nullptr, X(x, l - 1), c->d_box.as<int>(), c->d_box_slots.as<int2>(),
+                           L.blk0, L.nblk);
+    }
+    // copyto! includes the ghosts (src/blockfield.jl:557-576)
     void frame_copy(FieldBuf &dst, FieldBuf &src, int l) {
         const LevelInfo &L = c->lv[l];
         const size_t n = (size_t)L.nblk * FP, o = (size_t)L.blk0 * FP;
-        if (n) hipLaunchKernelGGL((k_copy<T>), dim3(nwg(n)), dim3(WG), 0, c->stream, frame(dst) + o, frame(src) + o, n);
-    }
-    void frame_diff(FieldBuf &dst, FieldBuf &a1, FieldBuf &a2, int l) {
-        const LevelInfo &L = c->lv[l];
-        const size_t n = (size_t)L.nblk * FP, o = (size_t)L.blk0 * FP;
         if (n)
-            hipLaunchKernelGGL((k_diff<T>), dim3(nwg(n)), dim3(WG), 0, c->stream, frame(dst) + o, frame(a1) + o,
-                               frame(a2) + o, n);
+            hipLaunchKernelGGL((k_copy<T>), dim3(nwg(n)), dim3(WG), 0, c->stream, frame(dst) + o, frame(src) + o, n);
     }
-    void gs4_iter(FieldBuf &u, FieldBuf &b, double sl, double omega, int n, int l, const Bc27<T> &bc) {
+    // u1 = u - u1 on level l, with the ghosts (diffto!); refill: the copy and
+    // boundary ghosts of u too
+    void diff4(FieldBuf &u1, FieldBuf &u, int l, const Bc27<T> &bc, bool refill) {
         const LevelInfo &L = c->lv[l];
         if (!L.nblk) return;
-        constexpr int NCC = D == 3 ? (M / 2) * (M / 2) * M : (M / 2) * (M / 2);
-        // the reference refills the copy and boundary ghosts after every
-        // colour pass; the passes after the first read those values live
-        // (k_gs4_pass<LIVE>), so only the last refill is made
-        for (int it = 0; it < n; it++)
-            for (int col = 0; col < 4; col++) {
-                const dim3 grid(nwg((int64_t)L.nblk * NCC));
-                if (it == 0 && col == 0)
-                    hipLaunchKernelGGL((k_gs4_pass<D, M, T, false>), grid, dim3(WG), 0, c->stream, X(u, l), X(b, l),
-                                       frame(u), coord(), rd4, L.blk0, L.nblk, (T)sl, (T)omega, col >> 1, col & 1,
-                                       c->d_box.as<int>(), bc);
-                else
-                    hipLaunchKernelGGL((k_gs4_pass<D, M, T, true>), grid, dim3(WG), 0, c->stream, X(u, l), X(b, l),
-                                       frame(u), coord(), rd4, L.blk0, L.nblk, (T)sl, (T)omega, col >> 1, col & 1,
-                                       c->d_box.as<int>(), bc);
+        const unsigned nval = nwg((int64_t)L.nblk * LY::V), nfr = nwg((int64_t)L.nblk * FP);
+        const unsigned ndiff = c->box_cf[l] ? nfr : 0, nref = refill ? nfr : 0;
+        hipLaunchKernelGGL((k4_diff<D, M, T>), dim3(nval + ndiff + nref), dim3(WG), 0, c->stream, X(u1, l), X(u, l),
+                           frame(u1), frame(u), c->d_box.as<int>(), L.blk0, L.nblk, bc, nval, ndiff);
+    }
+    // sweeps of level l. The reference refills the copy and boundary ghosts
+    // after every colour pass; the passes after the first read those values
+    // live, and the last refill is the caller's. fresh: the frames were filled
+    // just before
+    void gs4_iter(FieldBuf &u, FieldBuf &b, double sl, double omega, int n, int l, const Bc27<T> &bc, bool fresh) {
+        const LevelInfo &L = c->lv[l];
+        if (!L.nblk) return;
+        if constexpr (D == 2) {
+            need_alt(u);
+            for (int it = 0; it < n;) {
+                T *in = X(u, l);
+                T *out = u.cur[l] ? u.data.as<T>() : u.alt.as<T>();
+                const auto go = [&](auto k) {
+                    hipLaunchKernelGGL(k, dim3((unsigned)L.nblk), dim3(GS4_THREADS<M>), 0, c->stream, out, in, X(b, l),
+                                       frame(u), coord(), rd4, L.blk0, (T)sl, (T)omega, c->d_box.as<int>(), bc);
+                };
+                const bool frame0 = it == 0 && !(fresh && !c->box_cf[l]);
+                if (n - it >= 2) {
+                    if (frame0) go(k_gs4_sweep<M, T, 2, true>);
+                    else go(k_gs4_sweep<M, T, 2, false>);
+                    it += 2;
+                } else {
+                    if (frame0) go(k_gs4_sweep<M, T, 1, true>);
+                    else go(k_gs4_sweep<M, T, 1, false>);
+                    it++;
+                }
+                u.cur[l] ^= 1;
             }
-        if (n > 0) frame_fill(u, l, bc, false);
+        } else {
+            constexpr int NCC = (M / 2) * (M / 2) * M;
+            const dim3 grid(nwg((int64_t)L.nblk * NCC));
+            for (int it = 0; it < n; it++)
+                for (int col = 0; col < 4; col++) {
+                    const auto go = [&](auto k) {
+                        hipLaunchKernelGGL(k, grid, dim3(WG), 0, c->stream, X(u, l), X(b, l), frame(u), L.blk0, L.nblk,
+                                           (T)sl, (T)omega, col >> 1, col & 1, c->d_box.as<int>(), bc);
+                    };
+                    if (it == 0 && col == 0) go(k_gs4_pass<M, T, false>);
+                    else go(k_gs4_pass<M, T, true>);
+                }
+        }
+    }
+    // the way down from level l >= 1 after its sweeps: u restricted, kept in u1
+    // (unless keep is off), its ghosts filled on the coarse level, the residual
+    // restricted, the coarse right-hand side
+    void down4(FieldBuf &u, FieldBuf &b, FieldBuf &r, FieldBuf *u1, int l, double sl, const Bc27<T> &bc, bool refill) {
+        const LevelInfo &L = c->lv[l], &C = c->lv[l - 1];
+        const int *parent = c->d_parent.as<int>(), *sub = c->d_sub.as<int>(), *box = c->d_box.as<int>();
+        const unsigned nsub = nwg((int64_t)L.nblk * (LY::V / LY::NC)), nfr = refill ? nwg((int64_t)L.nblk * FP) : 0;
+        if (L.nblk)
+            hipLaunchKernelGGL((k4_refill_restrict<D, M, T>), dim3(nfr + nsub), dim3(WG), 0, c->stream, frame(u),
+                               X(u, l - 1), X(u, l), box, parent, sub, L.blk0, L.nblk, bc, nfr);
+        const unsigned nres = L.nblk ? nwg((int64_t)L.nblk * LY::V) : 0, ncf = C.nblk ? nwg((int64_t)C.nblk * FP) : 0;
+        const unsigned nk = C.nblk && u1 ? nwg((int64_t)C.nblk * LY::V) : 0;
+        if (nres + ncf + nk)
+            hipLaunchKernelGGL((k4_resid_coarse<D, M, T>), dim3(nres + ncf + nk), dim3(WG), 0, c->stream, X(r, l),
+                               X(u, l), X(b, l), frame(u), coord(), rd4, L.blk0, L.nblk, (T)sl, frame(u),
+                               u1 ? X(*u1, l - 1) : nullptr, X(u, l - 1), box, C.blk0, C.nblk, bc, nres, ncf);
+        frame_interp(u, u1, l - 1);
+        if (L.nblk)
+            hipLaunchKernelGGL((k_postrestrict4<D, M, T>), dim3(nsub), dim3(WG), 0, c->stream, X(b, l - 1),
+                               X(u, l - 1), X(r, l - 1), X(r, l), frame(u), coord(), rd4, parent, sub, L.blk0, L.nblk,
+                               (T)(4 * sl));
+    }
+    void interp_add4(FieldBuf &u, FieldBuf &u1, int l) {
+        const LevelInfo &L = c->lv[l];
+        if (L.nblk)
+            hipLaunchKernelGGL((k_interp_add4<D, M, T>), dim3(nwg((int64_t)L.nblk * LY::V)), dim3(WG), 0, c->stream,
+                               X(u, l), X(u1, l - 1), frame(u1), c->d_parent.as<int>(), c->d_sub.as<int>(), L.blk0,
+                               L.nblk);
     }
     void vcycle4(FieldBuf &u, FieldBuf &b, FieldBuf &r, FieldBuf &u1, double s, const srmg_op *op, int lmax,
                  int ndown, int ntop, int nup, double omega) {
@@ -1312,37 +1383,21 @@ struct Ops {
         for (FieldBuf *f : {&u, &b, &r, &u1}) settle(*f);
         for (int l = lmax - 1; l >= 1; l--) {
             const double sl = s / (double)((int64_t)1 << (2 * l));
-            const LevelInfo &L = c->lv[l];
-            gs4_iter(u, b, sl, omega, ndown, l, bc);
-            restrict_(u, l);
-            frame_fill(u, l - 1, bc);
-            copy(u1, u, l - 1);
-            frame_copy(u1, u, l - 1);
-            if (L.nblk)
-                hipLaunchKernelGGL((k_resid4<D, M, T>), dim3(nwg((int64_t)L.nblk * LY::V)), dim3(WG), 0, c->stream,
-                                   X(r, l), X(u, l), X(b, l), frame(u), coord(), rd4, L.blk0, L.nblk, (T)sl);
-            restrict_(r, l);
-            if (L.nblk)
-                hipLaunchKernelGGL((k_postrestrict4<D, M, T>), dim3(nwg((int64_t)L.nblk * (LY::V / LY::NC))),
-                                   dim3(WG), 0, c->stream, X(b, l - 1), X(u, l - 1), X(r, l - 1), frame(u),
-                                   coord(), rd4, c->d_parent.as<int>(), c->d_sub.as<int>(), L.blk0, L.nblk,
-                                   (T)(4 * sl));
+            gs4_iter(u, b, sl, omega, ndown, l, bc, l < lmax - 1);
+            down4(u, b, r, &u1, l, sl, bc, ndown > 0);
         }
-        gs4_iter(u, b, s, omega, ntop, 0, bc);
+        gs4_iter(u, b, s, omega, ntop, 0, bc, lmax > 1);
+        if (lmax == 1 && ntop > 0) frame_fill(u, 0, bc, false);
         for (int l = 1; l < lmax; l++) {
             const double sl = s / (double)((int64_t)1 << (2 * l));
-            const LevelInfo &L = c->lv[l];
-            diff(u1, u, u1, l - 1);
-            frame_diff(u1, u, u1, l - 1);
+            diff4(u1, u, l - 1, bc, l == 1 && ntop > 0);
             frame_fill(u1, l - 1, bc);
-            if (L.nblk)
-                hipLaunchKernelGGL((k_interp_add4<D, M, T>), dim3(nwg((int64_t)L.nblk * LY::V)), dim3(WG), 0,
-                                   c->stream, X(u, l), X(u1, l - 1), frame(u1), c->d_parent.as<int>(),
-                                   c->d_sub.as<int>(), L.blk0, L.nblk);
+            interp_add4(u, u1, l);
             frame_fill(u, l, bc);
-            gs4_iter(u, b, sl, omega, nup, l, bc);
+            gs4_iter(u, b, sl, omega, nup, l, bc, true);
             frame_fill(u, l, bc);
         }
+        settle(u);
     }
     // fmg! (src/multigrid.jl:17-51) with the order-4 operator
     void fmg4(FieldBuf &u, FieldBuf &b, FieldBuf &r, FieldBuf &u1, double s, const srmg_op *op, int ndown, int ntop,
@@ -1356,31 +1411,15 @@ struct Ops {
         for (FieldBuf *f : {&u, &b, &r, &u1}) settle(*f);
         for (int l = lmax - 1; l >= 1; l--) {
             const double sl = s / (double)((int64_t)1 << (2 * l));
-            const LevelInfo &L = c->lv[l];
-            restrict_(u, l);
-            frame_fill(u, l - 1, bc);
-            if (L.nblk)
-                hipLaunchKernelGGL((k_resid4<D, M, T>), dim3(nwg((int64_t)L.nblk * LY::V)), dim3(WG), 0, c->stream,
-                                   X(r, l), X(u, l), X(b, l), frame(u), coord(), rd4, L.blk0, L.nblk, (T)sl);
-            restrict_(r, l);
-            if (L.nblk)
-                hipLaunchKernelGGL((k_postrestrict4<D, M, T>), dim3(nwg((int64_t)L.nblk * (LY::V / LY::NC))),
-                                   dim3(WG), 0, c->stream, X(b, l - 1), X(u, l - 1), X(r, l - 1), frame(u),
-                                   coord(), rd4, c->d_parent.as<int>(), c->d_sub.as<int>(), L.blk0, L.nblk,
-                                   (T)(4 * sl));
+            down4(u, b, r, nullptr, l, sl, bc, false);
         }
         for (int l = 0; l < lmax; l++) {
             copy(u1, u, l);
             frame_copy(u1, u, l);
             if (l > 0) {
-                const LevelInfo &L = c->lv[l];
-                diff(u1, u, u1, l - 1);
-                frame_diff(u1, u, u1, l - 1);
+                diff4(u1, u, l - 1, bc, false);
                 frame_fill(u1, l - 1, bc);
-                if (L.nblk)
-                    hipLaunchKernelGGL((k_interp_add4<D, M, T>), dim3(nwg((int64_t)L.nblk * LY::V)), dim3(WG), 0,
-                                       c->stream, X(u, l), X(u1, l - 1), frame(u1), c->d_parent.as<int>(),
-                                       c->d_sub.as<int>(), L.blk0, L.nblk);
+                interp_add4(u, u1, l);
             }
             frame_fill(u, l, bc);
             vcycle4(u, b, r, u1, s, op, l + 1, ndown, ntop, nup, omega);
@@ -1424,14 +1463,6 @@ struct Ops {
         size_t o = (size_t)L.blk0 * LY::V;
         hipLaunchKernelGGL((k_copy<T>), dim3(nwg(n)), dim3(WG), 0, c->stream, X(dst, l) + o, X(src, l) + o, n);
     }
-    void diff(FieldBuf &dst, FieldBuf &a1, FieldBuf &a2, int l) {
-        const LevelInfo &L = c->lv[l];
-        size_t n = (size_t)L.nblk * LY::V;
-        if (!n) return;
-        size_t o = (size_t)L.blk0 * LY::V;
-        hipLaunchKernelGGL((k_diff<T>), dim3(nwg(n)), dim3(WG), 0, c->stream, X(dst, l) + o, X(a1, l) + o,
-                           X(a2, l) + o, n);
-    }
     void interp_add(FieldBuf &u, FieldBuf &u1, int l, const LevelArgs<T> &ac) {
         const LevelInfo &L = c->lv[l];
         if (!L.nblk) return;
@@ -1447,7 +1478,7 @@ struct Ops {
                            X(u, l), X(u1, l - 1), I(u1), nbr(), c->d_parent.as<int>(), c->d_sub.as<int>(), L.blk0,
                            L.nblk, ac);
     }
-    // diff(u1, u, u1, l) and, when acf is given, fill_interp(u1, l, *acf) in
+    // u1 = u - u1 on level l and, when acf is given, fill_interp(u1, l, *acf) in
     // one launch (the slab fill reads level l-1, the difference writes level l)
     void diff_fill(FieldBuf &u1, FieldBuf &u, int l, const LevelArgs<T> *acf) {
         const LevelInfo &L = c->lv[l];
@@ -3147,6 +3178,7 @@ static void box_table(srmg_ctx *c) {
     }
     std::vector<int> box((size_t)c->nb * NB3, 0);
     std::vector<int2> slots;
+    c->box_cf.assign(c->nlevels, 0);
     for (int bk = 0; bk < c->nb; bk++) {
         const int l = c->h_level[bk];
         for (int k = 0; k < NB3; k++) {
@@ -3177,6 +3209,7 @@ static void box_table(srmg_ctx *c) {
             if (l == 0 || ip == at[l - 1].end()) fail("proper nesting broken for the box stencil");
             e = -16 - (int)slots.size();
             slots.push_back(make_int2(ip->second, sb));
+            c->box_cf[l] = 1;
         }
     }
     c->d_box.alloc(box.size() * sizeof(int));
@@ -3208,6 +3241,7 @@ static void do_vcycle4(srmg_ctx *c, int u, int b, int r, int u1, double s, const
         for (FieldBuf *f : {&fu, &fb, &fr, &fu1}) o.settle(*f);
         o.frame(fu);
         o.frame(fu1);
+        if (c->D == 2) o.need_alt(fu);
     });
     std::string k = "order4";
     auto add = [&](const auto &v) { k.append(reinterpret_cast<const char *>(&v), sizeof(v)); };
