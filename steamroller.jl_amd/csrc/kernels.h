@@ -1767,6 +1767,241 @@ __global__ __launch_bounds__(NT) void k_gs_sweep(T *__restrict__ uo, const T *__
     }
 }
 
+// The blocks around each block of a 2D level, for k_gs_sweep2: in nine[45 blk],
+// the same-level block at offset (n % 3 - 1, n / 3 - 1), -1 where there is none
+// or -2 beyond the domain (n = 0 .. 8; a diagonal one by way of a face
+// neighbour, as values reach this block), then the neighbour-table entries of
+// each.
+constexpr int NINE = 45;
+__global__ __launch_bounds__(WG) void k_nine(int *__restrict__ nine, const int *__restrict__ nbr, int nb) {
+    const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int blk = (int)(gt / NINE), i = (int)(gt - (int64_t)blk * NINE);
+    if (blk >= nb) return;
+    const int n = i < 9 ? i : (i - 9) / 4, dx = n % 3, dy = n / 3;
+    int e = blk;
+    if (dx != 1 && dy != 1) {
+        const int ex = nbr[(size_t)blk * 4 + (dx >> 1)], ey = nbr[(size_t)blk * 4 + 2 + (dy >> 1)];
+        e = ex >= 0 ? nbr[(size_t)ex * 4 + 2 + (dy >> 1)] : (ey >= 0 ? nbr[(size_t)ey * 4 + (dx >> 1)] : -2);
+    } else if (dx != 1) {
+        e = nbr[(size_t)blk * 4 + (dx >> 1)];
+    } else if (dy != 1) {
+        e = nbr[(size_t)blk * 4 + 2 + (dy >> 1)];
+    }
+    if (e < 0) e = e == NB_BOUNDARY ? -2 : -1;
+    nine[gt] = i < 9 ? e : (e >= 0 ? nbr[(size_t)e * 4 + (i - 9) % 4] : NB_BOUNDARY);
+}
+
+// Two sweeps of a 2D level in one launch: k_gs_sweep's scheme with a deeper
+// halo. A work group takes a block with the cells within four steps of it and
+// runs the four half-sweeps there, each on the cells within one step less
+// (the neighbours' cells by the operations of their owners), so the result is
+// that of two launches. On a small level a launch is its round trips and costs
+// the same whatever it does; on a large one the two sweeps read the field once.
+// Two sweeps of 16 to 256 blocks of 16^2 in FP64: 10.5 -> 4.8 us, of 1,024: 11.2
+// -> 6.2, of 4,096: 16.0 -> 12.0, of 16,384: 53.8 -> 33.6 (3.2 TB/s of what one
+// pass over u, b and u must move; the halo's arithmetic bounds it).
+//
+// Ghosts: a boundary ghost is the cell itself times the face's sign. Frozen
+// slab values stand in the tile where they are seen, those seen across a y face
+// in a second tile, since beyond a concave corner of the level one place is
+// two blocks' ghost.
+//
+// Of a large level it is the index arithmetic that costs: the cells of each
+// thread are a table (Gs2Table), and what only blocks at a face of the level
+// need is behind a branch on the wave's view of the surroundings.
+template <int M>
+constexpr int GS2_THREADS = M == 16 ? 256 : 128;
+// What thread tid does: cells 0 and 1 of half-sweeps k and k + 2, and cell 2 of
+// the ring four steps from the block (read only). Of each: the place co in its
+// block and cq in the tile (by row, the columns of one colour together: a
+// half-sweep reads the other), the offset cn of its block, the distance cd
+// from this one (7: no such cell); of the first two cells the offsets of the
+// blocks of the four cells they read.
+template <int M>
+struct Gs2Table {
+    static constexpr int HD = 4, W = M + 2 * HD, WH = W / 2, NX = M / 2 + 3, NRING = 4 * M + 12;
+    struct E {
+        uint32_t q[4];  // co, cq: 12 bits each (cells 0, 1, 2); co of cell k at 12 k of q[0..1] as 64 bits, cq of q[2..3]
+        uint32_t c;     // cn: 4 bits each; cd: 3 bits each from bit 12; x even: bits 24, 25
+        uint32_t r;     // 4 bits each: cell k, face f at 4 (4 k + f)
+        uint32_t pad[2];
+    } e[GS2_THREADS<M>];
+    static constexpr int side(int c) { return c < 0 ? 0 : (c >= M ? 2 : 1); }
+    static constexpr int over(int c) { return c < 0 ? -c : (c >= M ? c - M + 1 : 0); }
+    static constexpr int pos(int x, int y) { return ((y + HD) * 2 + ((x + y) & 1)) * WH + ((x + HD) >> 1); }
+    constexpr Gs2Table() : e() {
+        static_assert(NX * (M + 6) <= GS2_THREADS<M> && NRING <= GS2_THREADS<M> && W * W < 4096 && HD <= M,
+                      "work of each thread");
+        for (int t = 0; t < GS2_THREADS<M>; t++) {
+            uint64_t co = 0, cq = 0;
+            uint32_t c = 0, r = 0;
+            for (int k = 0; k < 3; k++) {
+                int x = 0, y = t / NX - 3;
+                bool in = y < M + 3;
+                if (k < 2) {
+                    x = 2 * (t % NX) - 3 + ((y + k) & 1);
+                    in = in && over(x) + over(y) < HD;
+                } else {
+                    const int f = t / M, q = t % M, j = t - 4 * M, dx = j % 3 + 1;
+                    x = f == 0 ? -HD : (f == 1 ? M - 1 + HD : q);
+                    y = f == 2 ? -HD : (f == 3 ? M - 1 + HD : q);
+                    if (f >= 4) {
+                        x = (j / 3) & 1 ? M - 1 + dx : -dx;
+                        y = (j / 3) & 2 ? M - 1 + HD - dx : dx - HD;
+                    }
+                    in = t < NRING;
+                }
+                if (!in) {
+                    c |= 7u << (12 + 3 * k);
+                    continue;
+                }
+                const int bx = x - M * (side(x) - 1), by = y - M * (side(y) - 1);
+                const int odd = (bx + by) & 1;  // Lay<2, M>::sidx
+                co |= (uint64_t)((odd ? 0 : M * M / 2) + (bx >> 1) + M / 2 * by) << (12 * k);
+                cq |= (uint64_t)pos(x, y) << (12 * k);
+                c |= (uint32_t)(side(x) + 3 * side(y)) << (4 * k);
+                c |= (uint32_t)(over(x) + over(y)) << (12 + 3 * k);
+                if (k == 2) continue;
+                if (!(x & 1)) c |= 1u << (24 + k);
+                for (int f = 0; f < 4; f++) {
+                    const int nx = x + (f == 0 ? -1 : (f == 1 ? 1 : 0)), ny = y + (f == 2 ? -1 : (f == 3 ? 1 : 0));
+                    r |= (uint32_t)(side(nx) + 3 * side(ny)) << (4 * (4 * k + f));
+                }
+            }
+            e[t].q[0] = (uint32_t)co;
+            e[t].q[1] = (uint32_t)(co >> 32);
+            e[t].q[2] = (uint32_t)cq;
+            e[t].q[3] = (uint32_t)(cq >> 32);
+            e[t].c = c;
+            e[t].r = r;
+        }
+    }
+};
+template <int M>
+__device__ const Gs2Table<M> GS2_TABLE{};
+
+template <int M, typename T, int RD>
+__global__ __launch_bounds__(GS2_THREADS<M>) void k_gs_sweep2(T *__restrict__ uo, const T *__restrict__ ui,
+                                                              const T *__restrict__ b, const T *__restrict__ ib,
+                                                              const int *__restrict__ nine,
+                                                              const int *__restrict__ coord, LevelArgs<T> a) {
+    using LY = Lay<2, M>;
+    using TB = Gs2Table<M>;
+    constexpr int HD = TB::HD, W = TB::W, WH = TB::WH;
+    __shared__ T t[2 * W * W];  // the tile, then the one seen across y faces
+    __shared__ int nn[NINE];
+    const int tid = threadIdx.x, blk = a.blk0 + xcd_remap(blockIdx.x, gridDim.x);
+
+    // round trip 1: the block's surroundings and parameters, this thread's cells
+    const uint4 q4 = *reinterpret_cast<const uint4 *>(GS2_TABLE<M>.e[tid].q);
+    const uint2 q2 = *reinterpret_cast<const uint2 *>(&GS2_TABLE<M>.e[tid].c);
+    int nv = 0;
+    if (tid < NINE) nv = nine[(size_t)blk * NINE + tid];
+    const BP<T> bp = bparams(a, blk);
+    const int J = rbase<2, M, RD>(coord, blk);
+    const uint64_t qo = q4.x | (uint64_t)q4.y << 32, qq = q4.z | (uint64_t)q4.w << 32;
+    int co[3], cq[3], cd[3], e[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        co[k] = (int)(qo >> (12 * k)) & 4095;
+        cq[k] = (int)(qq >> (12 * k)) & 4095;
+        cd[k] = (int)(q2.x >> (12 + 3 * k)) & 7;
+    }
+    if (tid < NINE) nn[tid] = nv;
+    __syncthreads();
+
+    // round trip 2: the cells, the radial weights. miss, dom: the offsets
+    // without a block, and beyond the domain
+    const int lane = tid & 63, ns = nn[lane < 9 ? lane : 4];
+    const unsigned miss = (unsigned)__ballot(ns < 0) & 511u, dom = (unsigned)__ballot(ns == -2) & 511u;
+    T v[3], vb[2], wm[2] = {T(1), T(1)}, wp[2] = {T(1), T(1)};
+    const int tn[2] = {2 * (tid % TB::NX) - 3, tid / TB::NX - 3};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        v[k] = T(0);
+        if (k < 2) vb[k] = T(0);
+        e[k] = -1;
+        if (cd[k] == 7) continue;
+        e[k] = nn[q2.x >> (4 * k) & 15];
+        if (e[k] < 0) continue;
+        const size_t o = (size_t)e[k] * LY::V + co[k];
+        v[k] = ui[o];
+        if (k < 2) {
+            vb[k] = b[o];
+            rweights<T, RD>(a, J + (RD == 0 ? tn[0] + ((tn[1] + k) & 1) : tn[1]), wm[k], wp[k]);
+        }
+    }
+    // the faces of the two cells beyond which there is no block, or no domain
+    unsigned fm = 0, fd = 0;
+    if (miss) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const unsigned n = q2.y >> (4 * j) & 15;
+            fm |= (miss >> n & 1) << j;
+            fd |= (dom >> n & 1) << j;
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if (cd[k] == 7 || e[k] >= 0) continue;
+            // a slab cell, seen from the column beside (across its face fx) or the row beside
+            const int q = cq[k], h = q % WH, yy = q / (2 * WH), y = yy - HD;
+            const int x = 2 * h - HD + ((q / WH + y) & 1);
+            const int n = q2.x >> (4 * k) & 15, sx = n % 3, sy = n / 3;
+            const int nx = x == 0 ? 0 : (x == -1 || x == M ? 1 : (x == M - 1 ? 2 : 3));
+            const int fx = x == 0 || x == M ? 1 : 0;
+            const int ny = y == 0 ? 0 : (y == -1 || y == M ? 1 : (y == M - 1 ? 2 : 3));
+            const int fy = y == 0 || y == M ? 3 : 2;
+            const int g0 = nx < 3 ? nn[9 + 4 * (nx + 3 * sy) + fx] : NB_BOUNDARY;
+            const int g1 = ny < 3 ? nn[9 + 4 * (sx + 3 * ny) + fy] : NB_BOUNDARY;
+            if (g0 < NB_BOUNDARY) v[k] = ib[(size_t)nb_slot(g0) * LY::F + y - M * (sy - 1)];
+            if (g1 < NB_BOUNDARY) t[W * W + q] = ib[(size_t)nb_slot(g1) * LY::F + x - M * (sx - 1)];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        if (cd[k] != 7) t[cq[k]] = v[k];
+    __syncthreads();
+    // where the four cells are: beside, in the other colour's half of the row
+    int px[2], ym[2], yp[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int r = cq[k] + (k == 0 ? -WH : WH);
+        px[k] = r - (int)(q2.x >> (24 + k) & 1);
+        ym[k] = r - 2 * WH + (fm >> (4 * k + 2) & 1 ? W * W : 0);
+        yp[k] = r + 2 * WH + (fm >> (4 * k + 3) & 1 ? W * W : 0);
+    }
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        const int k = p & 1;
+        if (e[k] >= 0 && cd[k] < HD - p) {
+            const T o = v[k];
+            T xa = t[px[k]], xb = t[px[k] + 1], ya = t[ym[k]], yb = t[yp[k]];
+            if (dom) {
+                if (fd >> (4 * k) & 1) xa = a.sg[0] * o;
+                if (fd >> (4 * k) & 2) xb = a.sg[1] * o;
+                if (fd >> (4 * k) & 4) ya = a.sg[2] * o;
+                if (fd >> (4 * k) & 8) yb = a.sg[3] * o;
+            }
+            T Lu = T(0);
+            if (RD == 1) Lu += wm[k] * ya;
+            else Lu += ya;
+            if (RD == 0) Lu += wm[k] * xa;
+            else Lu += xa;
+            Lu += bp.cc * o;
+            if (RD == 0) Lu += wp[k] * xb;
+            else Lu += xb;
+            if (RD == 1) Lu += wp[k] * yb;
+            else Lu += yb;
+            v[k] = fma_t<T>(bp.nwc, fma_t<T>(bp.s, vb[k], Lu), o);
+            if (p < 3) t[cq[k]] = v[k];
+        }
+        if (p < 3) lds_barrier();
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+        if (cd[k] == 0) uo[(size_t)blk * LY::V + co[k]] = v[k];
+}
+
 // k_gs_sweep on sibling groups: the 2^D children of one parent (consecutive
 // in the Morton order of a level, always created together) form one
 // (2M)^D tile. The faces between siblings need no halo and no recompute; the

@@ -186,6 +186,7 @@ struct srmg_ctx {
     std::vector<int4> h_slots;
     // device tables
     DevBuf d_nbr, d_coord, d_parent, d_sub, d_slots, d_leaves, d_halo, d_isleaf, d_pix;
+    DevBuf d_nine;  // 2D: k_nine's table
     DevBuf d_w64, d_w32;    // radial weights (double / float), per level and dim
     DevBuf d_partial;
     PinnedBuf norms;        // per tree: the sum of the norm queued last, written by the device
@@ -648,6 +649,12 @@ static void upload_tables(srmg_ctx *c) {
     up(c->d_slots, c->h_slots.data(), c->h_slots.size() * sizeof(int4));
     up(c->d_leaves, c->h_leaves.data(), c->h_leaves.size() * sizeof(int));
     up(c->d_halo, htab.data(), htab.size() * sizeof(int));
+    if (D == 2) {
+        c->d_nine.alloc((size_t)nb * NINE * sizeof(int));
+        if (nb)
+            hipLaunchKernelGGL(k_nine, dim3((unsigned)(((int64_t)nb * NINE + WG - 1) / WG)), dim3(WG), 0, c->stream,
+                               c->d_nine.as<int>(), c->d_nbr.as<int>(), nb);
+    }
     up(c->d_isleaf, isleaf.data(), isleaf.size() * sizeof(int));
     up(c->d_pix, pix.data(), pix.size() * sizeof(int));
     up(c->d_w64, w64.data(), w64.size() * sizeof(double));
@@ -1148,9 +1155,27 @@ struct Ops {
         }
         u.cur[l] ^= 1;
     }
+    // 2D sweeps go in pairs (k_gs_sweep2) at every size of 16^2 blocks (16,384
+    // blocks in FP64: 33.6 us for 46.9 with the best shape of two single sweeps,
+    // FP32 28.9 for 30.2; 1,024: 6.2 for 10.0) and up to 8,192 blocks of 8^2
+    // (11.2 for 13.0, FP32 9.9 for 10.3; 16,384 blocks: 17.7 for 17.3, FP32 15.3
+    // for 13.6: half of what a work group computes there is halo)
+    bool pairs(int nblk) const { return D == 2 && (M == 16 || nblk <= 8192); }
     // gauss_seidel_iter! (src/multigrid.jl:250-265)
     void smooth(FieldBuf &u, FieldBuf &b, const LevelArgs<T> &a, int l, int n, bool zin = false) {
-        for (int i = 0; i < n; i++) sweep(u, b, a, l, -1, zin && i == 0);
+        int i = 0;
+        if constexpr (D == 2)
+            for (; i + 2 <= n && a.nblk && pairs(a.nblk); i += 2) {
+                need_alt(u);
+                T *in = X(u, l), *out = u.cur[l] ? u.data.as<T>() : u.alt.as<T>();
+                with_rd(a.rdim, [&](auto rd) {
+                    constexpr int RD = decltype(rd)::value;
+                    hipLaunchKernelGGL((k_gs_sweep2<M, T, RD>), dim3((unsigned)a.nblk), dim3(GS2_THREADS<M>), 0,
+                                       c->stream, out, in, X(b, l), I(u), c->d_nine.as<int>(), coord(), a);
+                });
+                u.cur[l] ^= 1;
+            }
+        for (; i < n; i++) sweep(u, b, a, l, -1, zin && i == 0);
     }
     // residual kernels from LDS tiles (base tile shape)
     static constexpr int RB = SMALL ? 256 / LY::H : 1;
