@@ -717,9 +717,20 @@ static void upload_tables(srmg_ctx *c) {
         btabs.push_back(std::move(tab));
         up(G.btab, btabs.back().data(), btabs.back().size() * sizeof(int));
     }
-    // until autotuned or set: the column sweep on two threads per column for
-    // 8^3 blocks (levels without complete sibling groups run shape 0)
-    c->sweep_cfg.assign(2 * nlevels, (c->D == 3 && c->M == 8) ? 8 : 0);
+    // until autotuned or set: for 8^3 blocks the column sweep on two threads per
+    // column (shape 8; levels without complete sibling groups run shape 0),
+    // except on levels small enough that the launch is latency and its groups
+    // fill the chip unevenly: there a work group takes one block. FP64, shapes
+    // 0 / 8: 512 blocks 4.5 / 6.8 us, 1,200 6.5 / 7.6, 5,184 15.6 / 16.8, 14,976
+    // 36.2 / 38.8, 32,768 119 / 97. FP32: 512 blocks 4.0 / 5.5, 1,200 5.6 / 6.1,
+    // 1,728 equal, 2,744 8.3 / 7.5 (the finest level keeps shape 8, which can
+    // start from zero without reading it)
+    c->sweep_cfg.assign(2 * nlevels, 0);
+    if (c->D == 3 && c->M == 8)
+        for (int l = 0; l < nlevels; l++) {
+            c->sweep_cfg[l] = c->lv[l].nblk <= 16384 ? 0 : 8;
+            c->sweep_cfg[nlevels + l] = c->lv[l].nblk <= 1200 && l < nlevels - 1 ? 0 : 8;
+        }
     c->zero[0].reset();
     c->zero[1].reset();
     c->ps.clear();
