@@ -2988,20 +2988,30 @@ __global__ __launch_bounds__(NT) void k_resid_group(TO *__restrict__ out, const 
 // groups past ngroups copy u -> u1 on the coarse level's leaf blocks (lists
 // leaves[0..nleafc)), completing copyto!(u1, u) on that level. Same values
 // and operations as residual + restrict(u) + copy + restrict(r).
+//
+// 2D: the coarse right-hand side of the parent's cells too (k_postrestrict_group
+// on its own: 3.3 to 4.8 us of launch and two round trips a level). What it
+// needs beyond the parent's cells are the coarse cells around: a covered one is
+// the mean of its children (restricted here again, in the same order), a leaf's
+// is read, a mirror or a slab as ever. FP64 levels of 504 / 1,976 / 3,872 blocks:
+// 5.8 / 7.0 / 9.0 us for 4.7 + 4.1 / 5.9 + 4.2 / 7.5 + 4.8 in two launches.
 template <int D, int M, typename T, int RT, int RD, int NT = 1024>
 __global__ __launch_bounds__(NT) void k_resid_restrict(const T *__restrict__ u, const T *__restrict__ b,
                                                          const T *__restrict__ ib, const int *__restrict__ htab,
                                                          const int *__restrict__ coord,
                                                          const int *__restrict__ parent, LevelArgs<T> a,
                                                          unsigned ngroups, T *__restrict__ rc, T *__restrict__ uc,
-                                                         T *__restrict__ u1c, const T *__restrict__ ucin,
-                                                         const int *__restrict__ leaves, int nleafc) {
+                                                         T *__restrict__ u1c, const T *ucin,
+                                                         const int *__restrict__ leaves, int nleafc, T *__restrict__ bc,
+                                                         LevelArgs<T> ac) {
     using LY = Lay<D, M>;
     using TL = Tile<D, M, 2>;
     using HT = Halo<D>;
+    using TC = Tile<D, M>;
     constexpr int NB = 1 << D, V = LY::V, F = LY::F, MH = LY::MH;
     constexpr int TEAMS = NT / RT;
     static_assert(NB % TEAMS == 0 && RT >= 64, "team layout");
+    static_assert(D == 3 || (V <= NT && 4 * M <= NT), "2D: a coarse cell, and one of those around, for each thread");
     const int tid = threadIdx.x;
     if (blockIdx.x >= ngroups) {
         // u1 = u on the coarse level's leaf blocks
@@ -3047,13 +3057,51 @@ __global__ __launch_bounds__(NT) void k_resid_restrict(const T *__restrict__ u, 
             }
     };
     int pb = 0;
+    // the coarse cell beyond face f, tangential index ct, of the parent
+    const int f = tid / M, ct = tid % M, fr0 = f & 1 ? 0 : M - 2;
+    T hc = T(0), cw[2] = {T(1), T(1)};
+    BP<T> cbp{};
+    auto around = [&] {
+        if constexpr (D == 2) {
+            cbp = bparams(ac, pb);
+            if constexpr (RD >= 0) {
+                int x, y, z;
+                LY::decode(tid % V, x, y, z);
+                // the parent's radial index, from its first child's
+                const int Jp = M * ((rbase<D, M, RD>(coord, g0) - 1) / M / 2) + 1;
+                rweights<T, RD>(ac, Jp + (RD == 0 ? x : y), cw[0], cw[1]);
+            }
+            if (f >= 4) return;
+            // the child on that face
+            const int half = ct >= MH, k = f < 2 ? (f & 1) + 2 * half : half + 2 * (f & 1);
+            const int e = tab[k * 2 * D + f];
+            if (e >= 0) {
+                T m = T(0);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int in = f < 2 ? q & 1 : q >> 1, it = f < 2 ? q >> 1 : q & 1;
+                    const int cn = fr0 + in, cf = 2 * (ct - half * MH) + it;
+                    m += u[(size_t)e * V + LY::sidx(f < 2 ? cn : cf, f < 2 ? cf : cn, 0)];
+                }
+                hc = m / T(LY::NC);
+            } else if (e != NB_BOUNDARY) {
+                const int pe = htab[(size_t)pb * HT::N + f];
+                const int cn = f & 1 ? 0 : M - 1;
+                hc = pe >= 0 ? ucin[(size_t)pe * V + LY::sidx(f < 2 ? cn : ct, f < 2 ? ct : cn, 0)]
+                             : ib[(size_t)max(nb_slot(pe), 0) * F + ct];
+            }
+        }
+    };
     stage_group<D, M, T, NT>(
         tile, tab, prm, u, ib, htab, a, g0,
         [&] {
             coords();
             pb = parent[g0];
         },
-        weights);
+        [&] {
+            weights();
+            around();
+        });
 #pragma unroll
     for (int round = 0; round < NR; round++) {
         const int lb = team + round * TEAMS;
@@ -3070,6 +3118,8 @@ __global__ __launch_bounds__(NT) void k_resid_restrict(const T *__restrict__ u, 
         }
     }
     __syncthreads();
+    __shared__ T ctile[D == 2 ? TC::SZ : 1];
+    T rcv = T(0);
     // the parent's cells: coarse cell X of sub-block k = (X >= MH per dim)
     for (int i = tid; i < V; i += NT) {
         int X0, X1, X2;
@@ -3089,6 +3139,27 @@ __global__ __launch_bounds__(NT) void k_resid_restrict(const T *__restrict__ u, 
         const T uv = fu / T(LY::NC);
         uc[o] = uv;
         if (u1c) u1c[o] = uv;
+        if constexpr (D == 2) {
+            rcv = fr / T(LY::NC);
+            ctile[TC::at(X0, X1, 0)] = uv;
+        }
+    }
+    if constexpr (D == 2) {
+        __syncthreads();
+        if (f < 4) {
+            const int cn = f & 1 ? M : -1, in = f & 1 ? M - 1 : 0;
+            const int k = (f < 2 ? (f & 1) : (ct >= MH)) + 2 * (f < 2 ? (ct >= MH) : (f & 1));
+            if (tab[k * 2 * D + f] == NB_BOUNDARY) hc = ac.sg[f] * ctile[f < 2 ? TC::at(in, ct, 0) : TC::at(ct, in, 0)];
+            ctile[f < 2 ? TC::at(cn, ct, 0) : TC::at(ct, cn, 0)] = hc;
+        }
+        __syncthreads();
+        if (tid < V) {
+            int X0, X1, X2;
+            LY::decode(tid, X0, X1, X2);
+            const int p = TC::at(X0, X1, 0);
+            const T Lu = tstencil<D, M, T, RD>(ctile, p, ctile[p], cbp.cc, cw[0], cw[1]);
+            bc[(size_t)pb * V + tid] = -(rcv + Lu / cbp.s);
+        }
     }
 }
 

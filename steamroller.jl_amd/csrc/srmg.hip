@@ -1222,10 +1222,12 @@ struct Ops {
                                (const int *)nullptr, a.nblk, a, 0.0, (double *)nullptr);
         });
     }
-    // residual(r, u, b, l); restrict_(u, l); [copy(u1, u, l - 1);] restrict_(r, l)
+    // residual(r, u, b, l); restrict_(u, l); [copy(u1, u, l - 1);] restrict_(r, l);
+    // in 2D postrestrict(b, u, r, l, ac) as well;
     // in one launch on grouped levels (r on level l itself is not written);
     // false when the level is not grouped (the caller runs the four steps)
-    bool resid_restrict(FieldBuf &r, FieldBuf &u, FieldBuf *u1, FieldBuf &b, const LevelArgs<T> &a, int l) {
+    bool resid_restrict(FieldBuf &r, FieldBuf &u, FieldBuf *u1, FieldBuf &b, const LevelArgs<T> &a, int l,
+                        const LevelArgs<T> &ac) {
         if constexpr (GROUP_OK) {
             if (!a.nblk || !grouped(l)) return false;
             const LevelInfo &Lc = c->lv[l - 1];
@@ -1246,7 +1248,8 @@ struct Ops {
                                        c->stream, X(u, l), X(b, l), I(u), c->d_halo.as<int>(), coord(),
                                        c->d_parent.as<int>(), a, ng, X(r, l - 1), X(u, l - 1),
                                        u1 ? X(*u1, l - 1) : (T *)nullptr, X(u, l - 1),
-                                       c->d_leaves.as<int>() + Lc.leaf0, nleafc);
+                                       c->d_leaves.as<int>() + Lc.leaf0, nleafc,
+                                       D == 2 ? X(b, l - 1) : (T *)nullptr, ac);
                 }
             });
             return true;
@@ -1727,13 +1730,14 @@ struct Ops {
             LevelArgs<T> a = level_args<T>(c, l, s, op, omega);
             LevelArgs<T> ac = level_args<T>(c, l - 1, s, op, omega);
             smooth(u, b, a, l, ndown, zin && l == lmax - 1);
-            if (!resid_restrict(r, u, &u1, b, a, l)) {
+            const bool done = resid_restrict(r, u, &u1, b, a, l, ac);
+            if (!done) {
                 residual(r, u, b, a, l);
                 restrict_(u, l);
                 copy(u1, u, l - 1);
                 restrict_(r, l);
             }
-            postrestrict(b, u, r, l, ac);
+            if (D == 3 || !done) postrestrict(b, u, r, l, ac);
         }
         top(u, b, s, op, ntop, omega);
         for (int l = 1; l < lmax; l++) {
