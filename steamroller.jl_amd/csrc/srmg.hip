@@ -220,6 +220,7 @@ struct srmg_ctx {
     // the order-4 operator's box neighbour table and coarse-fine slots (built
     // on first use; see box_table)
     DevBuf d_box, d_box_slots;
+    bool slabs_apart = false;  // no coarse-fine slab is interpolated from another one
     std::vector<uint8_t> box_cf;  // per level: some direction of a block is coarse-fine (with box_ok)
     bool box_ok = false;  // bumped when coarse-solve matrices are rebuilt (older graphs point to freed ones)
 };
@@ -489,6 +490,15 @@ static void build_tables(srmg_ctx *c, const std::vector<TreeRecords> &tr) {
         if (c->h_nbr[i] == INT32_MIN)
             fail("block " + std::to_string(c->dev2host[i / ND]) + " face " + std::to_string(i % ND) +
                  " has no neighbour, boundary or refinement record");
+    // whether a slab's interpolation reads another slab: of the coarse block's
+    // neighbours it reads those beyond the faces that its half of the block touches
+    c->slabs_apart = true;
+    for (const int4 &q : c->h_slots)
+        for (int d = 0; d < D; d++) {
+            const int up = (q.w >> d) & 1;
+            if (d == (q.y >> 1) && up == (q.y & 1)) continue;  // that neighbour is inside the block
+            if (c->h_nbr[(size_t)q.z * ND + 2 * d + up] < NB_BOUNDARY) c->slabs_apart = false;
+        }
     for (int l = 1; l < nlevels; l++)
         for (int b = c->lv[l].blk0; b < c->lv[l].blk0 + c->lv[l].nblk; b++)
             if (c->h_parent[b] < 0) fail("block without Child record");
@@ -561,6 +571,7 @@ static void commit_tables(srmg_ctx *c, srmg_ctx &t) {
     c->trees = std::move(t.trees);
     c->groups = std::move(t.groups);
     c->h_nbr = std::move(t.h_nbr);
+    c->slabs_apart = t.slabs_apart;
     c->h_coord = std::move(t.h_coord);
     c->h_parent = std::move(t.h_parent);
     c->h_sub = std::move(t.h_sub);
@@ -1578,6 +1589,18 @@ struct Ops {
         hipLaunchKernelGGL((k_fill_interp<D, M, T>), dim3(nwg((int64_t)L.nslot * LY::F)), dim3(WG), 0, c->stream,
                            I(x), X(x, l - 1), nbr(), c->d_slots.as<int4>(), L.slot0, L.nslot, ac);
     }
+    // of every level, from the coarsest. In one launch where no slab is
+    // interpolated from another (trees whose refined blocks have all their
+    // neighbours, diagonal ones too) and the values are in one buffer: on small
+    // trees a launch a level was 3.1 us each of latency
+    void fill_interp_all(FieldBuf &x, const LevelArgs<T> &a) {
+        if (!c->nslot) return;
+        if (c->slabs_apart && x.settled())
+            hipLaunchKernelGGL((k_fill_interp<D, M, T>), dim3(nwg((int64_t)c->nslot * LY::F)), dim3(WG), 0, c->stream,
+                               I(x), X(x, 0), nbr(), c->d_slots.as<int4>(), 0, c->nslot, a);
+        else
+            for (int l = 1; l < c->nlevels; l++) fill_interp(x, l, a);
+    }
     // residual norms (NORM: of the leaf blocks, out unused) or defects into out
     // with the norms' partials (of every block), all levels in one launch for
     // each SEG_MAX of them; levels keep their values in the primary buffer
@@ -1876,7 +1899,7 @@ void Ops<D, M, T>::first_iterate(FieldBuf &u, FieldBuf &b, int mode, int nsmooth
     }
     for (int l = 1; l < c->nlevels; l++) interp_fill(u, u, l, level_args<T>(c, l - 1, s, op, 1.0));
     for (int l = c->nlevels - 1; l >= 1; l--) restrict_(u, l);
-    for (int l = 1; l < c->nlevels; l++) fill_interp(u, l, level_args<T>(c, l - 1, s, op, 1.0));
+    fill_interp_all(u, level_args<T>(c, 0, s, op, 1.0));
     if (!check) return;
     resnorm_partials(u, b, s, op);
     fall_back(u, read_norms(c), r0);
@@ -1901,7 +1924,7 @@ int Ops<D, M, T>::fall_back(FieldBuf &u, const std::vector<double> &rg, const st
         }
     }
     if (c->guess_fallbacks)
-        for (int l = 1; l < c->nlevels; l++) fill_interp(u, l, level_args<T>(c, l - 1, s, op, 1.0));
+        fill_interp_all(u, level_args<T>(c, 0, s, op, 1.0));
     return c->guess_fallbacks;
 }
 
@@ -2474,7 +2497,7 @@ static void solve_plain(srmg_ctx *c, int ui, int bi, int ri, int u1i, const srmg
             r0 = safe_r0(read_norms(c));
             done = record(r0, r0, o->tol, 0, o->max_cycles, hist);
         } else {
-            for (int l = 1; l < c->nlevels; l++) ops.fill_interp(u, l, level_args<T>(c, l - 1, s, op, 1.0));
+            ops.fill_interp_all(u, level_args<T>(c, 0, s, op, 1.0));
             ops.resnorm_partials(zero_field(c, t), b, s, op);
             r0 = safe_r0(read_norms(c));
             if (o->guess) ops.first_iterate(u, b, o->guess, o->guess_smooth, r0);
@@ -2544,7 +2567,7 @@ static void solve_mixed_dm(srmg_ctx *c, FieldBuf &u, FieldBuf &b, FieldBuf &e, F
         o64.bnorm_partials(b, be.data.as<float>());
         r0 = safe_r0(read_norms(c));
     } else {
-        for (int l = 1; l < c->nlevels; l++) o64.fill_interp(u, l, level_args<double>(c, l - 1, s, op, 1.0));
+        o64.fill_interp_all(u, level_args<double>(c, 0, s, op, 1.0));
         o64.bnorm_partials(b);  // resnorm(u = 0), from b alone
         r0 = safe_r0(read_norms(c));
         // a first iterate is checked against r0 with the norm of the first
@@ -2612,7 +2635,7 @@ static void solve_mixed_dm(srmg_ctx *c, FieldBuf &u, FieldBuf &b, FieldBuf &e, F
             // fixed point; otherwise the leaf residual would not pin them
             for (int l = c->nlevels - 1; l >= 1; l--) o64.restrict_(u, l);
         }
-        for (int l = 1; l < c->nlevels; l++) o64.fill_interp(u, l, level_args<double>(c, l - 1, s, op, 1.0));
+        o64.fill_interp_all(u, level_args<double>(c, 0, s, op, 1.0));
         defect_and_norm();
     };
     bool done;
@@ -2852,7 +2875,7 @@ static void regrid_fields(srmg_ctx *c, const std::vector<TreeRecords> &tr, const
             using T = std::remove_reference_t<decltype(*o.X(f, 0))>;
             o.settle(f);
             if (modes[k] & SRMG_REGRID_INTERP)
-                for (int l = 1; l < c->nlevels; l++) o.fill_interp(f, l, level_args<T>(c, l - 1, 1.0, &op, 1.0));
+                o.fill_interp_all(f, level_args<T>(c, 0, 1.0, &op, 1.0));
         });
     }
     // Blocks are matched through sorted Morton codes per (tree, level): the
@@ -3044,8 +3067,8 @@ int srmg_rhs(srmg_ctx *c, int b1, int b, const srmg_op *op) {
             o.settle(fb1);
             // fill_ghost!(b, l) then rhs_level!(b1, b, l), level by level
             // (src/streamer.jl:314-318)
+            o.fill_interp_all(fb, level_args<T>(c, 0, 1.0, op, 1.0));
             for (int l = 0; l < c->nlevels; l++) {
-                if (l > 0) o.fill_interp(fb, l, level_args<T>(c, l - 1, 1.0, op, 1.0));
                 if (op->disc == SRMG_LAPLACIAN4) o.rhs4_level(fb1, fb, l, level_args<T>(c, l, 1.0, op, 1.0));
             }
             // order 2: b1 = b, on all levels at once
@@ -3169,7 +3192,7 @@ int srmg_fill_ghost_all(srmg_ctx *c, int id, const int8_t *bc) {
         std::memcpy(op.bc, bc, 27);
         dispatch(c, f.dtype, [&](auto &o) {
             using T = std::remove_reference_t<decltype(*o.X(f, 0))>;
-            for (int l = 1; l < c->nlevels; l++) o.fill_interp(f, l, level_args<T>(c, l - 1, 1.0, &op, 1.0));
+            o.fill_interp_all(f, level_args<T>(c, 0, 1.0, &op, 1.0));
         });
     });
 }
