@@ -688,25 +688,34 @@ struct Ext {
     int n0, n1, n2;
 };
 
-__device__ inline int64_t vindex(const Ext &e, int x, int y, int z) {
-    return x + (int64_t)e.n0 * (y + (int64_t)e.n1 * z);
+// I: the type of the index arithmetic. 32 bits where the tensor's offsets fit
+// (for_index): 64-bit divisions were a third of what pooling and upsampling of
+// 64^3 x 8 took: 5.2 -> 3.4 and 4.3 -> 3.7 us, a forward pass 151 -> 146
+template <class I>
+__device__ inline I vindex(const Ext &e, int x, int y, int z) {
+    return x + (I)e.n0 * (y + (I)e.n1 * z);
+}
+template <class Fn>
+void for_index(int64_t values, Fn &&fn) {
+    if (values < ((int64_t)1 << 31)) fn((uint32_t)0);
+    else fn((int64_t)0);
 }
 
 // coarse voxel -> its 2^D children
-template <int D>
+template <int D, class I>
 __global__ __launch_bounds__(TPB) void k_pool(const uint16_t *__restrict__ in, uint16_t *__restrict__ out, int c8,
-                                              Ext ec, Ext ef, int64_t total) {
-    const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
+                                              Ext ec, Ext ef, I total) {
+    const I i = (I)blockIdx.x * TPB + threadIdx.x;
     if (i >= total) return;
     const int cg = (int)(i % c8);
-    const int64_t vc = i / c8, Vc = (int64_t)ec.n0 * ec.n1 * ec.n2, Vf = (int64_t)ef.n0 * ef.n1 * ef.n2;
-    const int64_t n = vc / Vc, r = vc - n * Vc;
-    const int xc = (int)(r % ec.n0), yc = (int)((r / ec.n0) % ec.n1), zc = (int)(r / ((int64_t)ec.n0 * ec.n1));
+    const I vc = i / c8, Vc = (I)ec.n0 * ec.n1 * ec.n2, Vf = (I)ef.n0 * ef.n1 * ef.n2;
+    const I n = vc / Vc, r = vc - n * Vc;
+    const int xc = (int)(r % ec.n0), yc = (int)((r / ec.n0) % ec.n1), zc = (int)(r / ((I)ec.n0 * ec.n1));
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int c = 0; c < (1 << D); c++) {
         const int xf = 2 * xc + (c & 1), yf = 2 * yc + ((c >> 1) & 1), zf = D == 3 ? 2 * zc + (c >> 2) : 0;
         float v[8];
-        unpack8(*reinterpret_cast<const uint4 *>(in + ((n * Vf + vindex(ef, xf, yf, zf)) * c8 + cg) * 8), v);
+        unpack8(*reinterpret_cast<const uint4 *>(in + ((n * Vf + vindex<I>(ef, xf, yf, zf)) * c8 + cg) * 8), v);
         for (int k = 0; k < 8; k++) acc[k] += v[k];
     }
     for (int k = 0; k < 8; k++) acc[k] *= 1.0f / (1 << D);
@@ -714,17 +723,17 @@ __global__ __launch_bounds__(TPB) void k_pool(const uint16_t *__restrict__ in, u
 }
 
 // fine voxel: out = coarse(parent) + skip
-template <int D>
+template <int D, class I>
 __global__ __launch_bounds__(TPB) void k_up_add(const uint16_t *__restrict__ coarse, const uint16_t *__restrict__ skip,
-                                                uint16_t *__restrict__ out, int c8, Ext ec, Ext ef, int64_t total) {
-    const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
+                                                uint16_t *__restrict__ out, int c8, Ext ec, Ext ef, I total) {
+    const I i = (I)blockIdx.x * TPB + threadIdx.x;
     if (i >= total) return;
     const int cg = (int)(i % c8);
-    const int64_t vf = i / c8, Vc = (int64_t)ec.n0 * ec.n1 * ec.n2, Vf = (int64_t)ef.n0 * ef.n1 * ef.n2;
-    const int64_t n = vf / Vf, r = vf - n * Vf;
-    const int x = (int)(r % ef.n0), y = (int)((r / ef.n0) % ef.n1), z = (int)(r / ((int64_t)ef.n0 * ef.n1));
+    const I vf = i / c8, Vc = (I)ec.n0 * ec.n1 * ec.n2, Vf = (I)ef.n0 * ef.n1 * ef.n2;
+    const I n = vf / Vf, r = vf - n * Vf;
+    const int x = (int)(r % ef.n0), y = (int)((r / ef.n0) % ef.n1), z = (int)(r / ((I)ef.n0 * ef.n1));
     float a[8], b[8];
-    unpack8(*reinterpret_cast<const uint4 *>(coarse + ((n * Vc + vindex(ec, x >> 1, y >> 1, z >> 1)) * c8 + cg) * 8),
+    unpack8(*reinterpret_cast<const uint4 *>(coarse + ((n * Vc + vindex<I>(ec, x >> 1, y >> 1, z >> 1)) * c8 + cg) * 8),
             a);
     unpack8(*reinterpret_cast<const uint4 *>(skip + i * 8), b);
     for (int k = 0; k < 8; k++) a[k] += b[k];
@@ -732,39 +741,39 @@ __global__ __launch_bounds__(TPB) void k_up_add(const uint16_t *__restrict__ coa
 }
 
 // coarse voxel: d coarse = sum of the children's d fine (adjoint of nearest upsampling)
-template <int D>
+template <int D, class I>
 __global__ __launch_bounds__(TPB) void k_up_bwd(const uint16_t *__restrict__ dfine, uint16_t *__restrict__ dcoarse,
-                                                int c8, Ext ec, Ext ef, int64_t total) {
-    const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
+                                                int c8, Ext ec, Ext ef, I total) {
+    const I i = (I)blockIdx.x * TPB + threadIdx.x;
     if (i >= total) return;
     const int cg = (int)(i % c8);
-    const int64_t vc = i / c8, Vc = (int64_t)ec.n0 * ec.n1 * ec.n2, Vf = (int64_t)ef.n0 * ef.n1 * ef.n2;
-    const int64_t n = vc / Vc, r = vc - n * Vc;
-    const int xc = (int)(r % ec.n0), yc = (int)((r / ec.n0) % ec.n1), zc = (int)(r / ((int64_t)ec.n0 * ec.n1));
+    const I vc = i / c8, Vc = (I)ec.n0 * ec.n1 * ec.n2, Vf = (I)ef.n0 * ef.n1 * ef.n2;
+    const I n = vc / Vc, r = vc - n * Vc;
+    const int xc = (int)(r % ec.n0), yc = (int)((r / ec.n0) % ec.n1), zc = (int)(r / ((I)ec.n0 * ec.n1));
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int c = 0; c < (1 << D); c++) {
         const int xf = 2 * xc + (c & 1), yf = 2 * yc + ((c >> 1) & 1), zf = D == 3 ? 2 * zc + (c >> 2) : 0;
         float v[8];
-        unpack8(*reinterpret_cast<const uint4 *>(dfine + ((n * Vf + vindex(ef, xf, yf, zf)) * c8 + cg) * 8), v);
+        unpack8(*reinterpret_cast<const uint4 *>(dfine + ((n * Vf + vindex<I>(ef, xf, yf, zf)) * c8 + cg) * 8), v);
         for (int k = 0; k < 8; k++) acc[k] += v[k];
     }
     *reinterpret_cast<uint4 *>(dcoarse + i * 8) = pack8(acc);
 }
 
 // fine voxel: d e = (d skip + d pooled(parent) / 2^D) * (e > 0)
-template <int D>
+template <int D, class I>
 __global__ __launch_bounds__(TPB) void k_pool_bwd(const uint16_t *__restrict__ dskip, const uint16_t *__restrict__ dp,
                                                   const uint16_t *__restrict__ e, uint16_t *__restrict__ de, int c8,
-                                                  Ext ec, Ext ef, int64_t total) {
-    const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
+                                                  Ext ec, Ext ef, I total) {
+    const I i = (I)blockIdx.x * TPB + threadIdx.x;
     if (i >= total) return;
     const int cg = (int)(i % c8);
-    const int64_t vf = i / c8, Vc = (int64_t)ec.n0 * ec.n1 * ec.n2, Vf = (int64_t)ef.n0 * ef.n1 * ef.n2;
-    const int64_t n = vf / Vf, r = vf - n * Vf;
-    const int x = (int)(r % ef.n0), y = (int)((r / ef.n0) % ef.n1), z = (int)(r / ((int64_t)ef.n0 * ef.n1));
+    const I vf = i / c8, Vc = (I)ec.n0 * ec.n1 * ec.n2, Vf = (I)ef.n0 * ef.n1 * ef.n2;
+    const I n = vf / Vf, r = vf - n * Vf;
+    const int x = (int)(r % ef.n0), y = (int)((r / ef.n0) % ef.n1), z = (int)(r / ((I)ef.n0 * ef.n1));
     float a[8], b[8];
     unpack8(*reinterpret_cast<const uint4 *>(dskip + i * 8), a);
-    unpack8(*reinterpret_cast<const uint4 *>(dp + ((n * Vc + vindex(ec, x >> 1, y >> 1, z >> 1)) * c8 + cg) * 8), b);
+    unpack8(*reinterpret_cast<const uint4 *>(dp + ((n * Vc + vindex<I>(ec, x >> 1, y >> 1, z >> 1)) * c8 + cg) * 8), b);
     const uint4 m = *reinterpret_cast<const uint4 *>(e + i * 8);
     const uint32_t mw[4] = {m.x, m.y, m.z, m.w};
     for (int k = 0; k < 8; k++) {
@@ -814,13 +823,13 @@ __global__ __launch_bounds__(TPB) void k_absmax(const double *__restrict__ part,
     if (threadIdx.x == 0) scale[blockIdx.x] = m > 0.0 ? m : 1.0;
 }
 
-template <int D, typename TF>
+template <int D, class I, typename TF>
 __global__ __launch_bounds__(TPB) void k_features(const TF *__restrict__ f, const double *__restrict__ scale,
-                                                  uint16_t *__restrict__ x, Ext e, int64_t nvox) {
-    const int64_t v = (int64_t)blockIdx.x * TPB + threadIdx.x;
+                                                  uint16_t *__restrict__ x, Ext e, I nvox) {
+    const I v = (I)blockIdx.x * TPB + threadIdx.x;
     if (v >= nvox) return;
-    const int64_t V = (int64_t)e.n0 * e.n1 * e.n2, n = v / V, r = v - n * V;
-    const int px = (int)(r % e.n0), py = (int)((r / e.n0) % e.n1), pz = (int)(r / ((int64_t)e.n0 * e.n1));
+    const I V = (I)e.n0 * e.n1 * e.n2, n = v / V, r = v - n * V;
+    const int px = (int)(r % e.n0), py = (int)((r / e.n0) % e.n1), pz = (int)(r / ((I)e.n0 * e.n1));
     float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     o[0] = (float)((double)f[v] / scale[n]);
     o[1] = 2.0f * ((float)px + 0.5f) / (float)e.n0 - 1.0f;
@@ -1145,8 +1154,11 @@ void forward(srmg_unet *n, hipStream_t st, int B) {
             in = n->X.v.as<uint16_t>();
         } else {
             const int64_t total = (int64_t)B * n->V[l] * (n->w[l - 1] / 8);
-            hipLaunchKernelGGL((k_pool<D>), dim3(nblocks(total)), dim3(TPB), 0, st, n->E[l - 1].v.as<uint16_t>(),
-                               n->P[l].v.as<uint16_t>(), n->w[l - 1] / 8, n->ext[l], n->ext[l - 1], total);
+            for_index(8 * total << D, [&](auto ix) {
+                using I = decltype(ix);
+                hipLaunchKernelGGL((k_pool<D, I>), dim3(nblocks(total)), dim3(TPB), 0, st, n->E[l - 1].v.as<uint16_t>(),
+                                   n->P[l].v.as<uint16_t>(), n->w[l - 1] / 8, n->ext[l], n->ext[l - 1], (I)total);
+            });
             in = n->P[l].v.as<uint16_t>();
         }
         conv_fwd<D>(n, st, n->conv[n->cA[l]], in, n->A[l].v.p, B);
@@ -1156,9 +1168,12 @@ void forward(srmg_unet *n, hipStream_t st, int B) {
         const uint16_t *src = (l == L - 2) ? n->E[L - 1].v.as<uint16_t>() : n->Dd[l + 1].v.as<uint16_t>();
         conv_fwd<D>(n, st, n->conv[n->cC[l]], src, n->C[l].v.p, B);
         const int64_t total = (int64_t)B * n->V[l] * (n->w[l] / 8);
-        hipLaunchKernelGGL((k_up_add<D>), dim3(nblocks(total)), dim3(TPB), 0, st, n->C[l].v.as<uint16_t>(),
-                           n->E[l].v.as<uint16_t>(), n->S[l].v.as<uint16_t>(), n->w[l] / 8, n->ext[l + 1], n->ext[l],
-                           total);
+        for_index(8 * total, [&](auto ix) {
+            using I = decltype(ix);
+            hipLaunchKernelGGL((k_up_add<D, I>), dim3(nblocks(total)), dim3(TPB), 0, st, n->C[l].v.as<uint16_t>(),
+                               n->E[l].v.as<uint16_t>(), n->S[l].v.as<uint16_t>(), n->w[l] / 8, n->ext[l + 1], n->ext[l],
+                               (I)total);
+        });
         conv_fwd<D>(n, st, n->conv[n->cDd[l]], n->S[l].v.as<uint16_t>(), n->Dd[l].v.p, B);
     }
     conv_fwd<D>(n, st, n->conv[n->cY], n->Dd[0].v.as<uint16_t>(), n->Y.p, B);
@@ -1179,8 +1194,11 @@ void backward(srmg_unet *n, hipStream_t st, int B) {
         conv_bwd_weights<D>(n, st, cd, g16(n->Dd[l]), v16(n->S[l]), B);
         conv_bwd_data<D>(n, st, cd, g16(n->Dd[l]), g16(n->S[l]), nullptr, B);
         const int64_t total = (int64_t)B * n->V[l + 1] * (n->w[l] / 8);
-        hipLaunchKernelGGL((k_up_bwd<D>), dim3(nblocks(total)), dim3(TPB), 0, st, g16(n->S[l]), g16(n->C[l]),
-                           n->w[l] / 8, n->ext[l + 1], n->ext[l], total);
+        for_index(8 * total << D, [&](auto ix) {
+            using I = decltype(ix);
+            hipLaunchKernelGGL((k_up_bwd<D, I>), dim3(nblocks(total)), dim3(TPB), 0, st, g16(n->S[l]), g16(n->C[l]),
+                               n->w[l] / 8, n->ext[l + 1], n->ext[l], (I)total);
+        });
         const ConvL &cc = n->conv[n->cC[l]];
         Tensor &src = (l == L - 2) ? n->E[L - 1] : n->Dd[l + 1];
         conv_bwd_weights<D>(n, st, cc, g16(n->C[l]), v16(src), B);
@@ -1196,9 +1214,12 @@ void backward(srmg_unet *n, hipStream_t st, int B) {
         if (l > 0) {
             conv_bwd_data<D>(n, st, ca, g16(n->A[l]), g16(n->P[l]), nullptr, B);
             const int64_t total = (int64_t)B * n->V[l - 1] * (n->w[l - 1] / 8);
-            hipLaunchKernelGGL((k_pool_bwd<D>), dim3(nblocks(total)), dim3(TPB), 0, st, g16(n->S[l - 1]),
-                               g16(n->P[l]), v16(n->E[l - 1]), g16(n->E[l - 1]), n->w[l - 1] / 8, n->ext[l],
-                               n->ext[l - 1], total);
+            for_index(8 * total, [&](auto ix) {
+                using I = decltype(ix);
+                hipLaunchKernelGGL((k_pool_bwd<D, I>), dim3(nblocks(total)), dim3(TPB), 0, st, g16(n->S[l - 1]),
+                                   g16(n->P[l]), v16(n->E[l - 1]), g16(n->E[l - 1]), n->w[l - 1] / 8, n->ext[l],
+                                   n->ext[l - 1], (I)total);
+            });
         }
     }
 }
@@ -1209,12 +1230,15 @@ void features(srmg_unet *n, hipStream_t st, const TF *f, int B) {
                        n->absmax_part.as<double>());
     hipLaunchKernelGGL(k_absmax, dim3(B), dim3(TPB), 0, st, n->absmax_part.as<double>(), n->scale.as<double>());
     const int64_t nvox = (int64_t)B * n->V[0];
-    if (n->D == 3)
-        hipLaunchKernelGGL((k_features<3, TF>), dim3(nblocks(nvox)), dim3(TPB), 0, st, f, n->scale.as<double>(),
-                           n->X.v.as<uint16_t>(), n->ext[0], nvox);
-    else
-        hipLaunchKernelGGL((k_features<2, TF>), dim3(nblocks(nvox)), dim3(TPB), 0, st, f, n->scale.as<double>(),
-                           n->X.v.as<uint16_t>(), n->ext[0], nvox);
+    for_index(nvox * FEAT, [&](auto ix) {
+        using I = decltype(ix);
+        const auto go = [&](auto k) {
+            hipLaunchKernelGGL(k, dim3(nblocks(nvox)), dim3(TPB), 0, st, f, n->scale.as<double>(),
+                               n->X.v.as<uint16_t>(), n->ext[0], (I)nvox);
+        };
+        if (n->D == 3) go(k_features<3, I, TF>);
+        else go(k_features<2, I, TF>);
+    });
 }
 
 void run_forward(srmg_unet *n, hipStream_t st, int B) {
