@@ -87,7 +87,8 @@ struct CoarseGroup {
 struct Graph {
     hipGraph_t g = nullptr;
     hipGraphExec_t x = nullptr;
-    uint64_t gen = 0;     // srmg_ctx::graph_gen when captured
+    uint64_t gen = 0;     // srmg_ctx::graph_gen when captured (V-cycle: of its eager calls)
+    bool exact = false;   // it points to the matrices of the exact level-1 solve
     bool ran = false;     // the step has run eagerly once (lazily built state exists)
     bool vcycle = false;  // a single V-cycle's, called `calls` times
     int calls = 0;
@@ -2015,38 +2016,45 @@ static void axis_decomp(int n, bool radial, double alow, double ahigh, double *l
         }
 }
 
+// The matrices of the exact level-1 solve for op's geometry and boundary table.
+// The context holds one set: another operator's solve replaces it, so whatever
+// captures an exact cycle calls this first, also where the same cycle has run
+// eagerly before.
+static void coarse_ready(srmg_ctx *c, const srmg_op *op) {
+    const int D = c->D;
+    for (CoarseGroup &G : c->groups) {
+        if (G.valid && G.geom == op->geometry && std::memcmp(G.bc, op->bc, 27) == 0) continue;
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(c->stream, &st));
+        if (st != hipStreamCaptureStatusNone) fail("coarse-solve setup inside graph capture");
+        c->graph_gen++;  // captured steps point to the matrices replaced here
+        G.valid = false;
+        int rdim = (op->geometry == SRMG_CYL1) ? 0 : (op->geometry == SRMG_CYL2 ? 1 : -1);
+        for (int d = 0; d < D; d++) {
+            int il = 0, ih = 0, m = 1;
+            for (int e = 0; e < D; e++) {
+                il += ((e == d ? -1 : 0) + 1) * m;
+                ih += ((e == d ? 1 : 0) + 1) * m;
+                m *= 3;
+            }
+            int n = G.N[d];
+            std::vector<double> lam(n), P((size_t)n * n), Q((size_t)n * n);
+            axis_decomp(n, d == rdim, (double)op->bc[il], (double)op->bc[ih], lam.data(), P.data(), Q.data());
+            G.lam[d].alloc(n * sizeof(double));
+            HIPCHK(hipMemcpy(G.lam[d].p, lam.data(), n * sizeof(double), hipMemcpyHostToDevice));
+            upload_axis_matrix(G.P[d], P, n);
+            upload_axis_matrix(G.Q[d], Q, n);
+        }
+        G.valid = true;
+        G.geom = op->geometry;
+        std::memcpy(G.bc, op->bc, 27);
+    }
+}
+
 template <int D, int M, typename T>
 void Ops<D, M, T>::coarse_exact(FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
     (void)s;  // each tree's -s and shift come from its group's tables (prepare())
-    for (CoarseGroup &G : c->groups) {
-        const int *N = G.N;
-        bool hit = G.valid && G.geom == op->geometry && std::memcmp(G.bc, op->bc, 27) == 0;
-        if (!hit) {
-            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-            HIPCHK(hipStreamIsCapturing(c->stream, &st));
-            if (st != hipStreamCaptureStatusNone) fail("coarse-solve setup inside graph capture");
-            c->graph_gen++;  // captured steps point to the matrices replaced here
-            int rdim = (op->geometry == SRMG_CYL1) ? 0 : (op->geometry == SRMG_CYL2 ? 1 : -1);
-            for (int d = 0; d < D; d++) {
-                int il = 0, ih = 0, m = 1;
-                for (int e = 0; e < D; e++) {
-                    il += ((e == d ? -1 : 0) + 1) * m;
-                    ih += ((e == d ? 1 : 0) + 1) * m;
-                    m *= 3;
-                }
-                int n = N[d];
-                std::vector<double> lam(n), P((size_t)n * n), Q((size_t)n * n);
-                axis_decomp(n, d == rdim, (double)op->bc[il], (double)op->bc[ih], lam.data(), P.data(), Q.data());
-                G.lam[d].alloc(n * sizeof(double));
-                HIPCHK(hipMemcpy(G.lam[d].p, lam.data(), n * sizeof(double), hipMemcpyHostToDevice));
-                upload_axis_matrix(G.P[d], P, n);
-                upload_axis_matrix(G.Q[d], Q, n);
-            }
-            G.valid = true;
-            G.geom = op->geometry;
-            std::memcpy(G.bc, op->bc, 27);
-        }
-    }
+    coarse_ready(c, op);
     if constexpr (D == 2)
         if (coarse_exact_2d(u, b)) return;
     for (CoarseGroup &G : c->groups) {
@@ -2398,7 +2406,7 @@ static Graph &solve_graph(srmg_ctx *c, int kind, std::initializer_list<const Fie
     // drop graphs captured before the last coarse-solve rebuild (no solve is
     // running here, so nothing refers to them; a V-cycle's replay may be)
     for (auto it = c->graphs.begin(); it != c->graphs.end();) {
-        if (it->second->x && it->second->gen != c->graph_gen) {
+        if (it->second->x && it->second->exact && it->second->gen != c->graph_gen) {
             HIPCHK(hipStreamSynchronize(c->stream));
             it = c->graphs.erase(it);
         } else {
@@ -2438,6 +2446,7 @@ static Graph &solve_graph(srmg_ctx *c, int kind, std::initializer_list<const Fie
     if (!slot) {
         slot = std::make_unique<Graph>();
         slot->vcycle = kind == 4;
+        slot->exact = c->pops[0].coarse == SRMG_COARSE_EXACT;
     }
     return *slot;
 }
@@ -2505,6 +2514,7 @@ static void solve_plain(srmg_ctx *c, int ui, int bi, int ri, int u1i, const srmg
             done = record(read_norms(c), r0, o->tol, 0, o->max_cycles, hist);
         }
         int k = 0;
+        if (o->max_cycles > 0 && !done && op->coarse == SRMG_COARSE_EXACT) coarse_ready(c, op);
         Graph &gr = solve_graph(c, 0, {&u, &b, &r, &u1}, o);
         Graph &gf = solve_graph(c, 2, {&u, &b, &r, &u1}, o);
         while (k < o->max_cycles && !done) {
@@ -2651,6 +2661,7 @@ static void solve_mixed_dm(srmg_ctx *c, FieldBuf &u, FieldBuf &b, FieldBuf &e, F
         done = record(rg, r0, o->tol, 0, o->max_cycles, hist);
     }
     int k = 0;
+    if (o->max_cycles > 0 && !done && op->coarse == SRMG_COARSE_EXACT) coarse_ready(c, op);
     Graph &gr = solve_graph(c, 1, {&u, &b, &e, &be, &re, &ue}, o);
     Graph &gf = solve_graph(c, 3, {&u, &b, &e, &be, &re, &ue}, o);
     while (k < o->max_cycles && !done) {
@@ -3212,7 +3223,15 @@ static void do_vcycle(srmg_ctx *c, int ui, int bi, int ri, int u1i, int lmax, in
     o.nup = nup;
     o.omega = omega;
     o.inner_cycles = lmax;
+    const bool exact = c->pops[0].coarse == SRMG_COARSE_EXACT;
+    if (exact) coarse_ready(c, &c->pops[0]);
     Graph &g = solve_graph(c, 4, {&u, &b, &r, &u1}, &o);
+    // operators that replace each other's matrices: calls count from the last
+    // rebuild, so that what the next one would drop is not captured
+    if (exact && !g.x && g.gen != c->graph_gen) {
+        g.gen = c->graph_gen;
+        g.calls = 0;
+    }
     dispatch(c, t, [&](auto &ops) {
         // the captured launches start from and end in the primary buffers
         for (FieldBuf *f : {&u, &b, &r, &u1}) ops.settle(*f);
@@ -3322,7 +3341,6 @@ static void do_vcycle4(srmg_ctx *c, int u, int b, int r, int u1, double s, const
     add(omega);
     auto &slot = c->graphs[k];
     if (!slot) slot = std::make_unique<Graph>();
-    slot->gen = c->graph_gen;
     run_maybe_graph(c, *slot, true, [&] {
         dispatch(c, t, [&](auto &o) { o.vcycle4(fu, fb, fr, fu1, s, op, lmax, ndown, ntop, nup, omega); });
     });
