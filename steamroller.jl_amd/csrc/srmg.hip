@@ -23,6 +23,7 @@
 #include "../../include/srmg.h"
 #include "common.h"
 #include "kernels.h"
+#include "roles.h"
 #include "layout.h"
 #include "unet.h"
 
@@ -2341,21 +2342,29 @@ static void field_to_host(srmg_ctx *c, FieldBuf &f, TH *host, int G,
 // ---------------------------------------------------------------------------
 
 // Record the launches of `body` (which only enqueues kernels on c->stream)
-// into gr without running them.
+// into gr without running them. When that fails, the fields and gr are as they
+// were before.
 template <class F>
 static void capture_graph(srmg_ctx *c, Graph &gr, F &&body) {
+    RolesKeeper roles(c->fields);
+    hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     try {
         body();
     } catch (...) {
-        hipGraph_t tmp = nullptr;
-        (void)hipStreamEndCapture(c->stream, &tmp);
-        if (tmp) (void)hipGraphDestroy(tmp);
+        (void)hipStreamEndCapture(c->stream, &g);
+        if (g) (void)hipGraphDestroy(g);
         throw;
     }
-    HIPCHK(hipStreamEndCapture(c->stream, &gr.g));
-    HIPCHK(hipGraphInstantiate(&gr.x, gr.g, nullptr, nullptr, 0));
+    HIPCHK(hipStreamEndCapture(c->stream, &g));
+    hipGraphExec_t x = nullptr;
+    const hipError_t e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+    if (e != hipSuccess) (void)hipGraphDestroy(g);
+    HIPCHK(e);
+    gr.g = g;
+    gr.x = x;
     gr.gen = c->graph_gen;
+    roles.keep();
 }
 
 // Run `body` either directly or via a graph captured on its first use.
