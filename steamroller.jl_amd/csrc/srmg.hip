@@ -3907,9 +3907,12 @@ static GridSolvePlan grid_solve_plan(srmg_ctx *c, int D, const int *n, const srm
     return g;
 }
 
-// whole planes per work group, in place in u
-static bool grid_solve_many(const srmg_ctx *c, const GridSolvePlan &g, int ngrid) {
-    return c->axis_gemm == 2 && l1_fused_ok(g.dims, g.N) && (int64_t)ngrid * g.N[2] >= L1B_PLANES;
+// whole planes per work group, in place in u: not where u lies across f, whose
+// later planes the first launch would read after others were written
+static bool grid_solve_many(const srmg_ctx *c, const GridSolvePlan &g, const double *f, const double *u, int ngrid) {
+    const uintptr_t pf = (uintptr_t)f, pu = (uintptr_t)u, bytes = g.total * ngrid * sizeof(double);
+    const bool across = pf != pu && pf < pu + bytes && pu < pf + bytes;
+    return c->axis_gemm == 2 && l1_fused_ok(g.dims, g.N) && (int64_t)ngrid * g.N[2] >= L1B_PLANES && !across;
 }
 
 // the mirror signs of axis d at its two ends
@@ -3966,7 +3969,7 @@ static void grid_solve_run(srmg_ctx *c, const GridSolvePlan &g, double s, const 
     const int dims = g.dims;
     hipLaunchKernelGGL(k_fill<double>, dim3(nwg(ngrid)), dim3(WG), 0, c->stream, bufs.shift,
                        op->disc == SRMG_HELMHOLTZ ? -s * op->k2 : 0.0, (size_t)ngrid);
-    if (grid_solve_many(c, g, ngrid)) {
+    if (grid_solve_many(c, g, f, u, ngrid)) {
         launch_l1_many(c->stream, ngrid, N, f, bufs.Q, bufs.P, bufs.lam, bufs.shift, u);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->stream));
@@ -4040,7 +4043,7 @@ int srmg_grid_solve(srmg_ctx *c, int D, const int *n, double s, const srmg_op *o
         // the two grids in between, where the kernels need them (launch_l1_many
         // does not); small ones stay with the context
         constexpr size_t GRID_KEEP = (size_t)64 << 20;
-        const bool many = grid_solve_many(c, g, ngrid);
+        const bool many = grid_solve_many(c, g, f, u, ngrid);
         const size_t bytes = many ? 16 : g.total * ngrid * sizeof(double);
         DevBuf l1, l2, l3;
         DevBuf &g1 = bytes > GRID_KEEP ? l1 : c->gs_g1, &g2 = bytes > GRID_KEEP ? l2 : c->gs_g2;
