@@ -1737,6 +1737,15 @@ struct Ops {
         }
     }
 
+    // launches of a V-cycle, at least (levels without complete sibling groups
+    // and odd numbers of sweeps take more)
+    int cycle_launches(int lmax, int ndown, int ntop, int nup, bool exact) const {
+        const auto sweeps = [&](int l, int k) { return pairs(c->lv[l].nblk) ? k / 2 + k % 2 : k; };
+        int n = exact ? 3 : sweeps(0, ntop);
+        for (int l = 1; l < lmax; l++)
+            if (c->lv[l].nblk) n += (D == 3 ? 3 : 2) + sweeps(l, ndown) + sweeps(l, nup);
+        return n;
+    }
     // vcycle! (src/multigrid.jl:60-106). The residual of level l is formed
     // right after smoothing: it reads only level-l cells and level-l ghosts, none
     // of which the restriction to l-1 changes. The fill_ghost! calls on r are not
@@ -3217,10 +3226,19 @@ int srmg_fill_ghost_all(srmg_ctx *c, int id, const int8_t *bc) {
     });
 }
 
-// A V-cycle on its own. Its 20 to 60 launches cost the host 3.6 us each when
-// issued one by one, more than a small tree's kernels take: from the third call
-// of a configuration on they are replayed as a graph (capturing costs about
-// what three calls save).
+// A V-cycle on its own. Its launches cost the host 2.5 to 3.6 us each when
+// issued one by one, more than a small tree's kernels take when a program has
+// several trees in hand: from the third call of a configuration on they are
+// replayed as a graph (capturing costs about what three calls save). A replay
+// costs the host 20 to 35 us whatever it holds and the GPU 2 to 5 us before its
+// first kernel, so cycles of few launches and cycles that the GPU is busy with
+// for longer than the host is stay as they are. One cycle after another on one
+// tree, one by one / replayed, the host's part in brackets: 64 blocks of 16^2 on
+// one level 9.4 (8.9) / 18.9 (18.9) us; 1,024 on five levels 83 (73) / 82 (35);
+// 2,112 on three, 541k cells, 53 (39) / 55 (21); 2,496 of 8^3 on three, 1.28M
+// cells, 106 (73) / 111 (36); 7,808 of 16^2 on three, 2.0M cells, 78 (38) / 83 (21).
+constexpr int REPLAY_LAUNCHES = 8;
+constexpr int64_t REPLAY_CELLS = (int64_t)1 << 20;
 static void do_vcycle(srmg_ctx *c, int ui, int bi, int ri, int u1i, int lmax, int ndown, int ntop, int nup,
                       double omega) {
     if (lmax < 0 || lmax > c->nlevels) fail("lmax out of range");
@@ -3244,7 +3262,12 @@ static void do_vcycle(srmg_ctx *c, int ui, int bi, int ri, int u1i, int lmax, in
     dispatch(c, t, [&](auto &ops) {
         // the captured launches start from and end in the primary buffers
         for (FieldBuf *f : {&u, &b, &r, &u1}) ops.settle(*f);
-        run_maybe_graph(c, g, g.calls >= 2, [&] {
+        const int top = lmax ? lmax : c->nlevels;
+        int64_t cells = 0;
+        for (int l = 0; l < top; l++) cells += (int64_t)c->lv[l].nblk * c->V;
+        const bool replay =
+            cells <= REPLAY_CELLS && ops.cycle_launches(top, ndown, ntop, nup, exact) >= REPLAY_LAUNCHES;
+        run_maybe_graph(c, g, replay && g.calls >= 2, [&] {
             ops.vcycle(u, b, r, u1, c->ps[0], &c->pops[0], lmax, ndown, ntop, nup, omega);
         });
     });
