@@ -3244,34 +3244,35 @@ static void do_vcycle(srmg_ctx *c, int ui, int bi, int ri, int u1i, int lmax, in
     if (lmax < 0 || lmax > c->nlevels) fail("lmax out of range");
     const int t = same_type(c, {ui, bi, ri, u1i});
     FieldBuf &u = field(c, ui), &b = field(c, bi), &r = field(c, ri), &u1 = field(c, u1i);
-    srmg_solve_opts o{};
-    o.ndown = ndown;
-    o.ntop = ntop;
-    o.nup = nup;
-    o.omega = omega;
-    o.inner_cycles = lmax;
     const bool exact = c->pops[0].coarse == SRMG_COARSE_EXACT;
-    if (exact) coarse_ready(c, &c->pops[0]);
-    Graph &g = solve_graph(c, 4, {&u, &b, &r, &u1}, &o);
-    // operators that replace each other's matrices: calls count from the last
-    // rebuild, so that what the next one would drop is not captured
-    if (exact && !g.x && g.gen != c->graph_gen) {
-        g.gen = c->graph_gen;
-        g.calls = 0;
-    }
+    const int top = lmax ? lmax : c->nlevels;
+    int64_t cells = 0;
+    for (int l = 0; l < top; l++) cells += (int64_t)c->lv[l].nblk * c->V;
     dispatch(c, t, [&](auto &ops) {
+        auto body = [&] { ops.vcycle(u, b, r, u1, c->ps[0], &c->pops[0], lmax, ndown, ntop, nup, omega); };
         // the captured launches start from and end in the primary buffers
         for (FieldBuf *f : {&u, &b, &r, &u1}) ops.settle(*f);
-        const int top = lmax ? lmax : c->nlevels;
-        int64_t cells = 0;
-        for (int l = 0; l < top; l++) cells += (int64_t)c->lv[l].nblk * c->V;
-        const bool replay =
-            cells <= REPLAY_CELLS && ops.cycle_launches(top, ndown, ntop, nup, exact) >= REPLAY_LAUNCHES;
-        run_maybe_graph(c, g, replay && g.calls >= 2, [&] {
-            ops.vcycle(u, b, r, u1, c->ps[0], &c->pops[0], lmax, ndown, ntop, nup, omega);
-        });
+        if (cells > REPLAY_CELLS || ops.cycle_launches(top, ndown, ntop, nup, exact) < REPLAY_LAUNCHES) {
+            body();
+            return;
+        }
+        if (exact) coarse_ready(c, &c->pops[0]);
+        srmg_solve_opts o{};
+        o.ndown = ndown;
+        o.ntop = ntop;
+        o.nup = nup;
+        o.omega = omega;
+        o.inner_cycles = lmax;
+        Graph &g = solve_graph(c, 4, {&u, &b, &r, &u1}, &o);
+        // operators that replace each other's matrices: calls count from the
+        // last rebuild, so that what the next one would drop is not captured
+        if (exact && !g.x && g.gen != c->graph_gen) {
+            g.gen = c->graph_gen;
+            g.calls = 0;
+        }
+        run_maybe_graph(c, g, g.calls >= 2, body);
+        g.calls = std::min(g.calls + 1, 2);
     });
-    g.calls = std::min(g.calls + 1, 2);
     HIPCHK(hipGetLastError());
 }
 
