@@ -733,15 +733,18 @@ static void upload_tables(srmg_ctx *c) {
     // until autotuned or set: for 8^3 blocks the column sweep on two threads per
     // column (shape 8; levels without complete sibling groups run shape 0),
     // except on levels small enough that the launch is latency and its groups
-    // fill the chip unevenly: there a work group takes one block. FP64, shapes
-    // 0 / 8: 512 blocks 4.5 / 6.8 us, 1,200 6.5 / 7.6, 5,184 15.6 / 16.8, 14,976
-    // 36.2 / 38.8, 32,768 119 / 97. FP32: 512 blocks 4.0 / 5.5, 1,200 5.6 / 6.1,
-    // 1,728 equal, 2,744 8.3 / 7.5 (the finest level keeps shape 8, which can
-    // start from zero without reading it)
+    // fill the chip unevenly: there a work group takes one block. What shape 8
+    // adds to V-cycles (2, 4, 2) of 50 to 1,100 us with shape 0 on the level
+    // (a sweep follows another, whose writes it finds in the caches), FP64: 384
+    // blocks +9 us, 1,152 +5, 2,560 +5, 3,752 -2, 5,760 -3, 7,352 +2, 12,288 +1,
+    // 12,544 -11, 22,400 -58; on level 1, whose blocks are a box: 1,728 +1, 4,096
+    // -5, 8,000 -1, 13,824 -8. FP32: 384 +6, 1,144 +3, 1,728 0, 2,560 -2, 3,752
+    // -6, 5,760 -11 (the finest level keeps shape 8, which can start from zero
+    // without reading it)
     c->sweep_cfg.assign(2 * nlevels, 0);
     if (c->D == 3 && c->M == 8)
         for (int l = 0; l < nlevels; l++) {
-            c->sweep_cfg[l] = c->lv[l].nblk <= 16384 ? 0 : 8;
+            c->sweep_cfg[l] = c->lv[l].nblk <= (l ? 10000 : 3000) ? 0 : 8;
             c->sweep_cfg[nlevels + l] = c->lv[l].nblk <= 1200 && l < nlevels - 1 ? 0 : 8;
         }
     c->zero[0].reset();
