@@ -1285,10 +1285,12 @@ __global__ __launch_bounds__(WG) void k_diff_fill(T *dst, const T *a1, const T *
 // SUM_NT-th partial with 16 loads in flight, then a halving tree. out is
 // host memory that the device can write: no copy follows. (Two launches and a
 // copy before: 12 us per norm on one tree, 8 on several.)
-constexpr int SUM_NT = 1024;
-__global__ __launch_bounds__(SUM_NT) void k_sum_ranges(const double *__restrict__ partial,
-                                                       const int2 *__restrict__ rng, int nr,
-                                                       double *__restrict__ out) {
+// One work group has a pass of SUM_PASS loads in flight and waits them out: on
+// one tree of more than SUM_ONE partials the passes are work groups of a launch
+// of their own (partial's tail as out), and the pieces' sums one more.
+constexpr int SUM_NT = 1024, SUM_PASS = 16 * SUM_NT, SUM_ONE = 2 * SUM_PASS;
+__global__ __launch_bounds__(SUM_NT) void k_sum_ranges(const double *partial, const int2 *__restrict__ rng, int nr,
+                                                       double *out) {
     __shared__ double red[SUM_NT / 64];
     const int tid = threadIdx.x;
     double acc = 0.0;
@@ -2535,9 +2537,10 @@ __device__ __forceinline__ void load_tile(T *tile, int *tab, int *blks, const X 
     constexpr int PI = (BPW * V + NT - 1) / NT, PH = (BPW * ND * F + NT - 1) / NT;
     const int tid = threadIdx.x;
     auto blk_at = [&](int lb) { return list ? list[first + min(lb, nloc - 1)] : first + min(lb, nloc - 1); };
+    static_assert(V % 64 == 0 && NT % 64 == 0, "the cells of a wave are one block's");
     int bl[PI];
 #pragma unroll
-    for (int j = 0; j < PI; j++) bl[j] = blk_at((tid + NT * j) / V);
+    for (int j = 0; j < PI; j++) bl[j] = blk_at(__builtin_amdgcn_readfirstlane((tid + NT * j) / V));
     const int bt = blk_at(tid / ND), bs = blk_at(min(tid, BPW - 1));
     T xv[PI];
 #pragma unroll
@@ -2672,7 +2675,8 @@ enum { RES_WRITE = 0, RES_NORM = 1, RES_DEFECT = 2 };
 
 // Residual of a level from LDS tiles (src/multigrid.jl:309-323).
 //   RES_WRITE:  r = -(b + L u / s) on the blocks [a.blk0, a.blk0 + a.nblk)
-//   RES_NORM:   leaf blocks list[0..n): partial[k] = wgt * sum of r^2 over block list[k]
+//   RES_NORM:   leaf blocks list[0..n), or where list is null the n blocks from
+//               a.blk0: partial[k] = wgt * sum of r^2 over block k of them
 //   RES_DEFECT: out (float) = b + L u / s = -r on the level's blocks, and
 //               partial[k] = wgt * sum of r^2 over block k if it is a leaf (else 0)
 // Each block's partial is an LDS tree sum in a fixed order.
@@ -2701,7 +2705,7 @@ __device__ __forceinline__ void resid_tile(ResidTileLds<D, M, T, BPW, NT, MODE> 
     const int first = xcd_remap(wg, nwg) * BPW;
     const int nloc = min(BPW, n - first);
     const int *lst = (MODE == RES_NORM) ? list : nullptr;
-    const int base = (MODE == RES_NORM) ? first : a.blk0 + first;
+    const int base = lst ? first : a.blk0 + first;
     // the right-hand sides of the thread's cells, their radial weights and the
     // block parameters come with the tile's two round trips
     constexpr int PER = (BPW * V + NT - 1) / NT;
@@ -2716,7 +2720,8 @@ __device__ __forceinline__ void resid_tile(ResidTileLds<D, M, T, BPW, NT, MODE> 
             if ((int)threadIdx.x < nloc) bpl = bparams(a, blk_at(threadIdx.x));
 #pragma unroll
             for (int j = 0; j < PER; j++) {
-                const int i = threadIdx.x + NT * j, lb = min(i / V, BPW - 1), blk = blk_at(lb);
+                const int i = threadIdx.x + NT * j, lb = min(i / V, BPW - 1);
+                const int blk = blk_at(__builtin_amdgcn_readfirstlane(lb));
                 bv[j] = (i < nloc * V) ? b[(size_t)blk * V + (i - lb * V)] : T(0);
                 Jc[j] = rbase<D, M, RD>(coord, blk);
                 leafs[j] = MODE == RES_DEFECT && isleaf[blk];
@@ -3441,6 +3446,16 @@ __device__ __forceinline__ void defect_col(typename ColDefect<D, M, RD>::Smem &s
     else CD::template run<0>(sm, out, u, b, ib, a, g0, w, lane, tv, bpl, wgt, partial);
 }
 
+// one level on its own
+template <int D, int M, int RD>
+__global__ __launch_bounds__(256) void k_defect_col(float *__restrict__ out, const double *__restrict__ u,
+                                                    const double *__restrict__ b, const double *__restrict__ ib,
+                                                    const int *__restrict__ htab, const int *__restrict__ isleaf,
+                                                    LevelArgs<double> a, double wgt, double *__restrict__ partial) {
+    __shared__ typename ColDefect<D, M, RD>::Smem sm;
+    defect_col<D, M, RD>(sm, blockIdx.x, gridDim.x, out, u, b, ib, htab, isleaf, a, wgt, partial);
+}
+
 // ---- residual norms and defects of several levels in one launch ----
 //
 // A solve's norm needs every level, and a level that does not fill the chip
@@ -3455,7 +3470,8 @@ struct ResidSeg {
     double wgt;
     int wg0, nwg;  // its work groups
     int kind;
-    int n, list0;  // SEG_TILE: blocks, and where its leaves start in the list (NORM)
+    int n, list0;  // SEG_TILE: blocks, and where its leaves start in the list (NORM;
+                   // -1: they are all blocks in their order)
     int p0;        // its first partial
 };
 constexpr int SEG_MAX = 12;
@@ -3465,13 +3481,25 @@ struct ResidSegs {
     int n;
 };
 
-template <int D, int M, typename T, typename TO, int BPW, int NT, bool NORM, int RD>
+// COLS: segments of defect_col among them. Its registers and LDS leave 12 waves
+// to a CU for 32, which a tile segment pays for: on 9,261 blocks of 8^3 without
+// sibling groups 42 us for 22, on 103,823 495 for 237. So large levels without
+// groups take a launch without it (TILE_APART). And a work group of it waits out
+// the look-up of its segment, with nothing else to run: 110,592 blocks with
+// groups took 212 us a norm for 197 in k_defect_col, so a column level of that
+// order (COL_APART: where the difference pays for a launch), or one with no other
+// beside it, goes there.
+constexpr int TILE_APART = 2000, COL_APART = 80000;
+template <int D, int M, typename T>
+constexpr bool RESID_COLS = D == 3 && M == 8 && sizeof(T) == 8;
+template <int D, int M, typename T, typename TO, int BPW, int NT, bool NORM, int RD, bool COLS>
 __global__ __launch_bounds__(NT) void k_resid_levels(ResidSegs<T> g, TO *__restrict__ out, const T *__restrict__ u,
                                                      const T *__restrict__ b, const T *__restrict__ ib,
                                                      const int *__restrict__ htab, const int *__restrict__ coord,
                                                      const int *__restrict__ leaves, const int *__restrict__ isleaf,
                                                      double *__restrict__ partial) {
-    constexpr bool GROUPS = D == 2 && M == 16 && NT == 256, COLS = D == 3 && M == 8 && RD < 0 && sizeof(T) == 8;
+    constexpr bool GROUPS = D == 2 && M == 16 && NT == 256;
+    static_assert(!COLS || RD < 0, "columns are Cartesian");
     constexpr int TM = NORM ? RES_NORM : RES_DEFECT;
     using TileLds = ResidTileLds<D, M, T, BPW, NT, TM>;
     using GroupLds = ResidGroupLds<D, M, T, RES_DEFECT, GROUPS ? NT : 1>;
@@ -3501,8 +3529,8 @@ __global__ __launch_bounds__(NT) void k_resid_levels(ResidSegs<T> g, TO *__restr
         }
     }
     resid_tile<D, M, T, TO, BPW, NT, TM, RD>(*reinterpret_cast<TileLds *>(sm), wg, s.nwg, out, u, b, ib, htab, coord,
-                                             NORM ? leaves + s.list0 : nullptr, isleaf, s.n, s.a, s.wgt,
-                                             partial + s.p0);
+                                             NORM && s.list0 >= 0 ? leaves + s.list0 : nullptr, isleaf, s.n, s.a,
+                                             s.wgt, partial + s.p0);
 }
 
 template <int D, int M, typename T, int RD>

@@ -192,7 +192,8 @@ struct srmg_ctx {
     DevBuf d_w64, d_w32;    // radial weights (double / float), per level and dim
     DevBuf d_partial;
     PinnedBuf norms;        // per tree: the sum of the norm queued last, written by the device
-    DevBuf d_rng_leaf, d_rng_blk;  // per (tree, level): ranges of the leaf / block partials
+    DevBuf d_rng_leaf, d_rng_blk;  // per (tree, level): ranges of the leaf / block partials (sum_ranges)
+    int nsum_leaf = 0, nsum_blk = 0;  // pieces that a sum of them takes first, 0: none
     DevBuf d_gord;                 // per grouped 3D level: processing order of its sibling groups
     DevBuf d_grid, d_grid2; // stacked level-1 uniform grids (coarse solve)
     std::vector<std::unique_ptr<FieldBuf>> fields;
@@ -672,6 +673,17 @@ static void upload_tables(srmg_ctx *c) {
     up(c->d_pix, pix.data(), pix.size() * sizeof(int));
     up(c->d_w64, w64.data(), w64.size() * sizeof(double));
     up(c->d_w32, w32.data(), w32.size() * sizeof(float));
+    // one tree with more partials than SUM_ONE: then the pieces of SUM_PASS, and
+    // the range of their sums behind the partials
+    c->maxpartials = nb + 16;
+    auto pieces = [&](std::vector<int2> &r, int n) {
+        const int np = nt == 1 && n > SUM_ONE ? (n + SUM_PASS - 1) / SUM_PASS : 0;
+        for (int k = 0; k < np; k++) r.push_back(make_int2(k * SUM_PASS, std::min(SUM_PASS, n - k * SUM_PASS)));
+        if (np) r.push_back(make_int2(c->maxpartials, np));
+        return np;
+    };
+    c->nsum_leaf = pieces(rl, pl);
+    c->nsum_blk = pieces(rb, pbk);
     up(c->d_rng_leaf, rl.data(), rl.size() * sizeof(int2));
     up(c->d_rng_blk, rb.data(), rb.size() * sizeof(int2));
     // a second processing order of the sibling groups of grouped 3D levels
@@ -703,8 +715,7 @@ static void upload_tables(srmg_ctx *c) {
     }
     up(c->d_gord, gord.data(), gord.size() * sizeof(int));
     // per-block partials: at most one per block of every level
-    c->maxpartials = nb + 16;
-    c->d_partial.alloc((size_t)c->maxpartials * sizeof(double));
+    c->d_partial.alloc((size_t)(c->maxpartials + std::max(c->nsum_leaf, c->nsum_blk)) * sizeof(double));
     c->norms.reserve(nt * sizeof(double));
     size_t ng = 0;
     // the 2D solve takes all groups at once, the others one after the other
@@ -1278,10 +1289,21 @@ struct Ops {
         hipLaunchKernelGGL((k_residual<D, M, T>), dim3(nwg((int64_t)a.nblk * LY::V)), dim3(WG), 0, c->stream,
                            X(r, l), X(u, l), X(b, l), I(u), nbr(), coord(), a);
     }
-    // fixed-order total of every tree's partials over its (tree, level) ranges
-    void sum_partials(const DevBuf &ranges) {
-        hipLaunchKernelGGL(k_sum_ranges, dim3((unsigned)c->trees.size()), dim3(SUM_NT), 0, c->stream,
-                           c->d_partial.as<double>(), ranges.as<int2>(), c->nlevels, c->norms.dev);
+    // fixed-order total of every tree's partials over its (tree, level) ranges,
+    // leaves' or blocks'
+    void sum_partials(bool leaf) {
+        const int2 *rng = (leaf ? c->d_rng_leaf : c->d_rng_blk).template as<int2>();
+        const int np = leaf ? c->nsum_leaf : c->nsum_blk;
+        double *p = c->d_partial.as<double>();
+        if (np) {
+            rng += c->nlevels;
+            hipLaunchKernelGGL(k_sum_ranges, dim3((unsigned)np), dim3(SUM_NT), 0, c->stream, p, rng, 1,
+                               p + c->maxpartials);
+            hipLaunchKernelGGL(k_sum_ranges, dim3(1), dim3(SUM_NT), 0, c->stream, p, rng + np, 1, c->norms.dev);
+        } else {
+            hipLaunchKernelGGL(k_sum_ranges, dim3((unsigned)c->trees.size()), dim3(SUM_NT), 0, c->stream, p, rng,
+                               c->nlevels, c->norms.dev);
+        }
     }
     void restrict_(FieldBuf &x, int l) {
         const LevelInfo &L = c->lv[l];
@@ -1613,50 +1635,81 @@ struct Ops {
     void resid_levels(TO *out, FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
         settle(u);
         settle(b);
-        ResidSegs<T> g{};
-        int wgs = 0, np = 0, rdim = -1;
-        auto flush = [&] {
-            if (!g.n) return;
+        // segments of a launch; cols: with those of the column form
+        struct Launch {
+            ResidSegs<T> g{};
+            int wgs = 0;
+        } with_cols, tiles;
+        int np = 0, rdim = -1;
+        auto flush = [&](Launch &f, auto cols) {
+            if (!f.g.n) return;
             with_rd(rdim, [&](auto rd) {
                 constexpr int RD = decltype(rd)::value;
-                hipLaunchKernelGGL((k_resid_levels<D, M, T, TO, RB, RNT, NORM, RD>), dim3((unsigned)wgs), dim3(RNT), 0,
-                                   c->stream, g, out, u.data.as<T>(), b.data.as<T>(), I(u), c->d_halo.as<int>(),
-                                   coord(), c->d_leaves.as<int>(), c->d_isleaf.as<int>(), c->d_partial.as<double>());
+                constexpr bool CO = decltype(cols)::value && RD < 0;
+                if constexpr (CO) {
+                    const ResidSeg<T> &q = f.g.s[0];
+                    if (f.g.n == 1 && q.kind == SEG_COL) {
+                        hipLaunchKernelGGL((k_defect_col<D, M, RD>), dim3((unsigned)q.nwg), dim3(256), 0, c->stream,
+                                           (float *)out, u.data.as<T>(), b.data.as<T>(), I(u), c->d_halo.as<int>(),
+                                           c->d_isleaf.as<int>(), q.a, q.wgt, c->d_partial.as<double>() + q.p0);
+                        return;
+                    }
+                }
+                hipLaunchKernelGGL((k_resid_levels<D, M, T, TO, RB, RNT, NORM, RD, CO>), dim3((unsigned)f.wgs),
+                                   dim3(RNT), 0, c->stream, f.g, out, u.data.as<T>(), b.data.as<T>(), I(u),
+                                   c->d_halo.as<int>(), coord(), c->d_leaves.as<int>(), c->d_isleaf.as<int>(),
+                                   c->d_partial.as<double>());
             });
-            g.n = 0;
-            wgs = 0;
+            f = Launch();
         };
-        // largest (finest) levels first: the small ones run beside their tail
+        using Cols = std::integral_constant<bool, RESID_COLS<D, M, T>>;
+        auto kind = [&](int l, int rdim) {
+            const LevelInfo &L = c->lv[l];
+            // complete sibling groups; for a norm only where every block is a
+            // leaf in block order (the same per-block sums)
+            if (!GROUP_OK || !grouped(l) || (NORM && !L.all_leaves)) return SEG_TILE;
+            return D == 2 ? SEG_GROUP : (rdim < 0 && Cols::value) ? SEG_COL : SEG_TILE;
+        };
         std::vector<int> p0(c->nlevels);
+        bool any_col = false;
         for (int l = 0; l < c->nlevels; l++) {
             p0[l] = np;
             np += NORM ? c->lv[l].nleaf : c->lv[l].nblk;
+            any_col = any_col || (c->lv[l].nblk && kind(l, level_args<T>(c, l, s, op, 1.0).rdim) == SEG_COL);
         }
+        // largest (finest) levels first: the small ones run beside their tail
         for (int l = c->nlevels - 1; l >= 0; l--) {
             const LevelInfo &L = c->lv[l];
-            if (!(NORM ? L.nleaf : L.nblk)) continue;
-            if (g.n == SEG_MAX) flush();
-            ResidSeg<T> &q = g.s[g.n++];
-            q.a = level_args<T>(c, l, s, op, 1.0);
-            rdim = q.a.rdim;
+            const int n = NORM ? L.nleaf : L.nblk;
+            if (!n) continue;
+            const LevelArgs<T> a = level_args<T>(c, l, s, op, 1.0);
+            rdim = a.rdim;
+            const int kd = kind(l, rdim);
+            const bool co = any_col && !(kd == SEG_TILE && n > TILE_APART);
+            Launch &f = co ? with_cols : tiles;
+            if (f.g.n == SEG_MAX) {
+                if (co) flush(f, Cols());
+                else flush(f, std::false_type());
+            }
+            ResidSeg<T> &q = f.g.s[f.g.n++];
+            q.a = a;
             q.wgt = std::ldexp(1.0, -c->D * l);
-            // complete sibling groups; for a norm only where every block is a
-            // leaf in block order (the same per-block sums)
-            const bool gr = GROUP_OK && grouped(l) && (!NORM || L.all_leaves);
-            q.kind = !gr ? SEG_TILE : D == 2 ? SEG_GROUP : (q.a.rdim < 0 && std::is_same<T, double>::value) ? SEG_COL : SEG_TILE;
-            q.n = NORM ? L.nleaf : L.nblk;
-            q.list0 = L.leaf0;
-            q.nwg = q.kind == SEG_TILE ? (q.n + RB - 1) / RB : L.nblk >> D;
-            q.wg0 = wgs;
+            q.kind = kd;
+            q.n = n;
+            q.list0 = L.all_leaves ? -1 : L.leaf0;
+            q.nwg = kd == SEG_TILE ? (q.n + RB - 1) / RB : L.nblk >> D;
+            q.wg0 = f.wgs;
             q.p0 = p0[l];
-            wgs += (q.nwg + 7) / 8 * 8;
+            f.wgs += (q.nwg + 7) / 8 * 8;
+            if (kd == SEG_COL && n > COL_APART && f.g.n == 1) flush(f, Cols());
         }
-        flush();
+        flush(with_cols, Cols());
+        flush(tiles, std::false_type());
     }
     // queue the squared-residual sums (leaf blocks, weighted by 2^(-D(l-1))) and their totals
     void resnorm_partials(FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
         resid_levels<true>((T *)nullptr, u, b, s, op);
-        sum_partials(c->d_rng_leaf);
+        sum_partials(true);
     }
     // resnorm partials of u = 0 from b alone (bitwise those of resnorm_partials
     // on a zero field); be (may be null): (float) b on every leaf block
@@ -1670,7 +1723,7 @@ struct Ops {
         if (n)
             hipLaunchKernelGGL((k_bnorm<D, M, T, BB, RNT>), dim3((unsigned)((n + BB - 1) / BB)), dim3(RNT), 0, c->stream,
                                b.data.as<T>(), c->d_leaves.as<int>(), n, lv, c->d_partial.as<double>(), be);
-        sum_partials(c->d_rng_leaf);
+        sum_partials(true);
     }
     // u = 0 on every level and slab (values in the primary buffer)
     void zero_all(FieldBuf &u) {
@@ -1683,7 +1736,7 @@ struct Ops {
     // residual norm partials, in one pass (T = double)
     void defect_and_norm(float *be, FieldBuf &u, FieldBuf &b, double s, const srmg_op *op) {
         resid_levels<false>(be, u, b, s, op);
-        sum_partials(c->d_rng_blk);
+        sum_partials(false);
     }
 
     // coarse_exact of 2D trees whose level-1 extents are at most 256, every
