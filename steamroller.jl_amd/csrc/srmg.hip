@@ -88,9 +88,8 @@ struct CoarseGroup {
 struct Graph {
     hipGraph_t g = nullptr;
     hipGraphExec_t x = nullptr;
-    uint64_t gen = 0;     // srmg_ctx::graph_gen when captured (V-cycle: of its eager calls)
+    uint64_t gen = 0;     // srmg_ctx::graph_gen when captured (V-cycle: after its last eager call)
     bool exact = false;   // it points to the matrices of the exact level-1 solve
-    bool ran = false;     // the step has run eagerly once (lazily built state exists)
     bool vcycle = false;  // a single V-cycle's, called `calls` times
     int calls = 0;
     ~Graph() {
@@ -2083,9 +2082,10 @@ static void axis_decomp(int n, bool radial, double alow, double ahigh, double *l
 }
 
 // The matrices of the exact level-1 solve for op's geometry and boundary table.
-// The context holds one set: another operator's solve replaces it, so whatever
-// captures an exact cycle calls this first, also where the same cycle has run
-// eagerly before.
+// The context holds one set, which another operator's solve replaces: an exact
+// cycle is captured only while the matrices of an eager run of it are in place
+// (graph_gen has not changed since). Made here, in the cycle, the host's work
+// runs beside the descent's kernels.
 static void coarse_ready(srmg_ctx *c, const srmg_op *op) {
     const int D = c->D;
     for (CoarseGroup &G : c->groups) {
@@ -2444,16 +2444,16 @@ static void run_maybe_graph(srmg_ctx *c, Graph &gr, bool use_graph, F &&body) {
 }
 
 // A solve's first step when it differs from the later ones (fmg! first, a
-// zero start, another FP32 cycle count): run eagerly the first time, so that
-// lazily built state exists, then recorded at once (a step leaves the host
-// state as it found it, so recording it again changes nothing), so that the
-// next solve replays it from its first step.
+// zero start, another FP32 cycle count): run eagerly where there is no graph of
+// it, so that lazily built state exists (that an earlier solve ran it so is not
+// enough: another operator's matrices may have replaced its own since), then
+// recorded at once (a step leaves the host state as it found it, so recording it
+// again changes nothing), so that the next solve replays it from its first step.
 template <class F>
 static void run_first_step(srmg_ctx *c, Graph &g, bool use_graph, F &&body) {
-    const bool replay = use_graph && (g.ran || g.x);
+    const bool replay = use_graph && g.x;
     run_maybe_graph(c, g, replay, body);
-    if (use_graph && !replay && !g.x) capture_graph(c, g, body);
-    g.ran = true;
+    if (use_graph && !replay) capture_graph(c, g, body);
 }
 
 // A caller who varies a V-cycle's parameters at every call leaves one entry
@@ -2588,7 +2588,6 @@ static void solve_plain(srmg_ctx *c, int ui, int bi, int ri, int u1i, const srmg
             done = record(read_norms(c), r0, o->tol, 0, o->max_cycles, hist);
         }
         int k = 0;
-        if (o->max_cycles > 0 && !done && op->coarse == SRMG_COARSE_EXACT) coarse_ready(c, op);
         Graph &gr = solve_graph(c, 0, {&u, &b, &r, &u1}, o);
         Graph &gf = solve_graph(c, 2, {&u, &b, &r, &u1}, o);
         while (k < o->max_cycles && !done) {
@@ -2607,7 +2606,6 @@ static void solve_plain(srmg_ctx *c, int ui, int bi, int ri, int u1i, const srmg
                 run_first_step(c, g, o->use_graph, step);
             } else {
                 run_maybe_graph(c, g, o->use_graph && (k > 0 || g.x), step);
-                g.ran = true;
             }
             k++;
             done = record(read_norms(c), r0, o->tol, k, o->max_cycles, hist);
@@ -2735,7 +2733,6 @@ static void solve_mixed_dm(srmg_ctx *c, FieldBuf &u, FieldBuf &b, FieldBuf &e, F
         done = record(rg, r0, o->tol, 0, o->max_cycles, hist);
     }
     int k = 0;
-    if (o->max_cycles > 0 && !done && op->coarse == SRMG_COARSE_EXACT) coarse_ready(c, op);
     Graph &gr = solve_graph(c, 1, {&u, &b, &e, &be, &re, &ue}, o);
     Graph &gf = solve_graph(c, 3, {&u, &b, &e, &be, &re, &ue}, o);
     while (k < o->max_cycles && !done) {
@@ -2746,7 +2743,6 @@ static void solve_mixed_dm(srmg_ctx *c, FieldBuf &u, FieldBuf &b, FieldBuf &e, F
             run_first_step(c, g, o->use_graph, step);
         } else {
             run_maybe_graph(c, g, o->use_graph && (k > 0 || g.x), step);
-            g.ran = true;
         }
         k++;
         done = record(read_norms(c), r0, o->tol, k, o->max_cycles, hist);
@@ -3312,7 +3308,6 @@ static void do_vcycle(srmg_ctx *c, int ui, int bi, int ri, int u1i, int lmax, in
             body();
             return;
         }
-        if (exact) coarse_ready(c, &c->pops[0]);
         srmg_solve_opts o{};
         o.ndown = ndown;
         o.ntop = ntop;
@@ -3320,13 +3315,11 @@ static void do_vcycle(srmg_ctx *c, int ui, int bi, int ri, int u1i, int lmax, in
         o.omega = omega;
         o.inner_cycles = lmax;
         Graph &g = solve_graph(c, 4, {&u, &b, &r, &u1}, &o);
-        // operators that replace each other's matrices: calls count from the
-        // last rebuild, so that what the next one would drop is not captured
-        if (exact && !g.x && g.gen != c->graph_gen) {
-            g.gen = c->graph_gen;
-            g.calls = 0;
-        }
+        // calls with other matrices do not count: a capture must find its own
+        // in place, and what the next operator would drop is not worth one
+        if (exact && !g.x && g.gen != c->graph_gen) g.calls = 0;
         run_maybe_graph(c, g, g.calls >= 2, body);
+        g.gen = c->graph_gen;
         g.calls = std::min(g.calls + 1, 2);
     });
     HIPCHK(hipGetLastError());
