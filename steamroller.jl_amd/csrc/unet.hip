@@ -1027,6 +1027,18 @@ int64_t tile_count(const Ext &e, int64_t nvox) {
     return per * (nvox / ((int64_t)e.n0 * e.n1 * e.n2));
 }
 
+// k_conv_tile where at least 45% of its tiles' voxels are the grid's: a tile costs
+// what it costs when full. A forward pass on two levels of 2^18 voxels (2D: 2^17),
+// gathered / tiles, 16 channels: 4^3 grids (12% of the tiles) 658 / 799 us, 18 x 10
+// x 6 (26%) 178 / 222, 2D 18^2 (32%) 140 / 148; 20 x 12 x 28 (47%) 156 / 154, 2D 16^2
+// (50%) 155 / 149, 12^3 (56%) 168 / 158, 24^3 (75%) 147 / 118; 32 channels: 18 x 10
+// x 6 (35%) 288 / 298, 6^3 (42%) 424 / 426, 12^3 (56%) 281 / 233.
+template <class TL>
+bool tile_fits(const Ext &e) {
+    const int64_t V = (int64_t)e.n0 * e.n1 * e.n2;
+    return 100 * V >= 45 * tile_count<TL>(e, V) * TL::NV;
+}
+
 template <int D, int OUT>
 void conv_launch_r(int R, unsigned grid, hipStream_t st, const uint16_t *in, int cin_log2, const uint16_t *w, int kp,
                    int ktot, const float *bias, int nbias, int relu, const uint16_t *mask, void *out, int cout_s,
@@ -1047,7 +1059,7 @@ void conv_launch_r(int R, unsigned grid, hipStream_t st, const uint16_t *in, int
         return;
     }
 #define SRMG_TILE(CC, RR)                                                                                          \
-    if (cin_log2 == ilog2(CC) && R == RR) {                                                              \
+    if (cin_log2 == ilog2(CC) && R == RR && tile_fits<ConvTile<D, CC>>(e)) {                             \
         hipLaunchKernelGGL((k_conv_tile<D, CC, RR, OUT>), dim3((unsigned)tile_count<ConvTile<D, CC>>(e, nvox)),    \
                            dim3(TPB), 0, st, in, w, kp, bias, nbias, relu, mask, out, cout_s, e.n0, e.n1, e.n2);   \
         return;                                                                                                    \
