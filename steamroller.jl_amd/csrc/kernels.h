@@ -996,17 +996,16 @@ __device__ __forceinline__ int rt_sidx(int D, int M, int x, int y, int z) {
     return (((x + y + z + D) & 1) ? 0 : V / 2) + (x >> 1) + (M / 2) * (y + M * z);
 }
 
-// Host blocks in the pinned ring -> device blocks (one work group each): the
+// Host blocks in the pinned ring -> device blocks dev (one work group each): the
 // planes of the last dimension from one cell below the valid ones to one above,
 // S = M + 2 G cells in the other dimensions, read once and in order, as the bus
 // likes it. Valid cells, and the depth-1 ghosts of coarse-fine faces into their
 // slabs.
 template <typename TH, typename TD>
 __global__ __launch_bounds__(WG) void k_host_in(TD *__restrict__ data, TD *__restrict__ ib, const TH *__restrict__ src,
-                                                const int *__restrict__ host2dev, const int *__restrict__ nbr, int D,
+                                                const int *__restrict__ dev, const int *__restrict__ nbr, int D,
                                                 int M, int G) {
-    const int b = host2dev[blockIdx.x];
-    if (b < 0) return;
+    const int b = dev[blockIdx.x];
     const int S = M + 2 * G, V = D == 2 ? M * M : M * M * M, F = V / M;
     const int n = (D == 2 ? S : S * S) * (M + 2);
     const TH *p = src + (size_t)blockIdx.x * n;
@@ -1036,15 +1035,14 @@ struct Faces6 {
 };
 
 // Device blocks -> boxes of M + 2 g cells per dimension (g = 0 or 1) in the
-// pinned ring, in the order of the host's block ids (one work group each): valid cells and, with
-// g = 1, the face ghosts (copies, +-mirrors, slabs); edges and corners are not
+// pinned ring, in the order of the host's block ids (one work group each, dev the
+// device blocks): valid cells and, with g = 1, the face ghosts (copies, +-mirrors, slabs); edges and corners are not
 // written.
 template <typename TD, typename TH>
 __global__ __launch_bounds__(WG) void k_host_out(TH *__restrict__ dst, const TD *__restrict__ data,
-                                                 const TD *__restrict__ ib, const int *__restrict__ host2dev,
+                                                 const TD *__restrict__ ib, const int *__restrict__ dev,
                                                  const int *__restrict__ nbr, int D, int M, int g, Faces6 sg) {
-    const int b = host2dev[blockIdx.x];
-    if (b < 0) return;
+    const int b = dev[blockIdx.x];
     const int B = M + 2 * g, n = D == 2 ? B * B : B * B * B, V = D == 2 ? M * M : M * M * M, F = V / M;
     TH *p = dst + (size_t)blockIdx.x * n;
     for (int i = threadIdx.x; i < n; i += WG) {

@@ -172,7 +172,10 @@ struct srmg_ctx {
     std::vector<std::unique_ptr<AxisPlan>> axes;
     uint64_t grid_calls = 0;
     DevBuf gs_shift, gs_g1, gs_g2;
-    DevBuf d_host2dev;      // host block id - 1 -> device block, or -1 (made on first use)
+    // the tree's blocks in the order of their host ids (made on first use): the
+    // ids (from 0), and on the device their device blocks
+    std::vector<int64_t> h_live;
+    DevBuf d_live;
     int D = 2, M = 16, V = 0, F = 0;
     int nlevels = 0;
     int64_t nhost = 0;      // host block ids 1..nhost (all trees)
@@ -564,7 +567,8 @@ static void commit_tables(srmg_ctx *c, srmg_ctx &t) {
     HIPCHK(hipStreamSynchronize(c->stream));  // a replay of them may be running
     c->graphs.clear();
     c->box_ok = false;
-    c->d_host2dev.release();
+    c->h_live.clear();
+    c->d_live.release();
     c->nlevels = t.nlevels;
     c->nhost = t.nhost;
     c->nb = t.nb;
@@ -2235,15 +2239,21 @@ static int same_type(srmg_ctx *c, std::initializer_list<int> ids) {
 // pageable memory, a V-cycle with two fields each way took 20.4 ms on a 2D tree
 // of 7,716 blocks of 16^2, now 3.3 ms.
 
-static const int *host_table(srmg_ctx *c) {
-    if (!c->d_host2dev.p) {
-        // kernels index it by host block id - 1
-        c->d_host2dev.alloc((size_t)std::max<int64_t>(c->nhost, 1) * sizeof(int));
-        HIPCHK(hipMemcpyAsync(c->d_host2dev.p, c->host2dev.data() + 1, (size_t)c->nhost * sizeof(int),
-                              hipMemcpyHostToDevice, c->stream));
+// Host ids that no block of the tree has (freed by a regrid) take no part.
+static const int *live_blocks(srmg_ctx *c) {
+    if (!c->d_live.p) {
+        std::vector<int> dev;
+        c->h_live.clear();
+        for (int64_t h = 0; h < c->nhost; h++) {
+            if (c->host2dev[h + 1] < 0) continue;
+            c->h_live.push_back(h);
+            dev.push_back(c->host2dev[h + 1]);
+        }
+        c->d_live.alloc(std::max<size_t>(dev.size(), 1) * sizeof(int));
+        HIPCHK(hipMemcpyAsync(c->d_live.p, dev.data(), dev.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
     }
-    return c->d_host2dev.as<int>();
+    return c->d_live.as<int>();
 }
 
 // The pieces 0 .. np-1 of a field, in order on this thread (which talks to the
@@ -2316,23 +2326,27 @@ static void host_to_field(srmg_ctx *c, const TH *host, int G, FieldBuf &f) {
     // of a block, the planes of the last dimension within one cell of the valid ones
     const size_t PB = SP * (M + 2), skip = SP * (G - 1);
     HostStage &st = c->stage;
-    st.reserve((size_t)c->nhost * PB * sizeof(TH), PB * sizeof(TH));
+    const int *dev = live_blocks(c);
+    const int64_t *live = c->h_live.data(), nlive = (int64_t)c->h_live.size();
+    st.reserve((size_t)nlive * PB * sizeof(TH), PB * sizeof(TH));
     const int64_t per = (int64_t)(st.bytes / (PB * sizeof(TH)));
-    const int *h2d = host_table(c);
-    const int np = (int)((c->nhost + per - 1) / per);
+    const int np = (int)((nlive + per - 1) / per);
     auto copy = [&](int k) {
-        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
+        const int64_t i0 = k * per, n = std::min(per, nlive - i0);
         TH *dst = reinterpret_cast<TH *>(st.host(k));
-        const TH *src = host + (size_t)h0 * SD + skip;
-        if (PB == SD)
-            std::memcpy(dst, src, (size_t)n * SD * sizeof(TH));
-        else
-            for (int64_t b = 0; b < n; b++) std::memcpy(dst + b * PB, src + b * SD, PB * sizeof(TH));
+        for (int64_t b = 0; b < n;) {
+            const int64_t h = live[i0 + b];
+            int64_t run = 1;  // whole blocks, one after the other
+            if (PB == SD)
+                while (b + run < n && live[i0 + b + run] == h + run) run++;
+            std::memcpy(dst + b * PB, host + (size_t)h * SD + skip, (size_t)run * PB * sizeof(TH));
+            b += run;
+        }
     };
     pipe_pieces(st, np, true, copy, [&](int k) {
-        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
+        const int64_t i0 = k * per, n = std::min(per, nlive - i0);
         hipLaunchKernelGGL((k_host_in<TH, TD>), dim3((unsigned)n), dim3(WG), 0, c->stream, f.data.as<TD>(),
-                           f.ib.as<TD>(), reinterpret_cast<const TH *>(st.device(k)), h2d + h0,
+                           f.ib.as<TD>(), reinterpret_cast<const TH *>(st.device(k)), dev + i0,
                            c->d_nbr.as<int>(), D, M, G);
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(st.ev[k % HostStage::SLOTS], c->stream));
@@ -2371,32 +2385,33 @@ static void field_to_host(srmg_ctx *c, FieldBuf &f, TH *host, int G,
     const int B = G ? M + 2 : M;
     const size_t BX = (D == 2) ? (size_t)B * B : (size_t)B * B * B;
     HostStage &st = c->stage;
-    st.reserve((size_t)c->nhost * BX * sizeof(TH), BX * sizeof(TH));
+    const int *dev = live_blocks(c);
+    const int64_t *live = c->h_live.data(), nlive = (int64_t)c->h_live.size();
+    st.reserve((size_t)nlive * BX * sizeof(TH), BX * sizeof(TH));
     const int64_t per = (int64_t)(st.bytes / (BX * sizeof(TH)));
-    const int *h2d = host_table(c);
-    const int np = (int)((c->nhost + per - 1) / per);
+    const int np = (int)((nlive + per - 1) / per);
     Faces6 sg;
     for (int q = 0; q < 6; q++) sg.s[q] = bcsign ? bcsign[q] : 1;
     auto issue = [&](int k) {
-        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
+        const int64_t i0 = k * per, n = std::min(per, nlive - i0);
         hipLaunchKernelGGL((k_host_out<TD, TH>), dim3((unsigned)n), dim3(WG), 0, c->stream,
-                           reinterpret_cast<TH *>(st.device(k)), f.data.as<TD>(), f.ib.as<TD>(), h2d + h0,
+                           reinterpret_cast<TH *>(st.device(k)), f.data.as<TD>(), f.ib.as<TD>(), dev + i0,
                            c->d_nbr.as<int>(), D, M, G ? 1 : 0, sg);
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(st.ev[k % HostStage::SLOTS], c->stream));
     };
     auto place = [&](int k) {
-        const int64_t h0 = k * per, n = std::min(per, c->nhost - h0);
+        const int64_t i0 = k * per, n = std::min(per, nlive - i0);
         const TH *box = reinterpret_cast<const TH *>(st.host(k));
         for (int64_t i = 0; i < n; i++) {
-            const int b = c->host2dev[h0 + i + 1];
-            if (b < 0) continue;
+            const int64_t h = live[i0 + i];
+            const int b = c->host2dev[h + 1];
             int skip = 0;
             if (!bcsign)
                 for (int q = 0; q < ND; q++)
                     if (c->h_nbr[(size_t)b * ND + q] == NB_BOUNDARY) skip |= 1 << q;
-            if (M == 16) box_to_host<TH, 16>(host + (size_t)(h0 + i) * SD, box + i * BX, D, G, skip);
-            else box_to_host<TH, 8>(host + (size_t)(h0 + i) * SD, box + i * BX, D, G, skip);
+            if (M == 16) box_to_host<TH, 16>(host + (size_t)h * SD, box + i * BX, D, G, skip);
+            else box_to_host<TH, 8>(host + (size_t)h * SD, box + i * BX, D, G, skip);
         }
     };
     pipe_pieces(st, np, false, place, issue);
