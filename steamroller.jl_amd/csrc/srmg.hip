@@ -2345,7 +2345,8 @@ static void host_to_field(srmg_ctx *c, const TH *host, int G, FieldBuf &f) {
     };
     pipe_pieces(st, np, true, copy, [&](int k) {
         const int64_t i0 = k * per, n = std::min(per, nlive - i0);
-        hipLaunchKernelGGL((k_host_in<TH, TD>), dim3((unsigned)n), dim3(WG), 0, c->stream, f.data.as<TD>(),
+        const unsigned parts = (unsigned)((PB + HOST_IN_CELLS - 1) / HOST_IN_CELLS);
+        hipLaunchKernelGGL((k_host_in<TH, TD>), dim3((unsigned)n, parts), dim3(WG), 0, c->stream, f.data.as<TD>(),
                            f.ib.as<TD>(), reinterpret_cast<const TH *>(st.device(k)), dev + i0,
                            c->d_nbr.as<int>(), D, M, G);
         HIPCHK(hipGetLastError());
