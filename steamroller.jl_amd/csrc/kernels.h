@@ -3486,12 +3486,13 @@ struct ResidSegs {
 // COLS: segments of defect_col among them. Its registers and LDS leave 12 waves
 // to a CU for 32, which a tile segment pays for: on 9,261 blocks of 8^3 without
 // sibling groups 42 us for 22, on 103,823 495 for 237. So large levels without
-// groups take a launch without it (TILE_APART). And a work group of it waits out
+// groups take a launch without it (TILE_APART; on 2,048 leaves beside 12,608 blocks
+// with groups one launch takes 26.0 us, two 26.4). And a work group of it waits out
 // the look-up of its segment, with nothing else to run: 110,592 blocks with
 // groups took 212 us a norm for 197 in k_defect_col, so a column level of that
 // order (COL_APART: where the difference pays for a launch), or one with no other
 // beside it, goes there.
-constexpr int TILE_APART = 2000, COL_APART = 80000;
+constexpr int TILE_APART = 3000, COL_APART = 80000;
 template <int D, int M, typename T>
 constexpr bool RESID_COLS = D == 3 && M == 8 && sizeof(T) == 8;
 template <int D, int M, typename T, typename TO, int BPW, int NT, bool NORM, int RD, bool COLS>
