@@ -345,7 +345,7 @@ int srmg_guess_fallbacks(srmg_ctx *ctx, int *n);
 /* Exact solve of L_1 u = f on ngrid stacked uniform level-1 grids (x fastest,
  * n[0] x n[1] (x n[2]) cells, the level-1 stencil of op with scale s: the
  * Helmholtz shift is -s k2), FP64 device pointers. Training targets for the
- * network; f = -s b for the problem of srmg_solve. */
+ * network; f = -s b for the problem of srmg_solve. u may be f, or lie across it. */
 int srmg_grid_solve(srmg_ctx *ctx, int D, const int *n, double s, const srmg_op *op, const double *f, double *u,
                     int ngrid);
 
@@ -417,10 +417,14 @@ int srmg_time_kernel(srmg_ctx *ctx, int kind, int level, int u, int b, int r, do
  * stores of the result, nontemporal loads of the right-hand side, or both
  * (levels without complete sibling groups, and thread counts that do not
  * divide a group's cells per colour, run 0; 7 to 11 run 4 and 5 where the
- * column forms do not apply). */
+ * column forms do not apply). The shapes are those of single sweeps: 2D levels
+ * of M=16, and of M=8 up to 8,192 blocks, run their sweeps two to a launch, which
+ * no shape tunes, and take a shape only for the last of an odd number. */
 int srmg_autotune(srmg_ctx *ctx, int u, int b, double s, const srmg_op *op, int reps, int *chosen);
 /* Force the tile shape (0..11) of the fused sweep for one element type and level (1-based).
- * Until autotuned or forced, 3D M=8 contexts run shape 8 and the others shape 0. */
+ * Until autotuned or forced, 3D M=8 levels run shape 8, but 0 where they are small
+ * (F64: up to 3,000 blocks on level 1, 10,000 above; F32: up to 1,200 below the
+ * finest); all others run shape 0. */
 int srmg_set_sweep_config(srmg_ctx *ctx, int dtype, int level, int cfg);
 /* 1 when the level's blocks form complete sibling groups (tile shapes 4..8 apply). */
 int srmg_level_grouped(srmg_ctx *ctx, int level, int *grouped);
@@ -430,7 +434,9 @@ int srmg_set_group_tiles(srmg_ctx *ctx, int enable);
 /* Kernels of the level-1 solve (exact coarsest solve and srmg_grid_solve):
  * 2 (default) three launches for 3D grids whose extents are multiples of 8 and
  * at most 64 (plane and column tiles in LDS: forward x and y, forward z with
- * the eigenvalue division and inverse z, inverse y and x), else as 1; 1 one
+ * the eigenvalue division and inverse z, inverse y and x), four for the 2D level
+ * 1 of extents up to 256 (one per transform, all trees' grids in each), else as
+ * 1; 1 one
  * launch per axis transform, one wave per work group without LDS where the
  * axis length is at most 64; 0 the LDS-tiled axis kernels. All give the same
  * bits. */
